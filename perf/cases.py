@@ -47,8 +47,8 @@ def listed():
         _join("join16m_nobf", 16_000_000, 16_000_000, 10, partition_size=1024),
         # every R key four times: more than one row per match
         _join("dups_9m_24m", 9_000_004, 24_000_001, 5, dup=4),
-        # two large ragged tables on a dense sorted id, no filter, half of S matches
-        _join("ids_100m_130m", 100_000_007, 130_000_001, 2, keys="ids"),
+        # two large ragged tables on a dense sorted id, no filter, a quarter of S matches
+        _join("ids_100m_130m", 100_000_007, 130_000_001, 4, keys="ids"),
         # the benchmark's headline join: 640M tuples on each side, filter, 10% match
         _join("join640m_bf10", 640_000_000, 640_000_000, 10, use_bf=1, bf_bits_per_key=10.0, num_hashes=3,
               partition_size=512, radix_bits=14),
@@ -261,7 +261,8 @@ def _columns_of(res):
 def _slots(c, r_val, s_val):
     if c.get("dup", 1) == 1:
         return s_val.long()
-    return s_val.long() * c["dup"] + torch.div(r_val, c["n_r"] // c["dup"], rounding_mode="floor")
+    copy = torch.div(r_val, c["n_r"] // c["dup"], rounding_mode="floor")
+    return torch.add(copy, s_val, alpha=c["dup"]).long()
 
 
 def _place(state, count, key, r_val, s_val):
