@@ -130,6 +130,16 @@ constexpr uint64_t L2_SLICE_BYTES = 3584ull << 10;
 // HBM write streams interleave more and a 640M-tuple pass runs 10-15% slower,
 // while smaller relations need the extra workgroups to hide latency.
 constexpr uint64_t SOLO_TUPLES = 32ull << 20;
+// The direct join's cost against the partitioned join's (choose_direct), in
+// picoseconds on the whole chip.  Measured per (probe tuple, table chunk): 2.4-2.7
+// ps at 10% match (500K x 500K 108 us, 16K x 50M 287 us); with a filter only the
+// survivors are probed, taken as half of S.  The partitioned join takes 130-170 us
+// for its launches alone and 25-40 ps per tuple at these sizes (500K x 500K 166
+// us, 100K x 5M 287 us), 9-11 ps per tuple from some 10M tuples on.  Both sides
+// of the line: 300K x 1M 153 against 178 us, 300K x 3M 402 against 246 us, 800K x
+// 800K 223 against 173 us.
+constexpr double DIRECT_PS_PROBE = 2.7, DIRECT_PS_BF_PROBE = 1.35, DIRECT_PS_SAVED = 100e6;
+constexpr double DIRECT_SMALL_TUPLES = 8e6, DIRECT_PS_SMALL = 20.0, DIRECT_PS_LARGE = 9.0;
 constexpr int PLAN_CUS = 256;  // CUs of an MI355X: only the work split depends on it
 
 int choose_G(uint64_t n)
@@ -148,6 +158,23 @@ void split_bits(int total, int& b1, int& b2)
         b1 = (total + 1) / 2;
         b2 = total - b1;
     }
+}
+
+// Whether a join whose caller left the partitioning to the library (no radix
+// bits, fan-outs, pass bits, tile, filter stage, scatter workgroup or probe
+// timers asked for) runs without a partition: the build side in chunks of one
+// LDS table, all of the probe side past every chunk.
+bool choose_direct(const bj_params& p, const Plan& pl)
+{
+    if (p.radix_bits > 0 || p.partition_size >= 0 || p.second_partition_size >= 0 || p.pass1_bits > 0 ||
+        p.s_pass1_bits > 0 || p.tile > 0 || p.bf_stage != 0 || p.scatter_wg != 0 || p.probe_breakdown != 0)
+        return false;
+    if (pl.bf && pl.bf_stage != 1) return false;
+    const bool build_r = build_from_r(pl.nr, pl.ns, (uint32_t)pl.tile);
+    const double nb = (double)(build_r ? pl.nr : pl.ns), np = (double)(build_r ? pl.ns : pl.nr);
+    const double n = (double)(pl.nr + pl.ns), small = std::min(n, DIRECT_SMALL_TUPLES);
+    return std::ceil(nb / pl.tile) * np * (pl.bf ? DIRECT_PS_BF_PROBE : DIRECT_PS_PROBE) <=
+           DIRECT_PS_SAVED + small * DIRECT_PS_SMALL + (n - small) * DIRECT_PS_LARGE;
 }
 
 int make_plan(const bj_params& p, Plan& pl)
@@ -389,12 +416,19 @@ int workspace_items(const Plan& pl, bool with_r, bool with_out,
     return BJ_OK;
 }
 
+// The buffers a direct join uses: the filter and S', the counters, the rows.
+static bool direct_uses(DevBuf bj_ctx::*m)
+{
+    return m == &bj_ctx::filter || m == &bj_ctx::sp_key || m == &bj_ctx::sp_val || m == &bj_ctx::counters ||
+           m == &bj_ctx::out_key || m == &bj_ctx::out_rval || m == &bj_ctx::out_sval;
+}
+
 int ensure_workspace(bj_ctx* c, const Plan& pl, uint64_t* total_bytes)
 {
     uint64_t total = 0;
     int rc = workspace_items(pl, true, true, [&](DevBuf bj_ctx::*m, uint64_t bytes) -> int {
         total += bytes;
-        return c ? ensure(c->*m, bytes) : BJ_OK;
+        return c && (!pl.direct || direct_uses(m)) ? ensure(c->*m, bytes) : BJ_OK;
     });
     if (rc) return rc;
     if (total_bytes) *total_bytes = total;
@@ -550,6 +584,37 @@ int enqueue_plan_probe(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t
                         P<HeavyItem>(c->items), item_start + nbins, pl.item_cap, ctr + CTR_WORK, ctr + CTR_OUT,
                         cap, o_key, o_rval, o_sval, c->num_cu,
                         pl.probe_breakdown ? P<uint64_t>(c->ptimers) : nullptr, st));
+    BJ_HIP(tl_end(c, BJ_K_PROBE));
+    return BJ_OK;
+}
+
+// The join of unpartitioned relations (Plan::direct): filter and S' first when
+// the plan has a filter, then one build + probe launch.
+static int enqueue_direct(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* r_val,
+                          const uint32_t* s_key, const uint32_t* s_val, uint32_t* o_key, uint32_t* o_rval,
+                          uint32_t* o_sval, uint64_t cap)
+{
+    hipStream_t st = c->stream;
+    uint64_t* ctr = P<uint64_t>(c->counters);
+    uint64_t* filter = pl.bf ? P<uint64_t>(c->filter) : nullptr;
+    const uint64_t* ns_dev = nullptr;
+    BJ_HIP(launch_direct_begin(ctr, CTR_N, filter, pl.bf ? pl.bf_words / 2 : 0, st));
+    if (pl.bf) {
+        BJ_HIP(tl_begin(c, BJ_K_BF_BUILD));
+        BJ_HIP(launch_direct_bloom(r_key, pl.nr, pl.geom, filter, st));
+        BJ_HIP(tl_end(c, BJ_K_BF_BUILD));
+        BJ_HIP(tl_begin(c, BJ_K_BF_FILTER));
+        BJ_HIP(launch_bloom_prefilter(s_key, s_val, pl.ns, filter, pl.geom, P<uint32_t>(c->sp_key),
+                                      P<uint32_t>(c->sp_val), c->sp_key.bytes / 4, ctr + CTR_SPRIME, ctr + CTR_ERR,
+                                      c->num_cu, st));
+        BJ_HIP(tl_end(c, BJ_K_BF_FILTER));
+        s_key = P<uint32_t>(c->sp_key);
+        s_val = P<uint32_t>(c->sp_val);
+        ns_dev = ctr + CTR_SPRIME;
+    }
+    BJ_HIP(tl_begin(c, BJ_K_PROBE));
+    BJ_HIP(launch_join_direct(r_key, r_val, pl.nr, s_key, s_val, pl.ns, ns_dev, ctr + CTR_OUT, cap, o_key, o_rval,
+                              o_sval, c->num_cu, st));
     BJ_HIP(tl_end(c, BJ_K_PROBE));
     return BJ_OK;
 }
@@ -1071,12 +1136,18 @@ int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uin
     int rc;
     hipStream_t st = c->stream;
     uint64_t* ctr = P<uint64_t>(c->counters);
-    BJ_HIP(launch_zero_u64(ctr, CTR_N, st));
-    if ((rc = probe_timers_begin(c, pl))) return rc;
     // slots without kernels (no filter) keep no events and read as 0 ms
-    if ((rc = enqueue_r(c, pl, r_key, r_val))) return rc;
-    const RSide R{P<uint32_t>(c->r_key), P<uint32_t>(c->r_val), P<uint64_t>(c->r_start), P<uint64_t>(c->filter)};
-    if ((rc = enqueue_s_probe(c, pl, R, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
+    int first_slot = BJ_K_HIST_R;
+    if (pl.direct) {
+        first_slot = pl.bf ? BJ_K_BF_BUILD : BJ_K_PROBE;
+        if ((rc = enqueue_direct(c, pl, r_key, r_val, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
+    } else {
+        BJ_HIP(launch_zero_u64(ctr, CTR_N, st));
+        if ((rc = probe_timers_begin(c, pl))) return rc;
+        if ((rc = enqueue_r(c, pl, r_key, r_val))) return rc;
+        const RSide R{P<uint32_t>(c->r_key), P<uint32_t>(c->r_val), P<uint64_t>(c->r_start), P<uint64_t>(c->filter)};
+        if ((rc = enqueue_s_probe(c, pl, R, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
+    }
 
     BJ_HIP(hipMemcpyAsync(c->h_counters, ctr, CTR_N * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
     BJ_HIP(hipStreamSynchronize(st));
@@ -1092,7 +1163,7 @@ int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uin
         double* k = out->kernel_ms;
         for (int i = 0; i < BJ_NUM_KERNELS; i++) k[i] = tl_ms(c, i);
         fill_phases(out, h2d_ms < 0 ? ev_ms(c, EV_H2D0, EV_H2D1) : h2d_ms,
-                    tl_span_ms(c, BJ_K_HIST_R, BJ_K_PROBE));
+                    tl_span_ms(c, first_slot, BJ_K_PROBE));
     }
     return probe_timers_end(c, pl, out);
 }
@@ -1116,6 +1187,7 @@ static int join_once(bj_ctx* c, const bj_params* p, const uint32_t* r_key, const
     int chunks = p->s_chunks;
     if (chunks == 0 && (rc = auto_s_chunks(c, *p, pl, chunks))) return rc;
     if (chunks > 1 && pl.ns > 1) return join_s_chunks(c, p, pl, chunks, r_key, r_val, s_key, s_val, out);
+    pl.direct = choose_direct(*p, pl);
     if ((rc = ensure_workspace(c, pl))) return rc;
     hipStream_t st = c->stream;
 

@@ -30,6 +30,15 @@ __host__ __device__ __forceinline__ uint32_t lowbias32(uint32_t x)
 constexpr uint32_t RADIX_MUL = 0x9E3779B1u;
 __host__ __device__ __forceinline__ uint32_t radix_hash(uint32_t key) { return key * RADIX_MUL; }
 
+// Build side of a sub-bucket: R whenever it fits one LDS table (the
+// reference's build side), else the smaller side.  Equal S keys, as under a
+// skewed S, then stream past distinct R keys instead of piling up in one run
+// of the table that every matching probe walks.
+__host__ __device__ __forceinline__ bool build_from_r(uint64_t nr, uint64_t ns, uint32_t tile)
+{
+    return nr <= tile || nr <= ns;
+}
+
 // ---------------------------------------------------------------- generator
 // 4 rounds of (add, odd multiply, xor-shift right) mod 2^w: each step is a
 // bijection on [0, 2^w), so the composition is a keyed permutation.

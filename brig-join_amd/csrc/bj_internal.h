@@ -102,6 +102,7 @@ struct Plan {
     int scatter_wg = 1024;               // scatter workgroup size
     int G_r = 1, G_s = 1;                // histogram / first-pass scatter workgroups
     bool solo_r = false, solo_s = false; // one scatter workgroup per CU (large relations)
+    bool direct = false;                 // joined without a partition (small build side)
     int tile = 8192;
     uint32_t slice = 65536;
     uint32_t max_slices = 16;
@@ -124,6 +125,9 @@ struct RSide {
 };
 
 int make_plan(const bj_params& p, Plan& pl);
+// Whether the one-pass join of this plan runs without a partition (Plan::direct,
+// which make_plan leaves false: only join_device knows the direct join).
+bool choose_direct(const bj_params& p, const Plan& pl);
 
 }  // namespace bj
 

@@ -96,6 +96,17 @@ hipError_t launch_probe(int tile, const uint32_t* rk, const uint32_t* rv, const 
                         const uint64_t* n_items, uint64_t item_cap, uint64_t* work_ctr, uint64_t* out_count,
                         uint64_t out_cap, uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, int num_cu,
                         uint64_t* timers, hipStream_t st);
+// Direct join of unpartitioned relations (small build sides): begin clears the
+// join's counters and its filter (64-bit blocks), bloom fills the filter, join
+// emits the rows.
+// ns_dev (nullable): device-side length of S, at most ns.
+hipError_t launch_direct_begin(uint64_t* ctr, int n_ctr, uint64_t* filter, uint64_t blocks, hipStream_t st);
+hipError_t launch_direct_bloom(const uint32_t* rkey, uint64_t n, const BloomGeom& g, uint64_t* filter,
+                               hipStream_t st);
+hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t nr, const uint32_t* sk,
+                              const uint32_t* sv, uint64_t ns, const uint64_t* ns_dev, uint64_t* out_count,
+                              uint64_t out_cap, uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, int num_cu,
+                              hipStream_t st);
 // Workgroups of a probe launch (persistent: a fixed number per CU).  With
 // timers, every workgroup adds its phase times (ticks, PT_* order of bj_tiles.h,
 // PT_N = 5 per workgroup) to its slots; the caller clears them.

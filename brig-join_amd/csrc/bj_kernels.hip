@@ -986,6 +986,67 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     }
 }
 
+// ============================================================== direct join (small build side)
+// Clears the join's counters and its filter in one launch.
+__global__ void k_direct_begin(uint64_t* __restrict__ ctr, int n_ctr, uint64_t* __restrict__ filter, uint64_t nf)
+{
+    const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i0 < (uint64_t)n_ctr) ctr[i0] = 0ull;
+    for (uint64_t i = i0; i < nf; i += (uint64_t)gridDim.x * blockDim.x) filter[i] = 0ull;
+}
+
+// The filter of an unpartitioned R: one 64-bit atomic OR per key (cleared
+// before).  The same bits as k_bloom_build's.
+__global__ void k_direct_bloom(const uint32_t* __restrict__ rkey, uint32_t n, BloomGeom g,
+                               uint64_t* __restrict__ filter)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        const uint32_t k = rkey[i];
+        atomicOr((unsigned long long*)&filter[bloom_block(k, g)], (unsigned long long)bloom_mask(k, g.k));
+    }
+}
+
+// Joins unpartitioned relations: the build side in C chunks of at most CAP
+// tuples, the probe side in slices, one (chunk, slice) pair per workgroup and
+// step.  Every chunk streams all of the probe side past its table, so the work
+// is C * np probes where the partitioned path moves every tuple two to four
+// times through sixteen or more launches.  Bound by launches and the build's
+// latency for small relations (1500 x 2000: 124 -> 53 us a call, 200K x 300K with
+// the filter 233 -> 115 us), by the probe's issue rate for long ones (6001 x 20M:
+// 4.99 -> 0.57 ms; the partitioned path had 32 work items there).  ns_dev, when not null, is the
+// device-side length of S (S' after the filter).  Workgroups of one slice run
+// on one XCD (slices are dealt in multiples of 8), so its keys come from that
+// XCD's L2 after the first chunk.
+template <int BLOCK, int CAP, int PITEMS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_join_direct(
+    const uint32_t* __restrict__ rk, const uint32_t* __restrict__ rv, uint32_t nr,
+    const uint32_t* __restrict__ sk, const uint32_t* __restrict__ sv, uint32_t ns_host,
+    const uint64_t* __restrict__ ns_dev, bool build_r, uint32_t grain, uint64_t* __restrict__ out_count,
+    uint64_t out_cap, uint32_t* __restrict__ o_key, uint32_t* __restrict__ o_rval, uint32_t* __restrict__ o_sval)
+{
+    __shared__ ProbeLds<BLOCK, CAP> L;
+    const uint32_t ns = ns_dev ? (uint32_t)min(*ns_dev, (uint64_t)ns_host) : ns_host;
+    const uint32_t nb = build_r ? nr : ns, np = build_r ? ns : nr;
+    if (nb == 0 || np == 0) return;
+    const uint32_t C = (nb + CAP - 1) / CAP;
+    const uint32_t cper = (nb + C - 1) / C;
+    uint32_t S = max(1u, min(gridDim.x / C, (np + grain - 1) / grain));
+    if (S > 8) S &= ~7u;
+    const uint32_t sper = (np + S - 1) / S;
+    const uint64_t items = (uint64_t)C * S;
+    for (uint64_t item = blockIdx.x; item < items; item += gridDim.x) {
+        const uint32_t c = (uint32_t)(item / S), sl = (uint32_t)(item % S);
+        const uint32_t b0 = min(c * cper, nb), p0 = (uint32_t)min((uint64_t)sl * sper, (uint64_t)np);
+        const int bn = (int)min(cper, nb - b0);
+        const uint32_t pn = min(sper, np - p0);
+        probe_item<BLOCK, CAP, PITEMS>(L, (build_r ? rk : sk) + b0, (build_r ? rv : sv) + b0, bn,
+                                       (build_r ? sk : rk) + p0, (build_r ? sv : rv) + p0, pn, build_r, 0,
+                                       out_count, out_cap, o_key, o_rval, o_sval);
+        __syncthreads();  // the table is rebuilt by the next item
+    }
+}
+
 // ============================================================== launchers
 static int ceil_div_i(uint64_t a, uint64_t b) { return (int)((a + b - 1) / b); }
 
@@ -1269,6 +1330,50 @@ int probe_grid(int tile, int num_cu) { return tile == 8192 ? num_cu * 2 : num_cu
 constexpr int PROBE_ITEMS = 10;
 
 static_assert(PT_N == PROBE_TIMER_SLOTS, "probe timer slots");
+
+hipError_t launch_direct_begin(uint64_t* ctr, int n_ctr, uint64_t* filter, uint64_t blocks, hipStream_t st)
+{
+    const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>(1024, (blocks + 255) / 256));
+    k_direct_begin<<<grid, 256, 0, st>>>(ctr, n_ctr, filter, blocks);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_bloom(const uint32_t* rkey, uint64_t n, const BloomGeom& g, uint64_t* filter,
+                               hipStream_t st)
+{
+    if (n == 0) return hipSuccess;
+    k_direct_bloom<<<ceil_div_i(n, 256), 256, 0, st>>>(rkey, (uint32_t)n, g, filter);
+    return hipGetLastError();
+}
+
+hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t nr, const uint32_t* sk,
+                              const uint32_t* sv, uint64_t ns, const uint64_t* ns_dev, uint64_t* out_count,
+                              uint64_t out_cap, uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, int num_cu,
+                              hipStream_t st)
+{
+    constexpr int CAP = 8192, B = 512;
+    if (nr == 0 || ns == 0) return hipSuccess;
+    const bool build_r = build_from_r(nr, ns, CAP);
+    const uint64_t nb = build_r ? nr : ns, np = build_r ? ns : nr;
+    const uint64_t C = (nb + CAP - 1) / CAP;
+    const uint64_t wgs = (uint64_t)probe_grid(CAP, num_cu);
+    // one short round (2 keys per thread) per workgroup while that fills at most
+    // one wave of workgroups, else rounds of PROBE_ITEMS keys per thread
+    constexpr int SMALL_ITEMS = 2;
+    const uint64_t small_slices = (np + B * SMALL_ITEMS - 1) / (B * SMALL_ITEMS);
+    const bool small = C * small_slices <= wgs;
+    const uint32_t grain = B * (small ? SMALL_ITEMS : PROBE_ITEMS);
+    const int grid = (int)std::min<uint64_t>(wgs, C * std::max<uint64_t>(1, (np + grain - 1) / grain));
+    if (small)
+        k_join_direct<B, CAP, SMALL_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
+                                                               build_r, grain, out_count, out_cap, o_key, o_rval,
+                                                               o_sval);
+    else
+        k_join_direct<B, CAP, PROBE_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
+                                                               build_r, grain, out_count, out_cap, o_key, o_rval,
+                                                               o_sval);
+    return hipGetLastError();
+}
 
 hipError_t launch_probe(int tile, const uint32_t* rk, const uint32_t* rv, const uint64_t* r_start,
                         const uint32_t* sk, const uint32_t* sv, const uint64_t* s_start,

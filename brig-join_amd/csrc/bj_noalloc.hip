@@ -115,6 +115,7 @@ int bj_join_noalloc(bj_ctx* c, const bj_params* p, const uint32_t* r_key, const 
         off += it.second;
     }
     pl.cap = out_cap;
+    pl.direct = choose_direct(*p, pl);
     const bool timing = p->collect_phase_times != 0;
     tl_reset(c, timing);
     g_no_alloc = true;

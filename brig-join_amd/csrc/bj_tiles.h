@@ -745,15 +745,6 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     // the caller synchronises before the next item rebuilds the table
 }
 
-// Build side of a sub-bucket: R whenever it fits one LDS table (the
-// reference's build side), else the smaller side.  Equal S keys, as under a
-// skewed S, then stream past distinct R keys instead of piling up in one run
-// of the table that every matching probe walks.
-__host__ __device__ __forceinline__ bool build_from_r(uint64_t nr, uint64_t ns, uint32_t tile)
-{
-    return nr <= tile || nr <= ns;
-}
-
 // Work-item split of one sub-bucket (vlsplit).  A sub-bucket whose build side
 // (build_from_r) fits one LDS tile and whose probe side fits one slice is
 // "regular": one work item, indexed by the sub-bucket itself.  Larger ones are
