@@ -328,8 +328,8 @@ int make_plan(const bj_params& p, Plan& pl)
 
 // Radix partition of one relation into out_key/out_val with sub-bucket starts
 // in start[0 .. 2^bits], in one or two physical scatter passes (p1 bits, then
-// the rest).  With l1_only, only the first pass runs and its output (grouped by
-// first-pass bucket, in the final positions' ranges) is left in out_key/out_val.
+// the rest).  With l1_only, only the first pass runs and its output (whole tuples
+// grouped by first-pass bucket, in the final positions' ranges) is left in c->tmp.
 int run_partition(bj_ctx* c, const Plan& pl, int p1, const uint32_t* key, const uint32_t* val,
                   uint64_t n_host, const uint64_t* n_dev, int G, bool solo, uint32_t* out_key,
                   uint32_t* out_val, uint64_t out_cap, uint64_t* start, int k_hist, bool l1_only = false)
@@ -356,16 +356,18 @@ int run_partition(bj_ctx* c, const Plan& pl, int p1, const uint32_t* key, const 
                           P<uint32_t>(c->l1h), start,
                           P<uint64_t>(c->l1off), st));
     BJ_HIP(end(k_hist + 1));
-    uint32_t* k1 = two_pass ? P<uint32_t>(c->tmp_key) : out_key;
-    uint32_t* v1 = two_pass ? P<uint32_t>(c->tmp_val) : out_val;
-    const uint64_t cap1 = two_pass ? c->tmp_key.bytes / 4 : out_cap;
+    // a first pass that another kernel reads writes whole tuples into c->tmp
+    const bool first = two_pass || l1_only;
+    uint32_t* k1 = first ? P<uint32_t>(c->tmp) : out_key;
+    const uint64_t cap1 = first ? c->tmp.bytes / 8 : out_cap;
     BJ_HIP(beg(k_hist + 2));
-    BJ_HIP(launch_scatter(key, val, k1, v1, cap1, n_host, n_dev, G, 0, pl.bits, p1, W2,
+    BJ_HIP(launch_scatter(first ? SCATTER_FIRST : SCATTER_ONLY, key, val, k1, first ? nullptr : out_val, cap1, n_host,
+                          n_dev, G, pl.bits, p1, W2,
                           P<uint64_t>(c->l1off), start, P<uint32_t>(c->colsum), err, pl.scatter_wg, min_lds, st));
     BJ_HIP(end(k_hist + 2));
     BJ_HIP(beg(k_hist + 3));
     if (two_pass)
-        BJ_HIP(launch_scatter(k1, v1, out_key, out_val, out_cap, n_host, n_dev, G, 1, pl.bits, p1, W2,
+        BJ_HIP(launch_scatter(SCATTER_SECOND, k1, nullptr, out_key, out_val, out_cap, n_host, n_dev, G, pl.bits, p1, W2,
                               P<uint64_t>(c->l1off), start, P<uint32_t>(c->colsum), err, pl.scatter_wg, min_lds, st));
     BJ_HIP(end(k_hist + 3));
     return BJ_OK;
@@ -389,7 +391,7 @@ int workspace_items(const Plan& pl, bool with_r, bool with_out,
     if ((rc = need(&bj_ctx::s_key, ns * 4)) || (rc = need(&bj_ctx::s_val, ns * 4))) return rc;
     if (pl.p1 < pl.bits || pl.p1_s < pl.bits || (pl.bf && pl.bf_stage == 2)) {
         const uint64_t t = with_r ? std::max(nr, ns) : ns;
-        if ((rc = need(&bj_ctx::tmp_key, t * 4)) || (rc = need(&bj_ctx::tmp_val, t * 4))) return rc;
+        if ((rc = need(&bj_ctx::tmp, t * 8))) return rc;
     }
     if (pl.bf) {
         if (pl.bf_stage == 1) {
@@ -544,13 +546,12 @@ int enqueue_s(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, 
         } else {
             // first-level pass of S, then filter each bucket against its L2-resident
             // filter slice while placing the survivors into their sub-buckets
-            if ((rc = run_partition(c, pl, pl.p1_s, s_key, s_val, pl.ns, nullptr, pl.G_s, pl.solo_s, P<uint32_t>(c->tmp_key),
-                                    P<uint32_t>(c->tmp_val), c->tmp_key.bytes / 4, P<uint64_t>(c->s_start),
-                                    BJ_K_HIST_S, true)))
+            if ((rc = run_partition(c, pl, pl.p1_s, s_key, s_val, pl.ns, nullptr, pl.G_s, pl.solo_s, nullptr,
+                                    nullptr, 0, P<uint64_t>(c->s_start), BJ_K_HIST_S, true)))
                 return rc;
             BJ_HIP(beg(BJ_K_BF_FILTER));
             BJ_HIP(launch_zero_u32(P<uint32_t>(c->s_fill), 1ull << pl.bits, st));
-            BJ_HIP(launch_filter_l1(P<uint32_t>(c->tmp_key), P<uint32_t>(c->tmp_val), P<uint64_t>(c->s_start),
+            BJ_HIP(launch_filter_l1(P<uint32_t>(c->tmp), P<uint64_t>(c->s_start),
                                     pl.bits, pl.bits - pl.p1_s, R.filter, pl.geom, o_key, o_val, o_cap,
                                     P<uint32_t>(c->s_fill),
                                     ctr + CTR_SPRIME, ctr + CTR_XCD, ctr + CTR_ERR, c->num_cu, st));
@@ -736,7 +737,7 @@ int bj_destroy(bj_ctx* c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     DevBuf* bufs[] = {&c->in_rk,  &c->in_rv,    &c->in_sk,   &c->in_sv,    &c->r_key,   &c->r_val,
-                      &c->s_key,  &c->s_val,    &c->tmp_key, &c->tmp_val,  &c->sp_key,  &c->sp_val,
+                      &c->s_key,  &c->s_val,    &c->tmp,  &c->sp_key,  &c->sp_val,
                       &c->filter, &c->part,     &c->totals,  &c->l1h,      &c->l1off,   &c->colsum,  &c->r_start,
                       &c->s_start, &c->s_fill,  &c->partials, &c->items,  &c->counters, &c->out_key,
                       &c->out_rval, &c->out_sval, &c->dtmp,  &c->plan_cnt, &c->item_start, &c->ptimers,
@@ -888,7 +889,7 @@ static uint64_t held_bytes(bj_ctx* c)
 {
     uint64_t t = 0;
     const DevBuf* bufs[] = {&c->in_rk,  &c->in_rv,  &c->in_sk,   &c->in_sv,   &c->r_key,  &c->r_val,
-                            &c->s_key,  &c->s_val,  &c->tmp_key, &c->tmp_val, &c->sp_key, &c->sp_val,
+                            &c->s_key,  &c->s_val,  &c->tmp, &c->sp_key, &c->sp_val,
                             &c->filter, &c->part,   &c->totals,  &c->l1h,     &c->l1off,  &c->colsum,
                             &c->r_start, &c->s_start, &c->s_fill, &c->partials, &c->items, &c->counters,
                             &c->out_key, &c->out_rval, &c->out_sval, &c->dtmp, &c->plan_cnt, &c->item_start,

@@ -339,7 +339,7 @@ struct bj_batch {
     int n = 0;
     Layout L;
     DevBuf dJ, dpx;
-    DevBuf r_key, r_val, s_key, s_val, sp_key, sp_val, tmp_key, tmp_val, part, cur_rel, tot_r, tot_s, start_r, start_s;
+    DevBuf r_key, r_val, s_key, s_val, sp_key, sp_val, tmp, part, cur_rel, tot_r, tot_s, start_r, start_s;
     DevBuf filter, plan_cnt, item_start, partials, items, ctr, out_key, out_rval, out_sval;
     uint64_t* h_ctr = nullptr;  // pinned: jc[n][JC_N], then err
     hipGraph_t graph = nullptr;
@@ -369,8 +369,7 @@ int batch_workspace(bj_batch* b, const Layout& L, int n, uint64_t* total_bytes)
         (rc = need(&bj_batch::r_val, L.tot_r * 4)) || (rc = need(&bj_batch::s_key, L.tot_s * 4)) ||
         (rc = need(&bj_batch::s_val, L.tot_s * 4)) || (rc = need(&bj_batch::sp_key, L.tot_sp * 4)) ||
         (rc = need(&bj_batch::sp_val, L.tot_sp * 4)) ||
-        (rc = need(&bj_batch::tmp_key, L.any_two || L.any_bf2 ? std::max(L.tot_r, L.tot_s) * 4 : 0)) ||
-        (rc = need(&bj_batch::tmp_val, L.any_two || L.any_bf2 ? std::max(L.tot_r, L.tot_s) * 4 : 0)) ||
+        (rc = need(&bj_batch::tmp, L.any_two || L.any_bf2 ? std::max(L.tot_r, L.tot_s) * 8 : 0)) ||
         (rc = need(&bj_batch::part, L.part_n * 4)) ||
         (rc = need(&bj_batch::cur_rel, L.part_n * 4)) || (rc = need(&bj_batch::tot_r, nsb * 4)) ||
         (rc = need(&bj_batch::tot_s, nsb * 4)) || (rc = need(&bj_batch::start_r, nsb * 8)) ||
@@ -417,10 +416,10 @@ int enqueue(bj_batch* b, hipStream_t st)
     for (int k = 0; k < 2; k++)
         BJ_HIP(launch_batch_scatter(B, 0, k, L.nt_p1[0][k], L.max_b1[0][k], nullptr, nullptr, jc,
                                     P<uint32_t>(b->cur_rel), P<uint64_t>(b->start_r), P<uint32_t>(b->r_key),
-                                    P<uint32_t>(b->r_val), b->r_key.bytes / 4, P<uint32_t>(b->tmp_key),
-                                    P<uint32_t>(b->tmp_val), b->tmp_key.bytes / 4, err, k == 1, st));
+                                    P<uint32_t>(b->r_val), b->r_key.bytes / 4, P<uint32_t>(b->tmp),
+                                    b->tmp.bytes / 8, err, k == 1, st));
     BJ_HIP(launch_batch_scatter2(B, 0, L.nt_r2, P<uint32_t>(b->cur_rel), P<uint64_t>(b->start_r),
-                                 P<uint32_t>(b->tot_r), P<uint32_t>(b->tmp_key), P<uint32_t>(b->tmp_val),
+                                 P<uint32_t>(b->tot_r), P<uint32_t>(b->tmp),
                                  P<uint32_t>(b->r_key), P<uint32_t>(b->r_val), b->r_key.bytes / 4, err, big_r,
                                  st));
     // Bloom joins: filter from the partitioned R, then S -> S'
@@ -439,12 +438,11 @@ int enqueue(bj_batch* b, hipStream_t st)
             for (int k = 0; k < 2; k++)
                 BJ_HIP(launch_batch_scatter(B, 2, k, L.nt_p1[2][k], L.max_b1[2][k], nullptr, nullptr, jc,
                                             P<uint32_t>(b->cur_rel), P<uint64_t>(b->start_s),
-                                            P<uint32_t>(b->tmp_key), P<uint32_t>(b->tmp_val),
-                                            b->tmp_key.bytes / 4, P<uint32_t>(b->tmp_key),
-                                            P<uint32_t>(b->tmp_val), b->tmp_key.bytes / 4, err, false, st));
+                                            nullptr, nullptr, 0, P<uint32_t>(b->tmp),
+                                            b->tmp.bytes / 8, err, false, st));
         }
-        BJ_HIP(launch_batch_prefilter(B, L.nf_tiles, P<uint64_t>(b->filter), P<uint32_t>(b->tmp_key),
-                                      P<uint32_t>(b->tmp_val), P<uint32_t>(b->sp_key), P<uint32_t>(b->sp_val), jc,
+        BJ_HIP(launch_batch_prefilter(B, L.nf_tiles, P<uint64_t>(b->filter), P<uint32_t>(b->tmp),
+                                      P<uint32_t>(b->sp_key), P<uint32_t>(b->sp_val), jc,
                                       err + 1, err, num_cu, st));
     }
     // S (or S'): one-level partition into the S arena
@@ -456,10 +454,10 @@ int enqueue(bj_batch* b, hipStream_t st)
         BJ_HIP(launch_batch_scatter(B, 1, k, L.nt_p1[1][k], L.max_b1[1][k], P<uint32_t>(b->sp_key),
                                     P<uint32_t>(b->sp_val), jc, P<uint32_t>(b->cur_rel), P<uint64_t>(b->start_s),
                                     P<uint32_t>(b->s_key), P<uint32_t>(b->s_val), b->s_key.bytes / 4,
-                                    P<uint32_t>(b->tmp_key), P<uint32_t>(b->tmp_val), b->tmp_key.bytes / 4, err,
+                                    P<uint32_t>(b->tmp), b->tmp.bytes / 8, err,
                                     k == 1, st));
     BJ_HIP(launch_batch_scatter2(B, 1, L.nt_s2, P<uint32_t>(b->cur_rel), P<uint64_t>(b->start_s),
-                                 P<uint32_t>(b->tot_s), P<uint32_t>(b->tmp_key), P<uint32_t>(b->tmp_val),
+                                 P<uint32_t>(b->tot_s), P<uint32_t>(b->tmp),
                                  P<uint32_t>(b->s_key), P<uint32_t>(b->s_val), b->s_key.bytes / 4, err, big_s,
                                  st));
     // vlsplit plan and the persistent build + probe, one launch per tile class
@@ -540,7 +538,7 @@ int bj_batch_destroy(bj_batch* b)
     if (b->e0) (void)hipEventDestroy(b->e0);
     if (b->e1) (void)hipEventDestroy(b->e1);
     DevBuf* bufs[] = {&b->dJ,      &b->dpx,     &b->r_key,   &b->r_val,    &b->s_key,      &b->s_val,
-                      &b->sp_key,  &b->sp_val,  &b->tmp_key, &b->tmp_val,  &b->part,       &b->cur_rel,
+                      &b->sp_key,  &b->sp_val,  &b->tmp,  &b->part,       &b->cur_rel,
                       &b->tot_r,   &b->tot_s,
                       &b->start_r, &b->start_s, &b->filter,  &b->plan_cnt, &b->item_start, &b->partials,
                       &b->items,   &b->ctr,     &b->out_key, &b->out_rval, &b->out_sval};

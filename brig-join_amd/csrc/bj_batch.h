@@ -79,7 +79,8 @@ hipError_t launch_batch_colscan(const BatchDev& B, int side, uint32_t ncolblk, c
 hipError_t launch_batch_binscan(const BatchDev& B, int side, const uint32_t* tot, uint64_t* start,
                                 hipStream_t st);
 // First pass: every join's chunks by its first-pass bits, to the final arena
-// (one-pass joins) or to the scratch arena tkey/tval at the final positions.
+// (one-pass joins) or, as whole 8-byte tuples, to the scratch arena tmp (tmp_cap
+// tuples) at the final positions.
 // One launch per class cls of first passes (ntasks tasks, PX_P1 + 2 * side + cls),
 // with LDS for max_b1 bits.  big: one workgroup per CU with 8192-tuple tiles and
 // whole-line carries (the class of wide first passes), else two per CU with
@@ -87,13 +88,13 @@ hipError_t launch_batch_binscan(const BatchDev& B, int side, const uint32_t* tot
 hipError_t launch_batch_scatter(const BatchDev& B, int side, int cls, uint32_t ntasks, int max_b1,
                                 const uint32_t* sp_key, const uint32_t* sp_val, const uint64_t* jc,
                                 const uint32_t* cur_rel, const uint64_t* start, uint32_t* okey, uint32_t* oval,
-                                uint64_t out_cap, uint32_t* tkey, uint32_t* tval, uint64_t tmp_cap, uint64_t* err,
-                                bool big, hipStream_t st);
+                                uint64_t out_cap, uint32_t* tmp, uint64_t tmp_cap, uint64_t* err, bool big,
+                                hipStream_t st);
 // Second pass of two-pass joins: scratch arena -> final arena.  big: one
 // workgroup per CU with 8192-tuple tiles (for launches over many tuples).
 hipError_t launch_batch_scatter2(const BatchDev& B, int side, uint32_t ntasks, const uint32_t* cur_rel,
-                                 const uint64_t* start, const uint32_t* cnt, const uint32_t* tkey,
-                                 const uint32_t* tval, uint32_t* okey, uint32_t* oval, uint64_t out_cap,
+                                 const uint64_t* start, const uint32_t* cnt, const uint32_t* tmp,
+                                 uint32_t* okey, uint32_t* oval, uint64_t out_cap,
                                  uint64_t* err, bool big, hipStream_t st);
 hipError_t launch_batch_bloom_build(const BatchDev& B, uint32_t nseg, uint32_t max_wps, const uint32_t* rkey,
                                     const uint64_t* r_start, const uint32_t* r_cnt, uint64_t* filter,
@@ -102,8 +103,8 @@ hipError_t launch_batch_bloom_build(const BatchDev& B, uint32_t nseg, uint32_t m
 // XCD x working through the x-th eighth of them on its own counter xctr[x]
 // (NXCD counters, zeroed).
 hipError_t launch_batch_prefilter(const BatchDev& B, uint32_t ntiles, const uint64_t* filter,
-                                  const uint32_t* tkey, const uint32_t* tval, uint32_t* sp_key,
-                                  uint32_t* sp_val, uint64_t* jc, uint64_t* xctr, uint64_t* err, int num_cu,
+                                  const uint32_t* tmp, uint32_t* sp_key, uint32_t* sp_val,
+                                  uint64_t* jc, uint64_t* xctr, uint64_t* err, int num_cu,
                                   hipStream_t st);
 hipError_t launch_batch_plan(const BatchDev& B, uint32_t nsb, const uint64_t* r_start, const uint32_t* r_cnt,
                              const uint64_t* s_start, const uint32_t* s_cnt, uint32_t slice,

@@ -195,9 +195,9 @@ __global__ __launch_bounds__(1024) void kb_binscan(BatchDev B, int side, const u
 // than 2^WIDE_B1 buckets, 1: the others).  ITEMS 4: two workgroups per CU,
 // 4096-tuple tiles; ITEMS 8: one per CU, 8192-tuple tiles and whole-line carries
 // up to 256 buckets (the wide class, and large second passes).
-__device__ __forceinline__ int kb_carry_log2(int nbk, bool big)
+__device__ __forceinline__ int kb_carry_log2(int nbk, bool big, bool opair)
 {
-    if (big && nbk <= 256) return 5;
+    if (big && !opair && nbk <= 256) return 5;
     return nbk <= 512 ? 4 : (nbk <= 1024 ? 3 : 2);  // scatter_carry
 }
 
@@ -208,8 +208,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
                                                     const uint32_t* __restrict__ cur_rel,
                                                     const uint64_t* __restrict__ start, uint32_t* __restrict__ okey,
                                                     uint32_t* __restrict__ oval, uint64_t out_cap,
-                                                    uint32_t* __restrict__ tkey, uint32_t* __restrict__ tval,
-                                                    uint64_t tmp_cap, uint64_t* __restrict__ err)
+                                                    Tuple* __restrict__ tmp, uint64_t tmp_cap,
+                                                    uint64_t* __restrict__ err)
 {
     extern __shared__ uint64_t lds64[];
     const uint32_t* px = px_of(B, PX_P1 + 2 * side + cls);
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
     const int bits = side_bits(J, side), b1 = side_b1(J, side);
     const int b2 = bits - b1;
     const int nbk = 1 << b1;
-    const int cs_log2 = kb_carry_log2(nbk, ITEMS == 8);
+    const int cs_log2 = kb_carry_log2(nbk, ITEMS == 8, b2 > 0 || side == 2);
     const ScatterLds L = scatter_lds<BLOCK, ITEMS>(lds64, nbk, cs_log2);
     const uint32_t* cr = cur_rel + (side ? J.part_s : J.part_r) + ((size_t)c << bits);
     const uint64_t* st = start + J.sb_base;
@@ -254,10 +254,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
     side_src(J, b, side, sp_key, sp_val, jc, key, val, n);
     uint64_t lo, hi;
     chunk_range(J, side, c, n, lo, hi);
-    const bool two = b2 > 0;
-    const bool bad = scatter_range<BLOCK, ITEMS>(L, key + lo, val + lo, (uint32_t)(hi - lo), nbk, 32 - b1,
-                                                 (uint32_t)nbk - 1u, cs_log2, two ? tkey : okey, two ? tval : oval,
-                                                 two ? tmp_cap : out_cap);
+    // side 2 and the first of two passes: whole tuples into the scratch arena
+    auto run = [&](auto out, uint64_t cap) {
+        return scatter_range<BLOCK, ITEMS>(L, TupleIn<false>{key + lo, val + lo}, (uint32_t)(hi - lo), nbk, 32 - b1,
+                                           (uint32_t)nbk - 1u, cs_log2, out, cap);
+    };
+    const bool bad = b2 > 0 || side == 2 ? run(TupleOut<true>{tmp}, tmp_cap) : run(TupleOut<false>{okey, oval}, out_cap);
     if (bad) atomicOr((unsigned long long*)err, 16ull);
 }
 
@@ -269,8 +271,7 @@ template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 4 ? 8 : 4, 8))) void kb_scatter2(BatchDev B, int side, const uint32_t* __restrict__ cur_rel,
                                                      const uint64_t* __restrict__ start,
                                                      const uint32_t* __restrict__ cnt,
-                                                     const uint32_t* __restrict__ tkey,
-                                                     const uint32_t* __restrict__ tval, uint32_t* __restrict__ okey,
+                                                     const Tuple* __restrict__ tmp, uint32_t* __restrict__ okey,
                                                      uint32_t* __restrict__ oval, uint64_t out_cap,
                                                      uint64_t* __restrict__ err)
 {
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
     const int nbk = 1 << b2;
     const int G = (int)side_chunks(J, side);
     const int g0 = (int)(((int64_t)w * G) / W2), g1 = (int)(((int64_t)(w + 1) * G) / W2);
-    const int cs_log2 = kb_carry_log2(nbk, ITEMS == 8);
+    const int cs_log2 = kb_carry_log2(nbk, ITEMS == 8, false);
     const ScatterLds L = scatter_lds<BLOCK, ITEMS>(lds64, nbk, cs_log2);
     const size_t f0 = (size_t)bb << b2;  // first sub-bucket of the bucket, within the join
     const uint32_t* base = cur_rel + (side ? J.part_s : J.part_r);
@@ -308,8 +309,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
     }
     __syncthreads();
     const uint64_t lo = st[0] + s_lo, hi = st[0] + s_hi;
-    const bool bad = scatter_range<BLOCK, ITEMS>(L, tkey + lo, tval + lo, (uint32_t)(hi - lo), nbk, 32 - J.bits,
-                                                 (uint32_t)nbk - 1u, cs_log2, okey, oval, out_cap);
+    const bool bad = scatter_range<BLOCK, ITEMS>(L, TupleIn<true>{tmp + lo}, (uint32_t)(hi - lo), nbk, 32 - J.bits,
+                                                 (uint32_t)nbk - 1u, cs_log2, TupleOut<false>{okey, oval}, out_cap);
     if (bad) atomicOr((unsigned long long*)err, 64ull);
 }
 
@@ -355,8 +356,7 @@ __global__ __launch_bounds__(BLOCK) void kb_bloom_build(BatchDev B, const uint32
 template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void kb_prefilter(BatchDev B, uint32_t ntiles,
                                                       const uint64_t* __restrict__ filter,
-                                                      const uint32_t* __restrict__ tkey,
-                                                      const uint32_t* __restrict__ tval,
+                                                      const Tuple* __restrict__ tmp,
                                                       uint32_t* __restrict__ sp_key, uint32_t* __restrict__ sp_val,
                                                       uint64_t* __restrict__ jc, uint64_t* __restrict__ xctr,
                                                       uint64_t* __restrict__ err)
@@ -381,11 +381,13 @@ __global__ __launch_bounds__(BLOCK) void kb_prefilter(BatchDev B, uint32_t ntile
         const int b = find_join(px, B.n, g);
         const BJoin J = B.J[b];
         const uint64_t tile = (uint64_t)(g - px[b]) * T;
-        const uint32_t* sk = J.bf2 ? tkey + J.s_base : J.sk;
-        const uint32_t* sv = J.bf2 ? tval + J.s_base : J.sv;
-        bad |= prefilter_tile<BLOCK, ITEMS>(sk, sv, tile, J.ns, filter + J.f_base, J.geom, sp_key + J.sp_base,
-                                            sp_val + J.sp_base, J.ns, jc + (size_t)b * JC_N + JC_SPRIME, gcnt,
-                                            &s_base);
+        auto run = [&](auto in) {
+            bad |= prefilter_tile<BLOCK, ITEMS>(in, tile, J.ns, filter + J.f_base, J.geom, sp_key + J.sp_base,
+                                                sp_val + J.sp_base, J.ns, jc + (size_t)b * JC_N + JC_SPRIME, gcnt,
+                                                &s_base);
+        };
+        if (J.bf2) run(TupleIn<true>{tmp + J.s_base});
+        else run(TupleIn<false>{J.sk, J.sv});
         t = s_next;
         __syncthreads();  // s_next is rewritten for the next tile
     }
@@ -559,37 +561,38 @@ hipError_t launch_batch_binscan(const BatchDev& B, int side, const uint32_t* tot
 hipError_t launch_batch_scatter(const BatchDev& B, int side, int cls, uint32_t ntasks, int max_b1,
                                 const uint32_t* sp_key, const uint32_t* sp_val, const uint64_t* jc,
                                 const uint32_t* cur_rel, const uint64_t* start, uint32_t* okey, uint32_t* oval,
-                                uint64_t out_cap, uint32_t* tkey, uint32_t* tval, uint64_t tmp_cap, uint64_t* err,
-                                bool big, hipStream_t st)
+                                uint64_t out_cap, uint32_t* tmp, uint64_t tmp_cap, uint64_t* err, bool big,
+                                hipStream_t st)
 {
     if (ntasks == 0) return hipSuccess;
     if (side < 0 || side > 2 || cls < 0 || cls > 1) return hipErrorInvalidValue;
     const size_t lds_big = std::max(scatter_lds_bytes_big(1 << max_b1), g_max_lds_b / 2 + 1024);
     if (big && lds_big <= g_max_lds_b) {
         kb_scatter<BS_BLOCK, 2 * BS_ITEMS><<<ntasks, BS_BLOCK, lds_big, st>>>(
-            B, side, cls, sp_key, sp_val, jc, cur_rel, start, okey, oval, out_cap, tkey, tval, tmp_cap, err);
+            B, side, cls, sp_key, sp_val, jc, cur_rel, start, okey, oval, out_cap, (Tuple*)tmp, tmp_cap, err);
         return hipGetLastError();
     }
     const size_t lds = scatter_lds_bytes(1 << max_b1);
     kb_scatter<BS_BLOCK, BS_ITEMS><<<ntasks, BS_BLOCK, lds, st>>>(B, side, cls, sp_key, sp_val, jc, cur_rel, start,
-                                                                  okey, oval, out_cap, tkey, tval, tmp_cap, err);
+                                                                  okey, oval, out_cap, (Tuple*)tmp, tmp_cap, err);
     return hipGetLastError();
 }
 
 hipError_t launch_batch_scatter2(const BatchDev& B, int side, uint32_t ntasks, const uint32_t* cur_rel,
-                                 const uint64_t* start, const uint32_t* cnt, const uint32_t* tkey,
-                                 const uint32_t* tval, uint32_t* okey, uint32_t* oval, uint64_t out_cap,
+                                 const uint64_t* start, const uint32_t* cnt, const uint32_t* tmp,
+                                 uint32_t* okey, uint32_t* oval, uint64_t out_cap,
                                  uint64_t* err, bool big, hipStream_t st)
 {
     if (ntasks == 0) return hipSuccess;
     const size_t lds_big = std::max(scatter_lds_bytes_big(1 << std::max(1, B.max_b2)), g_max_lds_b / 2 + 1024);
     if (big && lds_big <= g_max_lds_b) {
-        kb_scatter2<BS_BLOCK, 2 * BS_ITEMS><<<ntasks, BS_BLOCK, lds_big, st>>>(B, side, cur_rel, start, cnt, tkey,
-                                                                             tval, okey, oval, out_cap, err);
+        kb_scatter2<BS_BLOCK, 2 * BS_ITEMS><<<ntasks, BS_BLOCK, lds_big, st>>>(B, side, cur_rel, start, cnt,
+                                                                               (const Tuple*)tmp, okey, oval, out_cap,
+                                                                               err);
         return hipGetLastError();
     }
     const size_t lds = scatter_lds_bytes(1 << std::max(1, B.max_b2));
-    kb_scatter2<BS_BLOCK, BS_ITEMS><<<ntasks, BS_BLOCK, lds, st>>>(B, side, cur_rel, start, cnt, tkey, tval,
+    kb_scatter2<BS_BLOCK, BS_ITEMS><<<ntasks, BS_BLOCK, lds, st>>>(B, side, cur_rel, start, cnt, (const Tuple*)tmp,
                                                                    okey, oval, out_cap, err);
     return hipGetLastError();
 }
@@ -604,14 +607,14 @@ hipError_t launch_batch_bloom_build(const BatchDev& B, uint32_t nseg, uint32_t m
 }
 
 hipError_t launch_batch_prefilter(const BatchDev& B, uint32_t ntiles, const uint64_t* filter,
-                                  const uint32_t* tkey, const uint32_t* tval, uint32_t* sp_key,
-                                  uint32_t* sp_val, uint64_t* jc, uint64_t* xctr, uint64_t* err, int num_cu,
+                                  const uint32_t* tmp, uint32_t* sp_key, uint32_t* sp_val,
+                                  uint64_t* jc, uint64_t* xctr, uint64_t* err, int num_cu,
                                   hipStream_t st)
 {
     if (ntiles == 0) return hipSuccess;
     // four workgroups per CU, a multiple of NXCD
     const uint32_t grid = (uint32_t)std::max(1, num_cu / NXCD) * 4u * NXCD;
-    kb_prefilter<PF_BLOCK, PF_ITEMS><<<grid, PF_BLOCK, 0, st>>>(B, ntiles, filter, tkey, tval, sp_key, sp_val, jc,
+    kb_prefilter<PF_BLOCK, PF_ITEMS><<<grid, PF_BLOCK, 0, st>>>(B, ntiles, filter, (const Tuple*)tmp, sp_key, sp_val, jc,
                                                                 xctr, err);
     return hipGetLastError();
 }

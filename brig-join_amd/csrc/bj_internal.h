@@ -148,7 +148,8 @@ struct bj_ctx {
     // inputs copied from the host (only when inputs_on_device == 0)
     bj::DevBuf in_rk, in_rv, in_sk, in_sv;
     // partitioned relations and scratch
-    bj::DevBuf r_key, r_val, s_key, s_val, tmp_key, tmp_val, sp_key, sp_val;
+    bj::DevBuf r_key, r_val, s_key, s_val, sp_key, sp_val;
+    bj::DevBuf tmp;  // whole 8-byte tuples between a first pass and the kernel that reads it
     bj::DevBuf filter, part, totals, l1h, l1off, colsum, r_start, s_start, s_fill, partials, items, counters;
     bj::DevBuf plan_cnt, item_start;
     bj::DevBuf out_key, out_rval, out_sval, dtmp;

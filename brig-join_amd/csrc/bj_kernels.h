@@ -53,13 +53,18 @@ int scatter_carry(int nbk);
 size_t scatter_lds_bytes(int nbk);
 // LDS of a 1024-thread, 8192-tuple tile with the carries of scatter_carry_big
 size_t scatter_lds_bytes_big(int nbk);
-// pass 1 (mode 0): p1-bit buckets; pass 2 (mode 1): the remaining bits, W2
-// workgroups per pass-1 bucket, cursors from sb_start and colsum.  The launch reserves at
-// least min_lds bytes of LDS per workgroup (a way to cap workgroups per CU).
-hipError_t launch_scatter(const uint32_t* ikey, const uint32_t* ival, uint32_t* okey, uint32_t* oval,
-                          uint64_t out_cap, uint64_t n_host, const uint64_t* n_dev, int G, int mode,
-                          int bits, int p1, int W2, const uint64_t* l1off, const uint64_t* sb_start,
-                          const uint32_t* colsum, uint64_t* err, int wg, size_t min_lds, hipStream_t st);
+// One pass of a partition.  SCATTER_ONLY: the partition's only pass (p1 = bits),
+// keys and values in two arrays on both sides.  SCATTER_FIRST: by the top p1
+// bits, into whole 8-byte tuples (key, value) at okey (8-byte aligned, oval
+// unused).  SCATTER_SECOND: those tuples (ikey, ival unused) by the remaining
+// bits, W2 workgroups per first-pass bucket, cursors from sb_start and colsum,
+// into two arrays.  out_cap is in tuples.  The launch reserves at least min_lds
+// bytes of LDS per workgroup (a way to cap workgroups per CU).
+enum { SCATTER_ONLY = 0, SCATTER_FIRST, SCATTER_SECOND };
+hipError_t launch_scatter(int pass, const uint32_t* ikey, const uint32_t* ival, uint32_t* okey, uint32_t* oval,
+                          uint64_t out_cap, uint64_t n_host, const uint64_t* n_dev, int G, int bits, int p1, int W2,
+                          const uint64_t* l1off, const uint64_t* sb_start, const uint32_t* colsum, uint64_t* err,
+                          int wg, size_t min_lds, hipStream_t st);
 hipError_t launch_bloom_build(const uint32_t* rkey, const uint64_t* r_start, int bits,
                               const BloomGeom& g, uint64_t* filter, hipStream_t st);
 hipError_t launch_bloom_prefilter(const uint32_t* skey, const uint32_t* sval, uint64_t n,
@@ -67,7 +72,8 @@ hipError_t launch_bloom_prefilter(const uint32_t* skey, const uint32_t* sval, ui
                                   uint32_t* oval, uint64_t out_cap, uint64_t* count, uint64_t* err,
                                   int num_cu, hipStream_t st);
 // tile_ctr: 8 zeroed counters, one per XCD (the tile order of each XCD)
-hipError_t launch_filter_l1(const uint32_t* ikey, const uint32_t* ival, const uint64_t* sb_start, int bits,
+// (tuples: S after SCATTER_FIRST)
+hipError_t launch_filter_l1(const uint32_t* tuples, const uint64_t* sb_start, int bits,
                             int bits2, const uint64_t* filter, const BloomGeom& g, uint32_t* okey,
                             uint32_t* oval, uint64_t out_cap, uint32_t* s_fill, uint64_t* count,
                             uint64_t* tile_ctr, uint64_t* err, int num_cu, hipStream_t st);

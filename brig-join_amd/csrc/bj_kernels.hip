@@ -412,10 +412,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(const uint32_t* __rest
 // one for the 8192-tuple tile (launched one per CU), three 512-thread ones.
 constexpr int sc_min_waves(int block, int items) { return block == 1024 ? (items == 4 ? 8 : 4) : 6; }
 
-template <int BLOCK, int ITEMS>
+// IPAIR / OPAIR: whole tuples in one array (TupleIn / TupleOut) on that side.
+template <int BLOCK, int ITEMS, bool IPAIR, bool OPAIR>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sc_min_waves(BLOCK, ITEMS), 8))) void k_scatter(
-    const uint32_t* __restrict__ ikey, const uint32_t* __restrict__ ival,
-    uint32_t* __restrict__ okey, uint32_t* __restrict__ oval, uint64_t out_cap,
+    TupleIn<IPAIR> in, TupleOut<OPAIR> out, uint64_t out_cap,
     uint64_t n_host, const uint64_t* __restrict__ n_dev, int G, int mode, int bits, int p1, int W2,
     int cs_log2, const uint64_t* __restrict__ l1off, const uint64_t* __restrict__ sb_start,
     const uint32_t* __restrict__ colsum, uint64_t* __restrict__ err)
@@ -450,8 +450,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sc_min_wa
         }
     }
     // ranges are below 2^31 tuples
-    const bool bad = scatter_range<BLOCK, ITEMS>(L, ikey + lo, ival + lo, (uint32_t)(hi - lo), nbk, shift,
-                                                 bmask, cs_log2, okey, oval, out_cap);
+    const bool bad = scatter_range<BLOCK, ITEMS, IPAIR, OPAIR>(L, in.from(lo), (uint32_t)(hi - lo), nbk, shift, bmask,
+                                                               cs_log2, out, out_cap);
     if (bad) atomicOr((unsigned long long*)err, 1ull);
 }
 
@@ -494,8 +494,8 @@ __global__ __launch_bounds__(BLOCK) void k_bloom_prefilter(
     __shared__ uint64_t s_base;
     bool bad = false;
     for (uint64_t tile = (uint64_t)blockIdx.x * T; tile < n; tile += (uint64_t)gridDim.x * T)
-        bad |= prefilter_tile<BLOCK, ITEMS>(skey, sval, tile, n, filter, g, okey, oval, out_cap, count, gcnt,
-                                            &s_base);
+        bad |= prefilter_tile<BLOCK, ITEMS, false>({skey, sval}, tile, n, filter, g, okey, oval, out_cap, count, gcnt,
+                                                   &s_base);
     if (bad) atomicOr((unsigned long long*)err, 2ull);
 }
 
@@ -540,8 +540,7 @@ __device__ __forceinline__ void filter_walk_to(FilterWalk& w, uint64_t t, const 
 // K: the filter's bits per key when fixed at compile time (3 or 4), 0 = g.k.
 template <int BLOCK, int ITEMS, int K>
 __global__ __launch_bounds__(BLOCK) void k_filter_l1(
-    const uint32_t* __restrict__ ikey, const uint32_t* __restrict__ ival,
-    const uint64_t* __restrict__ sb_start, int bits, int bits2, const uint64_t* __restrict__ filter,
+    TupleIn<true> in, const uint64_t* __restrict__ sb_start, int bits, int bits2, const uint64_t* __restrict__ filter,
     BloomGeom g, uint32_t* __restrict__ okey, uint32_t* __restrict__ oval, uint64_t out_cap,
     uint32_t* __restrict__ s_fill, uint64_t* __restrict__ count, uint64_t* __restrict__ tile_ctr,
     uint64_t* __restrict__ err)
@@ -553,9 +552,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
     const uint32_t bmask = (uint32_t)P2 - 1u;
     extern __shared__ uint64_t lds64[];
     uint64_t* dst0 = lds64;                       // [P2] sub-bucket start + reserved base
-    uint32_t* skey = (uint32_t*)(dst0 + P2);      // [T]
-    uint32_t* sval = skey + T;                    // [T]
-    uint32_t* cnt0 = sval + T;                    // [2 * P2] survivors per sub-bucket (two tiles)
+    Tuple* stage = (Tuple*)(dst0 + P2);           // [T]
+    uint32_t* cnt0 = (uint32_t*)(stage + T);      // [2 * P2] survivors per sub-bucket (two tiles)
     uint32_t* off = cnt0 + 2 * P2;                // [P2]
     uint32_t* wtmp = off + P2;                    // [BLOCK/64 + 1]
     __shared__ uint32_t s_total;
@@ -593,13 +591,12 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
     int p = wk.p;
     uint64_t tile = wk.lo + (s_tile - wk.tb) * (uint64_t)T;
     uint64_t chi = min(tile + (uint64_t)T, wk.hi);
-    uint32_t nk[ITEMS];
+    Tuple nk[ITEMS];
     if (p < P1) {
+        const TupleIn<true> src = in.from(tile);
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) {
-            const uint64_t i = tile + (uint64_t)it * BLOCK + threadIdx.x;
-            nk[it] = (i < chi) ? __builtin_nontemporal_load(&ikey[i]) : 0u;
-        }
+        for (int it = 0; it < ITEMS; it++)
+            nk[it] = src.load(min((uint32_t)it * BLOCK + threadIdx.x, (uint32_t)(chi - 1 - tile)));
     }
 
     // Per tile three barriers: test + rank | offsets and reservations (one wave;
@@ -612,28 +609,26 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
         // the tile number after the next one, in flight during this tile
         unsigned long long t_after = 0ull;
         if (threadIdx.x == 0) t_after = atomicAdd(xctr, 1ull);
-        uint32_t k[ITEMS], bk[ITEMS], rk[ITEMS];
+        uint32_t bk[ITEMS], rk[ITEMS];
+        Tuple k[ITEMS];
         bool pass[ITEMS];
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) {
-            const int s = it * BLOCK + threadIdx.x;
-            k[it] = (s < tn) ? nk[it] : 0u;
-        }
+        for (int it = 0; it < ITEMS; it++) k[it] = nk[it];
         // all filter words of the tile in flight before any is tested.  The
-        // loads are unconditional (a lane past the tile reads the word of key
-        // 0): loads under a branch, with addresses from earlier loads, would
-        // each wait for all loads before them.
+        // loads are unconditional (a lane past the tile holds its last key):
+        // loads under a branch, with addresses from earlier loads, would each
+        // wait for all loads before them.
         uint64_t fw[ITEMS];
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it], g)];
+        for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it].x, g)];
 #pragma unroll
         for (int it = 0; it < ITEMS; it++) {
             const int s = it * BLOCK + threadIdx.x;
-            const uint64_t m = K ? bloom_mask_k<(K ? K : 1)>(k[it]) : bloom_mask(k[it], g.k);
+            const uint64_t m = K ? bloom_mask_k<(K ? K : 1)>(k[it].x) : bloom_mask(k[it].x, g.k);
             const bool ok = s < tn && (fw[it] & m) == m;
             pass[it] = ok;
             if (ok) {
-                bk[it] = (radix_hash(k[it]) >> shift) & bmask;
+                bk[it] = (radix_hash(k[it].x) >> shift) & bmask;
                 rk[it] = atomicAdd(&cnt[bk[it]], 1u);
             }
         }
@@ -666,45 +661,33 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
                 cnext[b] = 0u;
             }
         }
-        // survivors' values: loads first, then the LDS stores
-        uint32_t vv[ITEMS];
-#pragma unroll
-        for (int it = 0; it < ITEMS; it++)
-            if (pass[it]) vv[it] = __builtin_nontemporal_load(&ival[tile + it * BLOCK + threadIdx.x]);
         __syncthreads();
-        // the next tile: its keys are issued after this tile's value loads, so no
-        // wait of this tile covers them (clamped rather than skipped past the end,
-        // as above)
+        // the next tile, in flight while this one is written out (clamped rather
+        // than skipped past the end, as above)
         filter_walk_to(wk, t_next, sb_start, P1, bits2, T);
         const int p_next = wk.p;
         const uint64_t tile_next = wk.lo + (t_next - wk.tb) * (uint64_t)T;
         const uint64_t chi_next = min(tile_next + (uint64_t)T, wk.hi);
         if (p_next < P1) {
+            const TupleIn<true> src = in.from(tile_next);
+            const uint32_t last = (uint32_t)(chi_next - 1 - tile_next);
 #pragma unroll
-            for (int it = 0; it < ITEMS; it++) {
-                const uint64_t i = min(tile_next + (uint64_t)it * BLOCK + threadIdx.x, chi_next - 1);
-                nk[it] = __builtin_nontemporal_load(&ikey[i]);
-            }
+            for (int it = 0; it < ITEMS; it++) nk[it] = src.load(min((uint32_t)it * BLOCK + threadIdx.x, last));
         }
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) {
-            if (pass[it]) {
-                const uint32_t q = off[bk[it]] + rk[it];
-                skey[q] = k[it];
-                sval[q] = vv[it];
-            }
-        }
+        for (int it = 0; it < ITEMS; it++)
+            if (pass[it]) stage[off[bk[it]] + rk[it]] = k[it];
         // publish the tile number after the next (thread 0 waits for it only here)
         if (threadIdx.x == 0) s_tile = t_after;
         __syncthreads();
         const uint32_t ts = s_total;
         for (uint32_t q = threadIdx.x; q < ts; q += BLOCK) {
-            const uint32_t kk = skey[q];
-            const uint32_t b = (radix_hash(kk) >> shift) & bmask;
+            const Tuple x = stage[q];
+            const uint32_t b = (radix_hash(x.x) >> shift) & bmask;
             const uint64_t d = dst0[b] + (q - off[b]);
             if (d < out_cap) {
-                okey[d] = kk;
-                oval[d] = sval[q];
+                okey[d] = x.x;
+                oval[d] = x.y;
             } else {
                 bad = true;
             }
@@ -1132,13 +1115,22 @@ static hipError_t set_lds(const void* fn, size_t bytes)
                                (int)(bytes > stat ? bytes - stat : 0));
 }
 
+template <bool IPAIR, bool OPAIR>
+static hipError_t set_scatter_lds(int bytes)
+{
+    hipError_t e;
+    if ((e = set_lds((const void*)k_scatter<SC_BLOCK, SC_ITEMS, IPAIR, OPAIR>, bytes)) != hipSuccess) return e;
+    if ((e = set_lds((const void*)k_scatter<SC_BLOCK / 2, SC_ITEMS * 2, IPAIR, OPAIR>, bytes)) != hipSuccess) return e;
+    return set_lds((const void*)k_scatter<SC_BLOCK, SC_BIG_ITEMS, IPAIR, OPAIR>, bytes);
+}
+
 hipError_t kernels_init(int max_lds_bytes)
 {
     hipError_t e;
     if ((e = set_lds((const void*)k_hist<HIST_BLOCK>, max_lds_bytes)) != hipSuccess) return e;
-    if ((e = set_lds((const void*)k_scatter<SC_BLOCK, SC_ITEMS>, max_lds_bytes)) != hipSuccess) return e;
-    if ((e = set_lds((const void*)k_scatter<SC_BLOCK / 2, SC_ITEMS * 2>, max_lds_bytes)) != hipSuccess) return e;
-    if ((e = set_lds((const void*)k_scatter<SC_BLOCK, SC_BIG_ITEMS>, max_lds_bytes)) != hipSuccess) return e;
+    if ((e = set_scatter_lds<false, false>(max_lds_bytes)) != hipSuccess) return e;
+    if ((e = set_scatter_lds<false, true>(max_lds_bytes)) != hipSuccess) return e;
+    if ((e = set_scatter_lds<true, false>(max_lds_bytes)) != hipSuccess) return e;
     g_max_lds = (size_t)max_lds_bytes;
     if ((e = set_lds((const void*)k_bloom_build<1024>, max_lds_bytes)) != hipSuccess) return e;
     if ((e = set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, 0>, max_lds_bytes)) != hipSuccess) return e;
@@ -1200,48 +1192,66 @@ static int log2i(int x)
 }
 
 // One-workgroup-per-CU launches have the CU's LDS to themselves: whole 128-byte
-// lines of keys and of values per carried chunk up to 256 buckets.
-static int scatter_carry_big(int nbk) { return nbk <= 256 ? 32 : scatter_carry(nbk); }
+// lines of keys and of values per carried chunk up to 256 buckets.  (Tuples
+// written whole fill a 128-byte line with a chunk of 16.)
+static int scatter_carry_big(int nbk, bool opair) { return !opair && nbk <= 256 ? 32 : scatter_carry(nbk); }
 
 static size_t scatter_lds_tile(int nbk, int tile, int cs)
 {
-    return (size_t)nbk * 8 + (size_t)nbk * cs * 8 + (size_t)tile * 8 + (size_t)nbk * 20 + (SC_BLOCK / WAVE + 1) * 4;
+    return (size_t)nbk * SCATTER_BUCKET_BYTES + (size_t)nbk * cs * 8 + (size_t)tile * 8 + (SC_BLOCK / WAVE + 1) * 4;
 }
 
 size_t scatter_lds_bytes(int nbk) { return scatter_lds_tile(nbk, SC_BLOCK * SC_ITEMS, scatter_carry(nbk)); }
 
 size_t scatter_lds_bytes_big(int nbk)
 {
-    return scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, scatter_carry_big(nbk));
+    return scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, scatter_carry_big(nbk, false));
 }
 
-hipError_t launch_scatter(const uint32_t* ikey, const uint32_t* ival, uint32_t* okey, uint32_t* oval,
-                          uint64_t out_cap, uint64_t n_host, const uint64_t* n_dev, int G, int mode,
-                          int bits, int p1, int W2, const uint64_t* l1off, const uint64_t* sb_start,
-                          const uint32_t* colsum, uint64_t* err, int wg, size_t min_lds, hipStream_t st)
+template <bool IPAIR, bool OPAIR>
+static hipError_t scatter_pass(TupleIn<IPAIR> in, TupleOut<OPAIR> out, uint64_t out_cap, uint64_t n_host,
+                               const uint64_t* n_dev, int G, int mode, int bits, int p1, int W2,
+                               const uint64_t* l1off, const uint64_t* sb_start, const uint32_t* colsum, uint64_t* err,
+                               int wg, size_t min_lds, hipStream_t st)
 {
     const int nbk = (mode == 0) ? (1 << p1) : (1 << (bits - p1));
     const int grid = (mode == 0) ? G : (1 << p1) * W2;
     const int cs = log2i(scatter_carry(nbk));
     const size_t lds = std::max(scatter_lds_bytes(nbk), min_lds);
-    const int cs_big = scatter_carry_big(nbk);
+    const int cs_big = scatter_carry_big(nbk, OPAIR);
     const size_t lds_big = std::max(scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, cs_big), min_lds);
     if (wg != 512 && min_lds > 0 && lds_big <= g_max_lds) {
         // one workgroup per CU: twice the tile, twice the loads in flight, whole-line carries
-        k_scatter<SC_BLOCK, SC_BIG_ITEMS><<<grid, SC_BLOCK, lds_big, st>>>(
-            ikey, ival, okey, oval, out_cap, n_host, n_dev, G, mode, bits, p1, W2, log2i(cs_big), l1off, sb_start, colsum,
-            err);
+        k_scatter<SC_BLOCK, SC_BIG_ITEMS, IPAIR, OPAIR><<<grid, SC_BLOCK, lds_big, st>>>(
+            in, out, out_cap, n_host, n_dev, G, mode, bits, p1, W2, log2i(cs_big), l1off, sb_start, colsum, err);
     } else if (wg == 512) {
         // same tile (4096 tuples), half the threads: more workgroups per CU
-        k_scatter<SC_BLOCK / 2, SC_ITEMS * 2><<<grid, SC_BLOCK / 2, lds, st>>>(
-            ikey, ival, okey, oval, out_cap, n_host, n_dev, G, mode, bits, p1, W2, cs, l1off, sb_start, colsum,
-            err);
+        k_scatter<SC_BLOCK / 2, SC_ITEMS * 2, IPAIR, OPAIR><<<grid, SC_BLOCK / 2, lds, st>>>(
+            in, out, out_cap, n_host, n_dev, G, mode, bits, p1, W2, cs, l1off, sb_start, colsum, err);
     } else {
-        k_scatter<SC_BLOCK, SC_ITEMS><<<grid, SC_BLOCK, lds, st>>>(
-            ikey, ival, okey, oval, out_cap, n_host, n_dev, G, mode, bits, p1, W2, cs, l1off, sb_start, colsum,
-            err);
+        k_scatter<SC_BLOCK, SC_ITEMS, IPAIR, OPAIR><<<grid, SC_BLOCK, lds, st>>>(
+            in, out, out_cap, n_host, n_dev, G, mode, bits, p1, W2, cs, l1off, sb_start, colsum, err);
     }
     return hipGetLastError();
+}
+
+hipError_t launch_scatter(int pass, const uint32_t* ikey, const uint32_t* ival, uint32_t* okey, uint32_t* oval,
+                          uint64_t out_cap, uint64_t n_host, const uint64_t* n_dev, int G, int bits, int p1, int W2,
+                          const uint64_t* l1off, const uint64_t* sb_start, const uint32_t* colsum, uint64_t* err,
+                          int wg, size_t min_lds, hipStream_t st)
+{
+    switch (pass) {
+    case SCATTER_ONLY:
+        return scatter_pass<false, false>({ikey, ival}, {okey, oval}, out_cap, n_host, n_dev, G, 0, bits, p1, W2,
+                                          l1off, sb_start, colsum, err, wg, min_lds, st);
+    case SCATTER_FIRST:
+        return scatter_pass<false, true>({ikey, ival}, {(Tuple*)okey}, out_cap, n_host, n_dev, G, 0, bits, p1, W2,
+                                         l1off, sb_start, colsum, err, wg, min_lds, st);
+    case SCATTER_SECOND:
+        return scatter_pass<true, false>({(const Tuple*)ikey}, {okey, oval}, out_cap, n_host, n_dev, G, 1, bits, p1,
+                                         W2, l1off, sb_start, colsum, err, wg, min_lds, st);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_bloom_build(const uint32_t* rkey, const uint64_t* r_start, int bits,
@@ -1264,7 +1274,7 @@ hipError_t launch_bloom_prefilter(const uint32_t* skey, const uint32_t* sval, ui
     return hipGetLastError();
 }
 
-hipError_t launch_filter_l1(const uint32_t* ikey, const uint32_t* ival, const uint64_t* sb_start, int bits,
+hipError_t launch_filter_l1(const uint32_t* tuples, const uint64_t* sb_start, int bits,
                             int bits2, const uint64_t* filter, const BloomGeom& g, uint32_t* okey,
                             uint32_t* oval, uint64_t out_cap, uint32_t* s_fill, uint64_t* count,
                             uint64_t* tile_ctr, uint64_t* err, int num_cu, hipStream_t st)
@@ -1274,7 +1284,7 @@ hipError_t launch_filter_l1(const uint32_t* ikey, const uint32_t* ival, const ui
                        (FL_BLOCK / WAVE + 1) * 4;
     const int W = std::max(1, num_cu / 8) * 2;  // workgroups per XCD
 #define BJ_FILTER(K)                                                                                      \
-    k_filter_l1<FL_BLOCK, FL_ITEMS, K><<<8 * W, FL_BLOCK, lds, st>>>(ikey, ival, sb_start, bits, bits2, filter, g, \
+    k_filter_l1<FL_BLOCK, FL_ITEMS, K><<<8 * W, FL_BLOCK, lds, st>>>({(const Tuple*)tuples}, sb_start, bits, bits2, filter, g, \
                                                                      okey, oval, out_cap, s_fill, count, tile_ctr, err)
     if (g.k == 3) BJ_FILTER(3);
     else if (g.k == 4) BJ_FILTER(4);

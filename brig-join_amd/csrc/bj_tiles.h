@@ -8,6 +8,8 @@
 
 #include "bj_device.h"
 
+#include <type_traits>
+
 namespace bj {
 
 // ---------------------------------------------------------------- histogram
@@ -40,228 +42,270 @@ __device__ __forceinline__ void hist_range(const uint32_t* __restrict__ key, uin
 // within one tile.  Partial chunks occur only where two workgroups' ranges of
 // a bucket meet.  The next tile is loaded into registers while the current one
 // is written out.
+// A tuple as one 8-byte unit: key, then value.
+typedef uint32_t Tuple __attribute__((ext_vector_type(2)));
+
+// Where a scatter reads or writes: keys and values in two arrays (the caller's
+// relations, the final sub-bucket layout) or whole tuples in one (the layout
+// between two passes, and between S's first pass and the filter).
+template <bool PAIR>
+struct TupleIn;
+template <>
+struct TupleIn<false> {
+    const uint32_t* __restrict__ key;
+    const uint32_t* __restrict__ val;
+    __device__ __forceinline__ Tuple load(uint32_t i) const
+    {
+        return Tuple{__builtin_nontemporal_load(&key[i]), __builtin_nontemporal_load(&val[i])};
+    }
+    __device__ __forceinline__ TupleIn from(uint64_t lo) const { return {key + lo, val + lo}; }
+};
+template <>
+struct TupleIn<true> {
+    const Tuple* __restrict__ t;
+    __device__ __forceinline__ Tuple load(uint32_t i) const { return __builtin_nontemporal_load(&t[i]); }
+    __device__ __forceinline__ TupleIn from(uint64_t lo) const { return {t + lo}; }
+};
+template <bool PAIR>
+struct TupleOut;
+template <>
+struct TupleOut<false> {
+    uint32_t* __restrict__ key;
+    uint32_t* __restrict__ val;
+    __device__ __forceinline__ void store(uint64_t i, Tuple x) const
+    {
+        key[i] = x.x;
+        val[i] = x.y;
+    }
+};
+template <>
+struct TupleOut<true> {
+    Tuple* __restrict__ t;
+    __device__ __forceinline__ void store(uint64_t i, Tuple x) const { t[i] = x; }
+};
+
 struct ScatterLds {
     uint64_t* cur;   // [nbk] next global position
-    uint32_t* ck;    // [nbk * cs] carried keys
-    uint32_t* cv;    // [nbk * cs] carried values
-    uint32_t* skey;  // [T]
-    uint32_t* sval;  // [T]
-    uint32_t* cnt0;  // [nbk] tile tuples (even tiles)
-    uint32_t* cnt1;  // [nbk] tile tuples (odd tiles)
-    uint32_t* off;   // [nbk] staging offset
-    uint32_t* ccnt;  // [nbk] carried tuples
-    uint32_t* nw;    // [nbk] tuples written this tile
+    uint64_t* dst;   // [nbk] position of the tile's tuple s: dst + s
+    Tuple* carry;    // [nbk * cs] carried tuples
+    Tuple* stage;    // [T] the tile, bucket by bucket
+    uint32_t* cnt;   // [nbk] tile tuples (even tiles: low half, odd tiles: high half)
+    uint32_t* ol;    // [nbk] staging offset | end of the staged tuples written this tile << 16
+    uint32_t* nc;    // [nbk] tuples written this tile | carried tuples << 16
     uint32_t* wtmp;  // [BLOCK/64 + 1]
 };
+constexpr int SCATTER_BUCKET_BYTES = 28;  // cur, dst, cnt, ol, nc
 
 template <int BLOCK, int ITEMS>
 __device__ __forceinline__ ScatterLds scatter_lds(uint64_t* lds64, int nbk, int cs_log2)
 {
     constexpr int T = BLOCK * ITEMS;
+    static_assert(T <= 16384, "offsets and counts are kept in 16 bits");
     ScatterLds L;
     L.cur = lds64;
-    L.ck = (uint32_t*)(L.cur + nbk);
-    L.cv = L.ck + (nbk << cs_log2);
-    L.skey = L.cv + (nbk << cs_log2);
-    L.sval = L.skey + T;
-    L.cnt0 = L.sval + T;
-    L.cnt1 = L.cnt0 + nbk;
-    L.off = L.cnt1 + nbk;
-    L.ccnt = L.off + nbk;
-    L.nw = L.ccnt + nbk;
-    L.wtmp = L.nw + nbk;
+    L.dst = L.cur + nbk;
+    L.carry = (Tuple*)(L.dst + nbk);
+    L.stage = L.carry + (nbk << cs_log2);
+    L.cnt = (uint32_t*)(L.stage + T);
+    L.ol = L.cnt + nbk;
+    L.nc = L.ol + nbk;
+    L.wtmp = L.nc + nbk;
     return L;
 }
 
-// Bucket b after a tile: the nw[b] tuples written leave the carry / tile, the rest
-// (ccnt + cnt - nw) stay carried.
-__device__ __forceinline__ void scatter_retire(const ScatterLds& L, uint32_t* cprev, int b)
+// Buckets [b0, b0 + PER) of a thread after a tile's ranks: retire the previous
+// tile (its nw tuples leave the carry, the others stay carried), then size this
+// tile's writes from the bucket's count c and its staging offset.  scan turns a
+// thread's sum of counts into its exclusive prefix; on: the thread owns buckets.
+template <int PER, class Scan>
+__device__ __forceinline__ void scatter_offsets(const ScatterLds& L, int b0, bool on, uint32_t par, uint32_t cs,
+                                                Scan&& scan)
 {
-    const uint32_t w = L.nw[b];
-    L.cur[b] += w;
-    L.ccnt[b] = L.ccnt[b] + cprev[b] - w;
-    cprev[b] = 0u;
-}
-
-// Tuples of bucket b written this tile: up to its last whole chunk.
-__device__ __forceinline__ uint32_t scatter_nw(const ScatterLds& L, int b, uint32_t c, uint32_t cs)
-{
-    const uint32_t a0 = (uint32_t)L.cur[b] & (cs - 1u);
-    const uint32_t e = a0 + L.ccnt[b] + c;
-    return e >= cs ? (e & ~(cs - 1u)) - a0 : 0u;
-}
-
-// Scatters kin/vin[0, len) by bucket (radix_hash(key) >> shift) & bmask into
-// okey/oval at the cursors L.cur[] (initialised by the caller; this function
-// begins with a barrier).  Writes are bounds-checked against out_cap; returns
-// true on a violation.
-//
-// Per tile three barriers: ranks (LDS atomics) | offsets (one wave scans the
-// counts, retires the previous tile's buckets and sizes this tile's writes) |
-// staging + carried tuples out + next tile's loads | the tile's tuples out or
-// into the carry (which runs into the next tile's ranks).  Counts alternate
-// between two arrays so the next tile's ranks need no clearing barrier.
-template <int BLOCK, int ITEMS>
-__device__ __forceinline__ bool scatter_range(const ScatterLds& L, const uint32_t* __restrict__ kin,
-                                              const uint32_t* __restrict__ vin, uint32_t len, int nbk,
-                                              int shift, uint32_t bmask, int cs_log2,
-                                              uint32_t* __restrict__ okey, uint32_t* __restrict__ oval,
-                                              uint64_t out_cap)
-{
-    constexpr int T = BLOCK * ITEMS;
-    constexpr int SMALL = 8;  // buckets per lane of the one-wave scan
-    const uint32_t cs = 1u << cs_log2;
-    const bool small = nbk <= SMALL * WAVE;
-    for (int b = threadIdx.x; b < nbk; b += BLOCK) {
-        L.ccnt[b] = 0u;
-        L.cnt0[b] = 0u;
-        L.cnt1[b] = 0u;
-        L.nw[b] = 0u;
-    }
-    // cur/ccnt are read by other threads; an empty range skips the tile loop's barriers
-    __syncthreads();
-
-    uint32_t k[ITEMS], v[ITEMS];
+    uint32_t c[PER], cc[PER];
+    uint64_t cur[PER];
+    uint32_t sum = 0;
 #pragma unroll
-    for (int it = 0; it < ITEMS; it++) {
-        const uint32_t i = (uint32_t)it * BLOCK + threadIdx.x;
-        if (i < len) {
-            k[it] = __builtin_nontemporal_load(&kin[i]);
-            v[it] = __builtin_nontemporal_load(&vin[i]);
+    for (int j = 0; j < PER; j++) {
+        c[j] = cc[j] = 0;
+        cur[j] = 0;
+        if (on) {
+            const uint32_t cn = L.cnt[b0 + j], nc = L.nc[b0 + j], nw = nc & 0xFFFFu;
+            const uint32_t lo = cn & 0xFFFFu, hi = cn >> 16;
+            c[j] = par ? hi : lo;
+            cc[j] = (nc >> 16) + (par ? lo : hi) - nw;
+            cur[j] = L.cur[b0 + j] + nw;
+            L.cnt[b0 + j] = par ? hi << 16 : lo;  // the next tile counts from zero
+            sum += c[j];
         }
     }
+    uint32_t ex = scan(sum);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        if (on) {
+            const uint32_t b = b0 + j;
+            // written: up to the bucket's last whole chunk, then none of the carry
+            // stays (a0 + carried < cs: one more chunk always covers it)
+            const uint32_t a0 = (uint32_t)cur[j] & (cs - 1u);
+            const uint32_t e = a0 + cc[j] + c[j];
+            const uint32_t nw = e >= cs ? (e & ~(cs - 1u)) - a0 : 0u;
+            L.cur[b] = cur[j];
+            L.dst[b] = cur[j] + cc[j] - ex;
+            L.ol[b] = ex | ((nw ? ex + nw - cc[j] : ex) << 16);
+            L.nc[b] = nw | (cc[j] << 16);
+            ex += c[j];
+        }
+    }
+}
+
+// Scatters in[0, len) by bucket (radix_hash(key) >> shift) & bmask into out at the
+// cursors L.cur[] (initialised by the caller; this function begins with a
+// barrier).  Writes are bounds-checked against out_cap; returns true on a
+// violation.
+//
+// Per tile three barriers: ranks (LDS atomics) | offsets (scan of the counts,
+// retiring the previous tile's buckets and sizing this tile's writes) | staging +
+// next tile's loads + carried tuples out | the tile's tuples out or into the carry
+// (which runs into the next tile's ranks).  Counts alternate between the halves of
+// a word so the next tile's ranks need no clearing barrier.
+//
+// A whole tile runs without per-tuple branches, every group of LDS or global
+// accesses issued before the first of them is waited for, and the next tile's
+// loads are unconditional (clamped to the last tuple): with a branch per tuple the
+// compiler waited for each load, and for each LDS read, before it issued the next.
+// HBM bandwidth bounds large passes: 640M tuples by 128 buckets into whole tuples
+// 2.43 -> 2.25 ms (4.5 TB/s; a plain copy reaches 4.96), by 256 buckets 2.88 -> 2.47,
+// a second pass 2.67 -> 2.53; 100M tuples 0.45 -> 0.33 ms.  Whole tuples halve a
+// bucket's carry (16 tuples fill a 128-byte line) and the store instructions.
+template <int BLOCK, int ITEMS, bool IPAIR, bool OPAIR>
+__device__ __forceinline__ bool scatter_range(const ScatterLds& L, const TupleIn<IPAIR>& in, uint32_t len, int nbk,
+                                              int shift, uint32_t bmask, int cs_log2, const TupleOut<OPAIR>& out,
+                                              uint64_t out_cap)
+{
+    constexpr uint32_t T = BLOCK * ITEMS;
+    constexpr int U = 4;  // tuples of a thread handled together on the way out
+    static_assert(ITEMS % U == 0, "groups of U");
+    const uint32_t cs = 1u << cs_log2;
+    const uint32_t ncarry = (uint32_t)nbk << cs_log2;
+    for (int b = threadIdx.x; b < nbk; b += BLOCK) {
+        L.cnt[b] = 0u;
+        L.nc[b] = 0u;
+    }
+    __syncthreads();  // cur is read by other threads
+    if (len == 0) return false;
+
+    Tuple kv[ITEMS];
+    auto load_tile = [&](uint32_t at) {
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) kv[it] = in.load(min(at + (uint32_t)it * BLOCK + threadIdx.x, len - 1u));
+    };
+    load_tile(0);
     bool bad = false;
     uint32_t par = 0;
 
-    for (uint32_t tile = 0; tile < len; tile += T, par ^= 1u) {
-        // cnt1 follows cnt0: select by offset (a select between the two struct
-        // fields would put the struct in scratch memory)
-        uint32_t* cnt = L.cnt0 + (par ? nbk : 0);
-        uint32_t* cprev = L.cnt0 + (par ? 0 : nbk);
-        const int tn = (int)min((uint32_t)T, len - tile);
-        uint32_t bk[ITEMS], rk[ITEMS];
+    auto run_tile = [&](auto whole, uint32_t tile, uint32_t tn) {
+        constexpr bool WHOLE = decltype(whole)::value;
+        uint32_t br[ITEMS];  // bucket | rank << 16
+        const uint32_t one = par ? 1u << 16 : 1u, half = par ? 16u : 0u;
 #pragma unroll
         for (int it = 0; it < ITEMS; it++) {
-            const int s = it * BLOCK + threadIdx.x;
-            if (s < tn) {
-                bk[it] = (radix_hash(k[it]) >> shift) & bmask;
-                rk[it] = atomicAdd(&cnt[bk[it]], 1u);
-            }
+            br[it] = (radix_hash(kv[it].x) >> shift) & bmask;
+            if (WHOLE || (uint32_t)it * BLOCK + threadIdx.x < tn)
+                br[it] |= ((atomicAdd(&L.cnt[br[it]], one) >> half) & 0xFFFFu) << 16;
         }
         __syncthreads();
-        if (nbk > 2 * WAVE && nbk <= BLOCK) {
-            // one bucket per thread, scanned by the whole workgroup: from 3
-            // buckets per lane on, one wave working through them serially keeps
-            // the others waiting longer than the scan's two extra barriers
-            const int b = threadIdx.x;
-            uint32_t c = 0;
-            if (b < nbk) {
-                scatter_retire(L, cprev, b);
-                c = cnt[b];
-            }
-            uint32_t tot;
-            const uint32_t ex = block_exclusive_scan<BLOCK, uint32_t>(c, L.wtmp, &tot);
-            if (b < nbk) {
-                L.off[b] = ex;
-                L.nw[b] = scatter_nw(L, b, c, cs);
-            }
-        } else if (small) {
+        if (nbk <= 2 * WAVE) {
+            // one wave, up to two buckets per lane
             if (threadIdx.x < WAVE) {
-                // lane l owns buckets [l*per, l*per + per)
-                const int per = (nbk + WAVE - 1) / WAVE;
-                const int b0 = min((int)threadIdx.x * per, nbk), b1 = min(b0 + per, nbk);
-                uint32_t sum = 0;
-                for (int b = b0; b < b1; b++) {
-                    scatter_retire(L, cprev, b);
-                    sum += cnt[b];
-                }
-                uint32_t ex = wave_inclusive_scan<uint32_t>(sum) - sum;
-                for (int b = b0; b < b1; b++) {
-                    const uint32_t c = cnt[b];
-                    L.off[b] = ex;
-                    ex += c;
-                    L.nw[b] = scatter_nw(L, b, c, cs);
-                }
+                auto scan = [&](uint32_t x) { return wave_inclusive_scan<uint32_t>(x) - x; };
+                if (nbk <= WAVE) scatter_offsets<1>(L, threadIdx.x, (int)threadIdx.x < nbk, par, cs, scan);
+                else scatter_offsets<2>(L, 2 * threadIdx.x, true, par, cs, scan);
             }
         } else {
-            for (int b = threadIdx.x; b < nbk; b += BLOCK) scatter_retire(L, cprev, b);
-            lds_exclusive_scan<BLOCK>(cnt, L.off, nbk, L.wtmp);
-            for (int b = threadIdx.x; b < nbk; b += BLOCK) L.nw[b] = scatter_nw(L, b, cnt[b], cs);
+            // the whole workgroup: from 3 buckets per lane on, one wave working
+            // through them keeps the others waiting longer than the block scan's
+            // barriers
+            auto scan = [&](uint32_t x) {
+                uint32_t tot;
+                return block_exclusive_scan<BLOCK, uint32_t>(x, L.wtmp, &tot);
+            };
+            if (nbk <= BLOCK) scatter_offsets<1>(L, threadIdx.x, (int)threadIdx.x < nbk, par, cs, scan);
+            else if (nbk == 2 * BLOCK) scatter_offsets<2>(L, 2 * threadIdx.x, true, par, cs, scan);
+            else scatter_offsets<4>(L, 4 * threadIdx.x, 4 * (int)threadIdx.x < nbk, par, cs, scan);
         }
         __syncthreads();
+        uint32_t q[ITEMS];
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) {
-            const int s = it * BLOCK + threadIdx.x;
-            if (s < tn) {
-                const uint32_t p = L.off[bk[it]] + rk[it];
-                L.skey[p] = k[it];
-                L.sval[p] = v[it];
-            }
-        }
-        // prefetch the next tile while this one is written out
-        const uint32_t next = tile + T;
+        for (int it = 0; it < ITEMS; it++) q[it] = (L.ol[br[it] & 0xFFFFu] & 0xFFFFu) + (br[it] >> 16);
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) {
-            const uint32_t i = next + (uint32_t)it * BLOCK + threadIdx.x;
-            if (i < len) {
-                k[it] = __builtin_nontemporal_load(&kin[i]);
-                v[it] = __builtin_nontemporal_load(&vin[i]);
+        for (int it = 0; it < ITEMS; it++)
+            if (WHOLE || (uint32_t)it * BLOCK + threadIdx.x < tn) L.stage[q[it]] = kv[it];
+        // the next tile, in flight while this one is written out
+        if (WHOLE && tile + T < len) load_tile(tile + T);
+        // carried tuples of the buckets that are written go out
+        for (uint32_t i0 = threadIdx.x; i0 < ncarry; i0 += U * BLOCK) {
+            uint32_t nc[U];
+            uint64_t g[U];
+            Tuple x[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t i = min(i0 + (uint32_t)u * BLOCK, ncarry - 1u);
+                nc[u] = L.nc[i >> cs_log2];
+                g[u] = L.cur[i >> cs_log2] + (i & (cs - 1u));
+                x[u] = L.carry[i];
             }
-        }
-        // carried tuples inside the written range go out
-        for (int idx = threadIdx.x; idx < (nbk << cs_log2); idx += BLOCK) {
-            const int b = idx >> cs_log2;
-            const uint32_t i = (uint32_t)idx & (cs - 1u);
-            if (i < L.ccnt[b] && i < L.nw[b]) {
-                const uint64_t g = L.cur[b] + i;
-                if (g < out_cap) {
-                    okey[g] = L.ck[idx];
-                    oval[g] = L.cv[idx];
-                } else {
-                    bad = true;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t i = i0 + (uint32_t)u * BLOCK;
+                if (i < ncarry && (nc[u] & 0xFFFFu) && (i & (cs - 1u)) < nc[u] >> 16) {
+                    if (g[u] < out_cap) out.store(g[u], x[u]);
+                    else bad = true;
                 }
             }
         }
         __syncthreads();
         // the tile's tuples go out, or into the carry
-        for (int s = threadIdx.x; s < tn; s += BLOCK) {
-            const uint32_t kk = L.skey[s];
-            const uint32_t b = (radix_hash(kk) >> shift) & bmask;
-            const uint32_t rel = L.ccnt[b] + (uint32_t)s - L.off[b];
-            const uint32_t w_b = L.nw[b];
-            if (rel < w_b) {
-                const uint64_t g = L.cur[b] + rel;
-                if (g < out_cap) {
-                    okey[g] = kk;
-                    oval[g] = L.sval[s];
+#pragma unroll
+        for (int h = 0; h < ITEMS; h += U) {
+            Tuple x[U];
+            uint32_t b[U], ol[U];
+            uint64_t g[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) x[u] = L.stage[(uint32_t)(h + u) * BLOCK + threadIdx.x];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                b[u] = (radix_hash(x[u].x) >> shift) & bmask;
+                ol[u] = L.ol[b[u]];
+                g[u] = L.dst[b[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t s = (uint32_t)(h + u) * BLOCK + threadIdx.x;
+                if (!WHOLE && s >= tn) continue;
+                if (s < ol[u] >> 16) {
+                    g[u] += s;
+                    if (g[u] < out_cap) out.store(g[u], x[u]);
+                    else bad = true;
                 } else {
-                    bad = true;
+                    // behind the carried tuples, or first where those were written
+                    const uint32_t nc = L.nc[b[u]];
+                    L.carry[(b[u] << cs_log2) + s - (ol[u] >> 16) + ((nc & 0xFFFFu) ? 0u : nc >> 16)] = x[u];
                 }
-            } else {
-                const uint32_t slot = (b << cs_log2) + rel - w_b;
-                L.ck[slot] = kk;
-                L.cv[slot] = L.sval[s];
             }
         }
-    }
+        par ^= 1u;
+    };
+    uint32_t tile = 0;
+    for (; tile + T <= len; tile += T) run_tile(std::true_type{}, tile, T);
+    if (tile < len) run_tile(std::false_type{}, tile, len - tile);
     __syncthreads();
-    // retire the last tile, then the remaining carries (partial chunks at the range ends)
-    {
-        uint32_t* cprev = L.cnt0 + (par ? 0 : nbk);
-        for (int b = threadIdx.x; b < nbk; b += BLOCK) scatter_retire(L, cprev, b);
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < (nbk << cs_log2); idx += BLOCK) {
-        const int b = idx >> cs_log2;
-        const uint32_t i = (uint32_t)idx & (cs - 1u);
-        if (i < L.ccnt[b]) {
-            const uint64_t g = L.cur[b] + i;
-            if (g < out_cap) {
-                okey[g] = L.ck[idx];
-                oval[g] = L.cv[idx];
-            } else {
-                bad = true;
-            }
+    // retire the last tile: the remaining carries (partial chunks at the range ends)
+    for (uint32_t i = threadIdx.x; i < ncarry; i += BLOCK) {
+        const uint32_t b = i >> cs_log2, k = i & (cs - 1u);
+        const uint32_t cn = L.cnt[b], nc = L.nc[b], nw = nc & 0xFFFFu;
+        if (k < (nc >> 16) + (par ? cn & 0xFFFFu : cn >> 16) - nw) {
+            const uint64_t g = L.cur[b] + nw + k;
+            if (g < out_cap) out.store(g, L.carry[i]);
+            else bad = true;
         }
     }
     return bad;
@@ -294,15 +338,14 @@ __device__ __forceinline__ void bloom_build_range(const uint32_t* __restrict__ r
 }
 
 // ---------------------------------------------------------------- Bloom filter S -> S'
-// One tile [tile, tile + BLOCK*ITEMS) of skey/sval (clipped to n): every key
-// tests its 64-bit block; survivors are compacted with a wave ballot + mbcnt
-// per (item, wave) group, an LDS scan over the groups and one global atomic on
-// *count per tile, and written to okey/oval at that position.  Values are read
-// only for survivors.  gcnt holds ITEMS * BLOCK/64 entries, s_base one.
-// Returns true if a write would pass out_cap.
-template <int BLOCK, int ITEMS>
-__device__ __forceinline__ bool prefilter_tile(const uint32_t* __restrict__ skey,
-                                               const uint32_t* __restrict__ sval, uint64_t tile, uint64_t n,
+// One tile [tile, tile + BLOCK*ITEMS) of in (clipped to n): every key tests its
+// 64-bit block; survivors are compacted with a wave ballot + mbcnt per (item,
+// wave) group, an LDS scan over the groups and one global atomic on *count per
+// tile, and written to okey/oval at that position.  From two arrays, values are
+// read only for survivors; whole tuples come with theirs.  gcnt holds ITEMS *
+// BLOCK/64 entries, s_base one.  Returns true if a write would pass out_cap.
+template <int BLOCK, int ITEMS, bool PAIR>
+__device__ __forceinline__ bool prefilter_tile(const TupleIn<PAIR>& in, uint64_t tile, uint64_t n,
                                                const uint64_t* __restrict__ filter, const BloomGeom& g,
                                                uint32_t* __restrict__ okey, uint32_t* __restrict__ oval,
                                                uint64_t out_cap, uint64_t* __restrict__ count, uint32_t* gcnt,
@@ -313,25 +356,27 @@ __device__ __forceinline__ bool prefilter_tile(const uint32_t* __restrict__ skey
     static_assert(NG <= 2 * WAVE, "group scan handles at most 128 groups");
     const int wid = threadIdx.x / WAVE;
     const uint32_t lane = lane_id();
-    uint32_t k[ITEMS];
+    const TupleIn<PAIR> src = in.from(tile);
+    const uint32_t tn = (uint32_t)min((uint64_t)BLOCK * ITEMS, n - tile);
+    Tuple k[ITEMS];
     bool pass[ITEMS];
 #pragma unroll
     for (int it = 0; it < ITEMS; it++) {
-        const uint64_t i = tile + (uint64_t)it * BLOCK + threadIdx.x;
-        k[it] = (i < n) ? __builtin_nontemporal_load(&skey[i]) : 0u;
+        // past n: the tile's last tuple (no branches around the loads)
+        const uint32_t i = min((uint32_t)it * BLOCK + threadIdx.x, tn - 1u);
+        if constexpr (PAIR) k[it] = src.load(i);
+        else k[it].x = __builtin_nontemporal_load(&src.key[i]);
     }
     // every filter word in flight before any is tested; the loads are
-    // unconditional (a lane past n reads the word of key 0): loads under a
-    // branch, with addresses from earlier loads, would each wait for all loads
-    // before them
+    // unconditional: loads under a branch, with addresses from earlier loads, would
+    // each wait for all loads before them
     uint64_t fw[ITEMS];
 #pragma unroll
-    for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it], g)];
+    for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it].x, g)];
 #pragma unroll
     for (int it = 0; it < ITEMS; it++) {
-        const uint64_t i = tile + (uint64_t)it * BLOCK + threadIdx.x;
-        const uint64_t m = bloom_mask(k[it], g.k);
-        pass[it] = i < n && (fw[it] & m) == m;
+        const uint64_t m = bloom_mask(k[it].x, g.k);
+        pass[it] = (uint32_t)it * BLOCK + threadIdx.x < tn && (fw[it] & m) == m;
     }
     uint32_t rank[ITEMS];
 #pragma unroll
@@ -354,10 +399,11 @@ __device__ __forceinline__ bool prefilter_tile(const uint32_t* __restrict__ skey
             *s_base = total ? atomicAdd((unsigned long long*)count, (unsigned long long)total) : 0ull;
     }
     // survivors' values, all in flight before the stores
-    uint32_t vv[ITEMS];
+    if constexpr (!PAIR) {
 #pragma unroll
-    for (int it = 0; it < ITEMS; it++)
-        if (pass[it]) vv[it] = sval[tile + (uint64_t)it * BLOCK + threadIdx.x];
+        for (int it = 0; it < ITEMS; it++)
+            if (pass[it]) k[it].y = src.val[(uint32_t)it * BLOCK + threadIdx.x];
+    }
     __syncthreads();
     bool bad = false;
 #pragma unroll
@@ -365,8 +411,8 @@ __device__ __forceinline__ bool prefilter_tile(const uint32_t* __restrict__ skey
         if (pass[it]) {
             const uint64_t pos = *s_base + gcnt[it * NW + wid] + rank[it];
             if (pos < out_cap) {
-                okey[pos] = k[it];
-                oval[pos] = vv[it];
+                okey[pos] = k[it].x;
+                oval[pos] = k[it].y;
             } else {
                 bad = true;
             }
