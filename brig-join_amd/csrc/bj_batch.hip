@@ -354,7 +354,7 @@ __global__ __launch_bounds__(BLOCK) void kb_bloom_build(BatchDev B, const uint32
 // grouped by the top fb bits), so the keys of a tile probe one or two L2-sized
 // slices of the filter.
 template <int BLOCK, int ITEMS>
-__global__ __launch_bounds__(BLOCK) void kb_prefilter(BatchDev B, uint32_t ntiles,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void kb_prefilter(BatchDev B, uint32_t ntiles,
                                                       const uint64_t* __restrict__ filter,
                                                       const Tuple* __restrict__ tmp,
                                                       uint32_t* __restrict__ sp_key, uint32_t* __restrict__ sp_val,
@@ -362,35 +362,34 @@ __global__ __launch_bounds__(BLOCK) void kb_prefilter(BatchDev B, uint32_t ntile
                                                       uint64_t* __restrict__ err)
 {
     constexpr int T = BLOCK * ITEMS;
-    __shared__ uint32_t gcnt[ITEMS * (BLOCK / WAVE)];
+    __shared__ Tuple stage[2 * T];
+    __shared__ uint32_t gcnt[WAVE], s_next[2];
     __shared__ uint64_t s_base;
-    __shared__ uint32_t s_tile, s_next;
     const uint32_t* px = px_of(B, PX_FTILE);
     const uint32_t xcd = blockIdx.x % NXCD;
     const uint32_t lo = (uint32_t)(((uint64_t)ntiles * xcd) / NXCD);
     const uint32_t cnt = (uint32_t)(((uint64_t)ntiles * (xcd + 1)) / NXCD) - lo;
     unsigned long long* ctr = (unsigned long long*)xctr + xcd;
-    if (threadIdx.x == 0) s_tile = (uint32_t)min(atomicAdd(ctr, 1ull), (unsigned long long)cnt);
-    __syncthreads();
-    uint32_t t = s_tile;
-    bool bad = false;
-    while (t < cnt) {
-        // the next tile's number, read after the tile's first barrier
-        if (threadIdx.x == 0) s_next = (uint32_t)min(atomicAdd(ctr, 1ull), (unsigned long long)cnt);
+    auto next = [&]() { return (uint32_t)min(atomicAdd(ctr, 1ull), (unsigned long long)cnt); };
+    int b = -1;  // join of the last tile: numbers only grow, so the walk goes forward
+    auto desc = [&](uint32_t t) {
         const uint32_t g = lo + t;
-        const int b = find_join(px, B.n, g);
-        const BJoin J = B.J[b];
+        if (b < 0) b = find_join(px, B.n, g);
+        while (g >= px[b + 1]) b++;
+        const BJoin& J = B.J[b];
         const uint64_t tile = (uint64_t)(g - px[b]) * T;
-        auto run = [&](auto in) {
-            bad |= prefilter_tile<BLOCK, ITEMS>(in, tile, J.ns, filter + J.f_base, J.geom, sp_key + J.sp_base,
-                                                sp_val + J.sp_base, J.ns, jc + (size_t)b * JC_N + JC_SPRIME, gcnt,
-                                                &s_base);
-        };
-        if (J.bf2) run(TupleIn<true>{tmp + J.s_base});
-        else run(TupleIn<false>{J.sk, J.sv});
-        t = s_next;
-        __syncthreads();  // s_next is rewritten for the next tile
-    }
+        return FilterTile{J.sk + tile,
+                          J.sv + tile,
+                          J.bf2 ? tmp + J.s_base + tile : nullptr,
+                          (uint32_t)min((uint64_t)T, J.ns - tile),
+                          filter + J.f_base,
+                          J.geom,
+                          sp_key + J.sp_base,
+                          sp_val + J.sp_base,
+                          J.ns,
+                          jc + (size_t)b * JC_N + JC_SPRIME};
+    };
+    const bool bad = filter_run<BLOCK, ITEMS>(cnt, next, desc, stage, gcnt, &s_base, s_next);
     if (bad) atomicOr((unsigned long long*)err, 32ull);
 }
 
@@ -612,8 +611,8 @@ hipError_t launch_batch_prefilter(const BatchDev& B, uint32_t ntiles, const uint
                                   hipStream_t st)
 {
     if (ntiles == 0) return hipSuccess;
-    // four workgroups per CU, a multiple of NXCD
-    const uint32_t grid = (uint32_t)std::max(1, num_cu / NXCD) * 4u * NXCD;
+    // two workgroups per CU (LDS), a multiple of NXCD
+    const uint32_t grid = (uint32_t)std::max(1, num_cu / NXCD) * 2u * NXCD;
     kb_prefilter<PF_BLOCK, PF_ITEMS><<<grid, PF_BLOCK, 0, st>>>(B, ntiles, filter, (const Tuple*)tmp, sp_key, sp_val, jc,
                                                                 xctr, err);
     return hipGetLastError();

@@ -481,22 +481,32 @@ __global__ __launch_bounds__(BLOCK) void k_bloom_build(const uint32_t* __restric
 // ============================================================== Bloom filter S -> S' (before partitioning)
 // The reference's order (queryAndCompactKernelPartitioned): S is filtered
 // before it is partitioned.  Used when the filter fits the MALL, since each key
-// probes a random filter block.  Grid-stride over tiles (prefilter_tile).
+// probes a random filter block.  Grid-stride over tiles (filter_run).
 template <int BLOCK, int ITEMS>
-__global__ __launch_bounds__(BLOCK) void k_bloom_prefilter(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_bloom_prefilter(
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sval, uint64_t n,
     const uint64_t* __restrict__ filter, BloomGeom g, uint32_t* __restrict__ okey,
     uint32_t* __restrict__ oval, uint64_t out_cap, uint64_t* __restrict__ count,
     uint64_t* __restrict__ err)
 {
     constexpr int T = BLOCK * ITEMS;
-    __shared__ uint32_t gcnt[ITEMS * (BLOCK / WAVE)];
+    __shared__ Tuple stage[2 * T];
+    __shared__ uint32_t gcnt[WAVE], s_next[2];
     __shared__ uint64_t s_base;
-    bool bad = false;
-    for (uint64_t tile = (uint64_t)blockIdx.x * T; tile < n; tile += (uint64_t)gridDim.x * T)
-        bad |= prefilter_tile<BLOCK, ITEMS, false>({skey, sval}, tile, n, filter, g, okey, oval, out_cap, count, gcnt,
-                                                   &s_base);
-    if (bad) atomicOr((unsigned long long*)err, 2ull);
+    const uint32_t end = (uint32_t)((n + T - 1) / T);
+    uint32_t at = blockIdx.x;
+    auto next = [&]() {
+        const uint32_t t = at;
+        at += gridDim.x;
+        return t;
+    };
+    auto desc = [&](uint32_t t) {
+        const uint64_t lo = (uint64_t)t * T;
+        return FilterTile{skey + lo, sval + lo, nullptr, (uint32_t)min((uint64_t)T, n - lo), filter, g,
+                          okey, oval, out_cap, count};
+    };
+    if (filter_run<BLOCK, ITEMS>(end, next, desc, stage, gcnt, &s_base, s_next))
+        atomicOr((unsigned long long*)err, 2ull);
 }
 
 // ============================================================== Bloom filter after pass 1
@@ -537,9 +547,19 @@ __device__ __forceinline__ void filter_walk_to(FilterWalk& w, uint64_t t, const 
     }
 }
 
+// A tile's reservations and stores lag one tile behind: tile t's places are
+// requested (one atomic per sub-bucket) while it is staged in one of two LDS
+// buffers, and read, published and used after tile t + 1's test, so neither their
+// latency nor that of the values is on a tile's path.  The next tile's tuples are
+// issued after the test, not behind this tile's filter words (3.66 against 3.39 ms).
+// Bound by the XCD's L2, one request per key: 640M keys in 3 MB slices 3.53 -> 3.39
+// ms, 1.28B keys in 0.75 MB slices 5.87 -> 5.63 ms (227 G keys/s).
+//
 // K: the filter's bits per key when fixed at compile time (3 or 4), 0 = g.k.
-template <int BLOCK, int ITEMS, int K>
-__global__ __launch_bounds__(BLOCK) void k_filter_l1(
+// PER: sub-buckets per thread of the offset scan; 0: at most one per lane of one
+// wave (no block scan).
+template <int BLOCK, int ITEMS, int K, int PER>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_filter_l1(
     TupleIn<true> in, const uint64_t* __restrict__ sb_start, int bits, int bits2, const uint64_t* __restrict__ filter,
     BloomGeom g, uint32_t* __restrict__ okey, uint32_t* __restrict__ oval, uint64_t out_cap,
     uint32_t* __restrict__ s_fill, uint64_t* __restrict__ count, uint64_t* __restrict__ tile_ctr,
@@ -547,18 +567,18 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
 {
     constexpr int T = BLOCK * ITEMS;
     constexpr int NXCD = 8;
+    constexpr int NB = PER ? PER : 1;
     const int P1 = 1 << (bits - bits2), P2 = 1 << bits2;
     const int shift = 32 - bits;
     const uint32_t bmask = (uint32_t)P2 - 1u;
     extern __shared__ uint64_t lds64[];
-    uint64_t* dst0 = lds64;                       // [P2] sub-bucket start + reserved base
-    Tuple* stage = (Tuple*)(dst0 + P2);           // [T]
-    uint32_t* cnt0 = (uint32_t*)(stage + T);      // [2 * P2] survivors per sub-bucket (two tiles)
-    uint32_t* off = cnt0 + 2 * P2;                // [P2]
+    uint64_t* dst = lds64;                        // [P2] position of the last tile's tuple q: dst + q
+    Tuple* stage = (Tuple*)(dst + P2);            // [2 * T] survivors, sub-bucket by sub-bucket (two tiles)
+    uint32_t* cnt0 = (uint32_t*)(stage + 2 * T);  // [2 * P2] survivors per sub-bucket (two tiles)
+    uint32_t* off = cnt0 + 2 * P2;                // [P2] staging offset
     uint32_t* wtmp = off + P2;                    // [BLOCK/64 + 1]
-    __shared__ uint32_t s_total;
-    __shared__ uint64_t s_tile;
-    const bool small = P2 <= 8 * WAVE;
+    __shared__ uint32_t s_total[2];
+    __shared__ uint64_t s_tile, s_tile2;
 
     const int xcd = blockIdx.x % NXCD;
     unsigned long long* xctr = (unsigned long long*)tile_ctr + xcd;
@@ -567,13 +587,14 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
     for (int b = threadIdx.x; b < 2 * P2; b += BLOCK) cnt0[b] = 0u;
     // tile numbers are taken one tile ahead: the current one and the next are
     // known, the one after that is requested while the current tile runs
-    __shared__ uint64_t s_tile2;
     if (threadIdx.x == 0) {
         s_tile = atomicAdd(xctr, 1ull);
         s_tile2 = atomicAdd(xctr, 1ull);
     }
     __syncthreads();
-    uint64_t t_next = s_tile2;
+    // (in scalar registers: so is the walk then)
+    const uint64_t t_first = uniform_u64(s_tile);
+    uint64_t t_next = uniform_u64(s_tile2);
     uint32_t par = 0;
 
     FilterWalk wk;
@@ -584,107 +605,42 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
         wk.lo = sb_start[(uint64_t)wk.p << bits2];
         wk.hi = sb_start[(uint64_t)(wk.p + 1) << bits2];
     }
-    filter_walk_to(wk, s_tile, sb_start, P1, bits2, T);
-    // the current tile [tile, chi) of bucket p; keys are streamed once
-    // (non-temporal, so the filter slice keeps the L2) and the next tile's keys
-    // load while the current tile is written out
+    filter_walk_to(wk, t_first, sb_start, P1, bits2, T);
+    // the current tile [tile, chi) of bucket p; tuples are streamed once
+    // (non-temporal, so the filter slice keeps the L2), a tile ahead
     int p = wk.p;
-    uint64_t tile = wk.lo + (s_tile - wk.tb) * (uint64_t)T;
+    uint64_t tile = wk.lo + (t_first - wk.tb) * (uint64_t)T;
     uint64_t chi = min(tile + (uint64_t)T, wk.hi);
     Tuple nk[ITEMS];
-    if (p < P1) {
-        const TupleIn<true> src = in.from(tile);
+    // clamped to the tile's last tuple rather than skipped past it: no branches
+    auto load_tile = [&](uint64_t at, uint64_t end) {
+        const TupleIn<true> src = in.from(at);
+        const uint32_t last = (uint32_t)(end - 1 - at);
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++)
-            nk[it] = src.load(min((uint32_t)it * BLOCK + threadIdx.x, (uint32_t)(chi - 1 - tile)));
-    }
+        for (int it = 0; it < ITEMS; it++) nk[it] = src.load(min((uint32_t)it * BLOCK + threadIdx.x, last));
+    };
+    if (p < P1) load_tile(tile, chi);
 
-    // Per tile three barriers: test + rank | offsets and reservations (one wave;
-    // it also clears the other tile's counts and publishes the next tile
-    // number) | staging | out (runs into the next tile's test).
-    while (p < P1) {
-        const int tn = (int)(chi - tile);
-        uint32_t* cnt = cnt0 + (par ? P2 : 0);
-        uint32_t* cnext = cnt0 + (par ? 0 : P2);
-        // the tile number after the next one, in flight during this tile
-        unsigned long long t_after = 0ull;
-        if (threadIdx.x == 0) t_after = atomicAdd(xctr, 1ull);
-        uint32_t bk[ITEMS], rk[ITEMS];
-        Tuple k[ITEMS];
-        bool pass[ITEMS];
+    // this thread's sub-buckets [b0, b0 + NB) of the scan, and what it knows of
+    // their last tile's reservations
+    const int b0 = (int)threadIdx.x * NB;
+    const bool own = b0 < P2;
+    uint64_t rstart[NB];
+    uint32_t rbase[NB], roff[NB];
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) k[it] = nk[it];
-        // all filter words of the tile in flight before any is tested.  The
-        // loads are unconditional (a lane past the tile holds its last key):
-        // loads under a branch, with addresses from earlier loads, would each
-        // wait for all loads before them.
-        uint64_t fw[ITEMS];
+    for (int j = 0; j < NB; j++) {
+        rstart[j] = 0;
+        rbase[j] = roff[j] = 0;
+    }
+    auto publish = [&]() {  // the last tile's places
+        if (own)
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it].x, g)];
-#pragma unroll
-        for (int it = 0; it < ITEMS; it++) {
-            const int s = it * BLOCK + threadIdx.x;
-            const uint64_t m = K ? bloom_mask_k<(K ? K : 1)>(k[it].x) : bloom_mask(k[it].x, g.k);
-            const bool ok = s < tn && (fw[it] & m) == m;
-            pass[it] = ok;
-            if (ok) {
-                bk[it] = (radix_hash(k[it].x) >> shift) & bmask;
-                rk[it] = atomicAdd(&cnt[bk[it]], 1u);
-            }
-        }
-        __syncthreads();
-        if (small) {
-            if (threadIdx.x < WAVE) {
-                const int per = (P2 + WAVE - 1) / WAVE;
-                const int b0 = min((int)threadIdx.x * per, P2), b1 = min(b0 + per, P2);
-                uint32_t sum = 0;
-                for (int b = b0; b < b1; b++) sum += cnt[b];
-                const uint32_t inc = wave_inclusive_scan<uint32_t>(sum);
-                uint32_t ex = inc - sum;
-                for (int b = b0; b < b1; b++) {
-                    const uint32_t c = cnt[b];
-                    off[b] = ex;
-                    ex += c;
-                    const uint64_t sb = ((uint64_t)p << bits2) + b;
-                    dst0[b] = sb_start[sb] + (c ? atomicAdd(&s_fill[sb], c) : 0u);
-                    cnext[b] = 0u;
-                }
-                if (threadIdx.x == WAVE - 1) s_total = inc;
-            }
-        } else {
-            const uint32_t tot = lds_exclusive_scan<BLOCK>(cnt, off, P2, wtmp);
-            if (threadIdx.x == 0) s_total = tot;
-            for (int b = threadIdx.x; b < P2; b += BLOCK) {
-                const uint64_t sb = ((uint64_t)p << bits2) + b;
-                const uint32_t c = cnt[b];
-                dst0[b] = sb_start[sb] + (c ? atomicAdd(&s_fill[sb], c) : 0u);
-                cnext[b] = 0u;
-            }
-        }
-        __syncthreads();
-        // the next tile, in flight while this one is written out (clamped rather
-        // than skipped past the end, as above)
-        filter_walk_to(wk, t_next, sb_start, P1, bits2, T);
-        const int p_next = wk.p;
-        const uint64_t tile_next = wk.lo + (t_next - wk.tb) * (uint64_t)T;
-        const uint64_t chi_next = min(tile_next + (uint64_t)T, wk.hi);
-        if (p_next < P1) {
-            const TupleIn<true> src = in.from(tile_next);
-            const uint32_t last = (uint32_t)(chi_next - 1 - tile_next);
-#pragma unroll
-            for (int it = 0; it < ITEMS; it++) nk[it] = src.load(min((uint32_t)it * BLOCK + threadIdx.x, last));
-        }
-#pragma unroll
-        for (int it = 0; it < ITEMS; it++)
-            if (pass[it]) stage[off[bk[it]] + rk[it]] = k[it];
-        // publish the tile number after the next (thread 0 waits for it only here)
-        if (threadIdx.x == 0) s_tile = t_after;
-        __syncthreads();
-        const uint32_t ts = s_total;
+            for (int j = 0; j < NB; j++) dst[b0 + j] = rstart[j] + rbase[j] - roff[j];
+    };
+    auto write_out = [&](uint32_t buf, uint32_t ts) {
         for (uint32_t q = threadIdx.x; q < ts; q += BLOCK) {
-            const Tuple x = stage[q];
-            const uint32_t b = (radix_hash(x.x) >> shift) & bmask;
-            const uint64_t d = dst0[b] + (q - off[b]);
+            const Tuple x = stage[buf * T + q];
+            const uint64_t d = dst[(radix_hash(x.x) >> shift) & bmask] + q;
             if (d < out_cap) {
                 okey[d] = x.x;
                 oval[d] = x.y;
@@ -693,11 +649,98 @@ __global__ __launch_bounds__(BLOCK) void k_filter_l1(
             }
         }
         surv_total += ts;
+    };
+
+    bool have_last = false;  // a tile is staged and not yet written (uniform)
+    // Per tile two barriers (more with a block scan): test + rank | offsets,
+    // reservations, the last tile's places | staging, the last tile out (runs into
+    // the next tile's test).
+    while (p < P1) {
+        const int tn = (int)(chi - tile);
+        uint32_t* cnt = cnt0 + (par ? P2 : 0);
+        uint32_t* cnext = cnt0 + (par ? 0 : P2);
+        // the tile number after the next one, in flight during this tile
+        unsigned long long t_after = 0ull;
+        if (threadIdx.x == 0) t_after = atomicAdd(xctr, 1ull);
+        Tuple k[ITEMS];
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) k[it] = nk[it];
+        // all filter words of the tile in flight before any is tested
+        uint64_t fw[ITEMS];
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it].x, g)];
+        // then the next tile's tuples, so that no wait for a filter word covers them
+        // (on every path: after the last tile, this tile again, unused)
+        filter_walk_to(wk, t_next, sb_start, P1, bits2, T);
+        const int p_next = wk.p;
+        const uint64_t tile_next = wk.lo + (t_next - wk.tb) * (uint64_t)T;
+        const uint64_t chi_next = min(tile_next + (uint64_t)T, wk.hi);
+        uint32_t br[ITEMS];  // sub-bucket | rank << 16
+        uint32_t pass = 0;
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {
+            // used here on every path: the load is not sunk into the branch below
+            // (where it would wait for all loads before it)
+            asm volatile("" : "+v"(fw[it]));
+            const uint64_t m = K ? bloom_mask_k<(K ? K : 1)>(k[it].x) : bloom_mask(k[it].x, g.k);
+            if (it * BLOCK + (int)threadIdx.x < tn && (fw[it] & m) == m) {
+                const uint32_t b = (radix_hash(k[it].x) >> shift) & bmask;
+                br[it] = b | (atomicAdd(&cnt[b], 1u) << 16);
+                pass |= 1u << it;
+            }
+        }
+        __syncthreads();
+        if (PER || threadIdx.x < WAVE) {
+            publish();
+            uint32_t c[NB], sum = 0;
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                c[j] = own ? cnt[b0 + j] : 0u;
+                sum += c[j];
+            }
+            uint32_t ex, tot;
+            if constexpr (PER == 0) {
+                const uint32_t inc = wave_inclusive_scan<uint32_t>(sum);
+                ex = inc - sum;
+                tot = __builtin_amdgcn_readlane(inc, WAVE - 1);
+            } else {
+                ex = block_exclusive_scan<BLOCK, uint32_t>(sum, wtmp, &tot);
+            }
+            if (own) {
+#pragma unroll
+                for (int j = 0; j < NB; j++) {
+                    const uint64_t sb = ((uint64_t)p << bits2) + b0 + j;
+                    off[b0 + j] = ex;
+                    cnext[b0 + j] = 0u;
+                    roff[j] = ex;
+                    rstart[j] = sb_start[sb];
+                    if (c[j]) rbase[j] = atomicAdd(&s_fill[sb], c[j]);
+                    ex += c[j];
+                }
+            }
+            if (threadIdx.x == 0) {
+                s_total[par] = tot;
+                s_tile = t_after;
+            }
+        }
+        __syncthreads();
+        load_tile(p_next < P1 ? tile_next : tile, p_next < P1 ? chi_next : chi);
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++)
+            if ((pass >> it) & 1u) stage[par * T + off[br[it] & 0xFFFFu] + (br[it] >> 16)] = k[it];
+        t_next = uniform_u64(s_tile);
+        if (have_last) write_out(par ^ 1u, s_total[par ^ 1u]);
+        have_last = true;
         p = p_next;
         tile = tile_next;
         chi = chi_next;
-        t_next = s_tile;  // read before thread 0 rewrites it after the next tile's third barrier
         par ^= 1u;
+    }
+    if (have_last) {  // uniform: the last tile
+        __syncthreads();
+        if (PER || threadIdx.x < WAVE) publish();
+        __syncthreads();
+        write_out(par ^ 1u, s_total[par ^ 1u]);
     }
     if (threadIdx.x == 0 && surv_total)
         atomicAdd((unsigned long long*)count, (unsigned long long)surv_total);
@@ -1115,6 +1158,15 @@ static hipError_t set_lds(const void* fn, size_t bytes)
                                (int)(bytes > stat ? bytes - stat : 0));
 }
 
+template <int K>
+static hipError_t set_filter_lds(int bytes)
+{
+    hipError_t e;
+    if ((e = set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, K, 0>, bytes)) != hipSuccess) return e;
+    if ((e = set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, K, 1>, bytes)) != hipSuccess) return e;
+    return set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, K, 4>, bytes);
+}
+
 template <bool IPAIR, bool OPAIR>
 static hipError_t set_scatter_lds(int bytes)
 {
@@ -1133,9 +1185,9 @@ hipError_t kernels_init(int max_lds_bytes)
     if ((e = set_scatter_lds<true, false>(max_lds_bytes)) != hipSuccess) return e;
     g_max_lds = (size_t)max_lds_bytes;
     if ((e = set_lds((const void*)k_bloom_build<1024>, max_lds_bytes)) != hipSuccess) return e;
-    if ((e = set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, 0>, max_lds_bytes)) != hipSuccess) return e;
-    if ((e = set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, 3>, max_lds_bytes)) != hipSuccess) return e;
-    if ((e = set_lds((const void*)k_filter_l1<FL_BLOCK, FL_ITEMS, 4>, max_lds_bytes)) != hipSuccess) return e;
+    if ((e = set_filter_lds<0>(max_lds_bytes)) != hipSuccess) return e;
+    if ((e = set_filter_lds<3>(max_lds_bytes)) != hipSuccess) return e;
+    if ((e = set_filter_lds<4>(max_lds_bytes)) != hipSuccess) return e;
     return hipSuccess;
 }
 
@@ -1269,7 +1321,7 @@ hipError_t launch_bloom_prefilter(const uint32_t* skey, const uint32_t* sval, ui
 {
     if (n == 0) return hipSuccess;
     constexpr int B = 512, I = 8;
-    const int grid = (int)std::min<uint64_t>((uint64_t)num_cu * 8, (n + B * I - 1) / (B * I));
+    const int grid = (int)std::min<uint64_t>((uint64_t)num_cu * 2, (n + B * I - 1) / (B * I));
     k_bloom_prefilter<B, I><<<grid, B, 0, st>>>(skey, sval, n, filter, g, okey, oval, out_cap, count, err);
     return hipGetLastError();
 }
@@ -1280,16 +1332,25 @@ hipError_t launch_filter_l1(const uint32_t* tuples, const uint64_t* sb_start, in
                             uint64_t* tile_ctr, uint64_t* err, int num_cu, hipStream_t st)
 {
     const int P2 = 1 << bits2;
-    const size_t lds = (size_t)P2 * 8 + (size_t)FL_BLOCK * FL_ITEMS * 8 + (size_t)P2 * 12 +
+    const size_t lds = (size_t)P2 * 8 + 2 * (size_t)FL_BLOCK * FL_ITEMS * 8 + (size_t)P2 * 12 +
                        (FL_BLOCK / WAVE + 1) * 4;
     const int W = std::max(1, num_cu / 8) * 2;  // workgroups per XCD
-#define BJ_FILTER(K)                                                                                      \
-    k_filter_l1<FL_BLOCK, FL_ITEMS, K><<<8 * W, FL_BLOCK, lds, st>>>({(const Tuple*)tuples}, sb_start, bits, bits2, filter, g, \
-                                                                     okey, oval, out_cap, s_fill, count, tile_ctr, err)
+    static_assert((1 << 11) <= 4 * FL_BLOCK, "sub-buckets of one first-pass bucket: at most 4 per thread");
+    if (bits2 > 11) return hipErrorInvalidValue;
+#define BJ_FILTER_PER(K, PER)                                                                                \
+    k_filter_l1<FL_BLOCK, FL_ITEMS, K, PER><<<8 * W, FL_BLOCK, lds, st>>>(                                   \
+        {(const Tuple*)tuples}, sb_start, bits, bits2, filter, g, okey, oval, out_cap, s_fill, count, tile_ctr, err)
+#define BJ_FILTER(K)                                    \
+    do {                                                \
+        if (P2 <= WAVE) BJ_FILTER_PER(K, 0);            \
+        else if (P2 <= FL_BLOCK) BJ_FILTER_PER(K, 1);   \
+        else BJ_FILTER_PER(K, 4);                       \
+    } while (0)
     if (g.k == 3) BJ_FILTER(3);
     else if (g.k == 4) BJ_FILTER(4);
     else BJ_FILTER(0);
 #undef BJ_FILTER
+#undef BJ_FILTER_PER
     return hipGetLastError();
 }
 

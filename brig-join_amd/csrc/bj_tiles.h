@@ -12,6 +12,14 @@
 
 namespace bj {
 
+// 64-bit value that is the same in every lane, in scalar registers
+__device__ __forceinline__ uint64_t uniform_u64(uint64_t v)
+{
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // ---------------------------------------------------------------- histogram
 // h[] (LDS, zeroed by the caller) += histogram of the top (32 - sh) bits of the
 // radix hash over key[lo, hi).  8 loads in flight per thread.
@@ -338,87 +346,139 @@ __device__ __forceinline__ void bloom_build_range(const uint32_t* __restrict__ r
 }
 
 // ---------------------------------------------------------------- Bloom filter S -> S'
-// One tile [tile, tile + BLOCK*ITEMS) of in (clipped to n): every key tests its
-// 64-bit block; survivors are compacted with a wave ballot + mbcnt per (item,
-// wave) group, an LDS scan over the groups and one global atomic on *count per
-// tile, and written to okey/oval at that position.  From two arrays, values are
-// read only for survivors; whole tuples come with theirs.  gcnt holds ITEMS *
-// BLOCK/64 entries, s_base one.  Returns true if a write would pass out_cap.
-template <int BLOCK, int ITEMS, bool PAIR>
-__device__ __forceinline__ bool prefilter_tile(const TupleIn<PAIR>& in, uint64_t tile, uint64_t n,
-                                               const uint64_t* __restrict__ filter, const BloomGeom& g,
-                                               uint32_t* __restrict__ okey, uint32_t* __restrict__ oval,
-                                               uint64_t out_cap, uint64_t* __restrict__ count, uint32_t* gcnt,
-                                               uint64_t* s_base)
+// One tile of a filter run: its source (two arrays, or whole tuples at pair), its
+// tuples, the filter, and where its survivors go (reserved on *count).
+struct FilterTile {
+    const uint32_t* key;
+    const uint32_t* val;
+    const Tuple* pair;  // not null: the source
+    uint32_t n;         // 1 .. BLOCK * ITEMS
+    const uint64_t* filter;
+    BloomGeom g;
+    uint32_t* okey;
+    uint32_t* oval;
+    uint64_t out_cap;
+    uint64_t* count;
+};
+
+// Runs tiles through the filter: every key tests its 64-bit block; survivors are
+// ranked by wave ballots per (item, wave) group and a scan of the group counts,
+// staged in LDS and written, compacted, at places reserved with one global atomic
+// per tile.  The reservation and the stores lag one tile behind (two staging
+// buffers) and the next tile's tuples are loaded while this one is staged, so
+// neither latency is on a tile's path.  Values are loaded with the keys: from some
+// 10% survivors on their lines are touched anyway.  Tile numbers run below end:
+// next(t) is the number that follows the one it returned last (thread 0 requests
+// it a tile ahead), desc(t) its tile.  stage: 2 * BLOCK * ITEMS tuples, gcnt: 64
+// counts, s_base / s_next: one word each.  Returns true if a write would pass its
+// tile's out_cap.
+template <int BLOCK, int ITEMS, class Next, class Desc>
+__device__ __forceinline__ bool filter_run(uint32_t end, Next&& next, Desc&& desc, Tuple* stage, uint32_t* gcnt,
+                                           uint64_t* s_base, uint32_t* s_next)
 {
+    constexpr int T = BLOCK * ITEMS;
     constexpr int NW = BLOCK / WAVE;
-    constexpr int NG = ITEMS * NW;  // groups per tile
-    static_assert(NG <= 2 * WAVE, "group scan handles at most 128 groups");
+    static_assert(ITEMS * NW == WAVE, "one group count per lane");
     const int wid = threadIdx.x / WAVE;
     const uint32_t lane = lane_id();
-    const TupleIn<PAIR> src = in.from(tile);
-    const uint32_t tn = (uint32_t)min((uint64_t)BLOCK * ITEMS, n - tile);
-    Tuple k[ITEMS];
-    bool pass[ITEMS];
-#pragma unroll
-    for (int it = 0; it < ITEMS; it++) {
-        // past n: the tile's last tuple (no branches around the loads)
-        const uint32_t i = min((uint32_t)it * BLOCK + threadIdx.x, tn - 1u);
-        if constexpr (PAIR) k[it] = src.load(i);
-        else k[it].x = __builtin_nontemporal_load(&src.key[i]);
-    }
-    // every filter word in flight before any is tested; the loads are
-    // unconditional: loads under a branch, with addresses from earlier loads, would
-    // each wait for all loads before them
-    uint64_t fw[ITEMS];
-#pragma unroll
-    for (int it = 0; it < ITEMS; it++) fw[it] = filter[bloom_block(k[it].x, g)];
-#pragma unroll
-    for (int it = 0; it < ITEMS; it++) {
-        const uint64_t m = bloom_mask(k[it].x, g.k);
-        pass[it] = (uint32_t)it * BLOCK + threadIdx.x < tn && (fw[it] & m) == m;
-    }
-    uint32_t rank[ITEMS];
-#pragma unroll
-    for (int it = 0; it < ITEMS; it++) {
-        const uint64_t m = __ballot(pass[it]);
-        rank[it] = lanes_below(m);
-        if (lane == 0) gcnt[it * NW + wid] = (uint32_t)__popcll(m);
+    if (threadIdx.x == 0) {
+        s_next[0] = next();
+        s_next[1] = next();
     }
     __syncthreads();
-    if (wid == 0) {
-        // exclusive scan of NG (<= 128) group counts: two entries per lane
-        const uint32_t a0 = (2 * lane < (uint32_t)NG) ? gcnt[2 * lane] : 0u;
-        const uint32_t a1 = (2 * lane + 1 < (uint32_t)NG) ? gcnt[2 * lane + 1] : 0u;
-        const uint32_t inc = wave_inclusive_scan<uint32_t>(a0 + a1);
-        const uint32_t ex = inc - a0 - a1;
-        if (2 * lane < (uint32_t)NG) gcnt[2 * lane] = ex;
-        if (2 * lane + 1 < (uint32_t)NG) gcnt[2 * lane + 1] = ex + a0;
-        const uint32_t total = __shfl(inc, WAVE - 1, WAVE);
-        if (lane == 0)
-            *s_base = total ? atomicAdd((unsigned long long*)count, (unsigned long long)total) : 0ull;
-    }
-    // survivors' values, all in flight before the stores
-    if constexpr (!PAIR) {
+    // (in scalar registers: so are the tiles' addresses then)
+    const uint32_t t_first = __builtin_amdgcn_readfirstlane(s_next[0]);
+    uint32_t t_next = __builtin_amdgcn_readfirstlane(s_next[1]);
+    __syncthreads();  // s_next is rewritten
+    if (t_first >= end) return false;
+    FilterTile d = desc(t_first);
+    Tuple nk[ITEMS];
+    // clamped to the tile's last tuple rather than skipped past it: no branch per load
+    auto load_tile = [&](const FilterTile& f) {
+        if (f.pair) {
+            const TupleIn<true> in{f.pair};
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++)
-            if (pass[it]) k[it].y = src.val[(uint32_t)it * BLOCK + threadIdx.x];
-    }
-    __syncthreads();
-    bool bad = false;
+            for (int it = 0; it < ITEMS; it++) nk[it] = in.load(min((uint32_t)it * BLOCK + threadIdx.x, f.n - 1u));
+        } else {
+            const TupleIn<false> in{f.key, f.val};
 #pragma unroll
-    for (int it = 0; it < ITEMS; it++) {
-        if (pass[it]) {
-            const uint64_t pos = *s_base + gcnt[it * NW + wid] + rank[it];
-            if (pos < out_cap) {
-                okey[pos] = k[it].x;
-                oval[pos] = k[it].y;
-            } else {
-                bad = true;
-            }
+            for (int it = 0; it < ITEMS; it++) nk[it] = in.load(min((uint32_t)it * BLOCK + threadIdx.x, f.n - 1u));
         }
+    };
+    load_tile(d);
+    bool bad = false;
+    uint32_t par = 0, last_n = 0;  // survivors of the last tile, staged and not yet written
+    uint32_t *last_key = nullptr, *last_val = nullptr;
+    uint64_t last_cap = 0, base = 0;  // base: thread 0, the last tile's reservation
+    auto write_out = [&]() {
+        const uint64_t b = uniform_u64(*s_base);
+        const uint32_t nw = b >= last_cap ? 0u : (uint32_t)min<uint64_t>(last_n, last_cap - b);
+        bad |= nw < last_n;
+        const Tuple* src = stage + (par ^ 1u) * T;
+        for (uint32_t q = threadIdx.x; q < nw; q += BLOCK) {
+            const Tuple x = src[q];
+            (last_key + b)[q] = x.x;
+            (last_val + b)[q] = x.y;
+        }
+    };
+    for (;;) {
+        uint32_t t_after = end;
+        if (threadIdx.x == 0) t_after = next();
+        Tuple k[ITEMS];
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) k[it] = nk[it];
+        // every filter word in flight before any is tested
+        uint64_t fw[ITEMS];
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) fw[it] = d.filter[bloom_block(k[it].x, d.g)];
+        uint32_t rank[ITEMS], pass = 0;
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {
+            asm volatile("" : "+v"(fw[it]));  // used on every path: not sunk into a branch
+            const uint64_t m = bloom_mask(k[it].x, d.g.k);
+            const bool ok = (uint32_t)it * BLOCK + threadIdx.x < d.n && (fw[it] & m) == m;
+            const uint64_t b = __ballot(ok);
+            rank[it] = lanes_below(b);
+            pass |= (ok ? 1u : 0u) << it;
+            if (lane == 0) gcnt[it * NW + wid] = (uint32_t)__popcll(b);
+        }
+        __syncthreads();
+        const uint32_t c = gcnt[lane];
+        const uint32_t inc = wave_inclusive_scan<uint32_t>(c);
+        const uint32_t total = __builtin_amdgcn_readlane(inc, WAVE - 1);
+        if (threadIdx.x == 0) {
+            *s_base = base;
+            s_next[0] = t_after;
+            base = total ? atomicAdd((unsigned long long*)d.count, (unsigned long long)total) : 0ull;
+        }
+        const bool more = t_next < end;  // uniform
+        FilterTile dn = d;
+        if (more) {
+            dn = desc(t_next);
+            load_tile(dn);
+        }
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {
+            const uint32_t o = __builtin_amdgcn_readlane(inc - c, it * NW + wid);
+            if ((pass >> it) & 1u) stage[par * T + o + rank[it]] = k[it];
+        }
+        __syncthreads();
+        t_next = __builtin_amdgcn_readfirstlane(s_next[0]);
+        if (last_n) write_out();
+        last_n = total;
+        last_key = d.okey;
+        last_val = d.oval;
+        last_cap = d.out_cap;
+        d = dn;
+        par ^= 1u;
+        if (!more) break;
     }
-    __syncthreads();  // gcnt / s_base are rewritten by the next tile
+    if (last_n) {  // uniform: the last tile
+        __syncthreads();  // s_base may still be read for the tile before
+        if (threadIdx.x == 0) *s_base = base;
+        __syncthreads();
+        write_out();
+    }
     return bad;
 }
 
@@ -471,14 +531,6 @@ __device__ __forceinline__ void phase_tick(uint64_t* acc, uint64_t* mark, int ph
         acc[ph] += t - *mark;
         *mark = t;
     }
-}
-
-// 64-bit value that is the same in every lane, in scalar registers
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v)
-{
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return ((uint64_t)hi << 32) | lo;
 }
 
 // COLLECT: thread 0 adds the item's phase times to tacc[PT_CLEAR..PT_WRITE]
