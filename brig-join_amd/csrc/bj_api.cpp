@@ -131,21 +131,29 @@ constexpr uint64_t L2_SLICE_BYTES = 3584ull << 10;
 // while smaller relations need the extra workgroups to hide latency.
 constexpr uint64_t SOLO_TUPLES = 32ull << 20;
 // The direct join's cost against the partitioned join's (choose_direct), in
-// picoseconds on the whole chip.  Measured per (probe tuple, table chunk): 2.4-2.7
-// ps at 10% match (500K x 500K 108 us, 16K x 50M 287 us); with a filter only the
-// survivors are probed, taken as half of S.  The partitioned join takes 130-170 us
-// for its launches alone and 25-40 ps per tuple at these sizes (500K x 500K 166
-// us, 100K x 5M 287 us), 9-11 ps per tuple from some 10M tuples on.  Both sides
-// of the line: 300K x 1M 153 against 178 us, 300K x 3M 402 against 246 us, 800K x
-// 800K 223 against 173 us.
-constexpr double DIRECT_PS_PROBE = 2.7, DIRECT_PS_BF_PROBE = 1.35, DIRECT_PS_SAVED = 100e6;
-constexpr double DIRECT_SMALL_TUPLES = 8e6, DIRECT_PS_SMALL = 20.0, DIRECT_PS_LARGE = 9.0;
+// picoseconds on the whole chip.  Measured at 10% match: the direct join takes some
+// 25 us and 2.4-2.7 ps per (probe tuple, table chunk), the partitioned one some 60
+// us and 9 ps per tuple.  Both sides of the line, direct against partitioned: 100K x
+// 1M 66 / 72 us, 300K x 300K 66 / 65, 500K x 500K 108 / 71, 16K x 50M 291 / 535,
+// 30K x 30M 331 / 337, 60K x 30M 641 / 317.  With a filter only the survivors are
+// probed (at 10% match 0.8-1.4 ps per pair; twice as much allowed for): 500K x 500K
+// 73 / 101 us, 60K x 30M 229 / 423, 1M x 1M 119 / 114.
+constexpr double DIRECT_PS_PROBE = 2.6, DIRECT_PS_SAVED = 35e6, DIRECT_PS_TUPLE = 9.0;
+constexpr double DIRECT_PS_BF_PROBE = 1.0, DIRECT_PS_BF_SAVED = 50e6, DIRECT_PS_BF_TUPLE = 7.0;
+// Probe items below which sub-buckets are sliced finer than 64K probe tuples, and
+// the shortest slice so made (about a quarter of a table's build).
+constexpr uint32_t PROBE_ITEMS_MIN = 512;
+constexpr uint64_t MIN_SLICE = 2048;
 constexpr int PLAN_CUS = 256;  // CUs of an MI355X: only the work split depends on it
 
-int choose_G(uint64_t n)
+// Chunks (histogram and first-pass workgroups) of a relation.  16K tuples, four
+// tiles, per chunk: 3M x 4.5M's first pass 31 -> 29 us, 9M x 24M's 120 -> 106 us
+// against 32K; 8K is no faster.
+constexpr uint64_t CHUNK_TUPLES = 16384;
+int choose_G(uint64_t n, uint64_t per = CHUNK_TUPLES)
 {
     if (n >= SOLO_TUPLES) return PLAN_CUS;
-    uint64_t g = (n + 32767) / 32768;
+    uint64_t g = (n + per - 1) / per;
     return (int)std::max<uint64_t>(1, std::min<uint64_t>(512, g));
 }
 
@@ -172,9 +180,25 @@ bool choose_direct(const bj_params& p, const Plan& pl)
     if (pl.bf && pl.bf_stage != 1) return false;
     const bool build_r = build_from_r(pl.nr, pl.ns, (uint32_t)pl.tile);
     const double nb = (double)(build_r ? pl.nr : pl.ns), np = (double)(build_r ? pl.ns : pl.nr);
-    const double n = (double)(pl.nr + pl.ns), small = std::min(n, DIRECT_SMALL_TUPLES);
-    return std::ceil(nb / pl.tile) * np * (pl.bf ? DIRECT_PS_BF_PROBE : DIRECT_PS_PROBE) <=
-           DIRECT_PS_SAVED + small * DIRECT_PS_SMALL + (n - small) * DIRECT_PS_LARGE;
+    const double n = (double)(pl.nr + pl.ns), probes = std::ceil(nb / pl.tile) * np;
+    return pl.bf ? probes * DIRECT_PS_BF_PROBE <= DIRECT_PS_BF_SAVED + n * DIRECT_PS_BF_TUPLE
+                 : probes * DIRECT_PS_PROBE <= DIRECT_PS_SAVED + n * DIRECT_PS_TUPLE;
+}
+
+void coarse_chunks(Plan& pl)
+{
+    pl.G_r = choose_G(pl.nr, 2 * CHUNK_TUPLES);
+    pl.G_s = choose_G(pl.ns, 2 * CHUNK_TUPLES);
+}
+
+bool choose_merge(const Plan& pl)
+{
+    // the same number of passes on both sides (with a filter, S takes its first
+    // only), both below the one-workgroup-per-CU sizes; a filter before the
+    // partition of S needs R's first
+    return !pl.solo_r && !pl.solo_s && !(pl.bf && pl.bf_stage == 1) &&
+           (pl.bf ? pl.p1 < pl.bits : (pl.p1 < pl.bits) == (pl.p1_s < pl.bits)) &&
+           pl.nr > 0 && pl.ns > 0;
 }
 
 int make_plan(const bj_params& p, Plan& pl)
@@ -321,18 +345,67 @@ int make_plan(const bj_params& p, Plan& pl)
     pl.solo_r = pl.nr >= SOLO_TUPLES;
     pl.solo_s = pl.ns >= SOLO_TUPLES;
     if (const int rc = row_capacity(std::max(pl.nr, pl.ns), p.answer_scale, pl.cap)) return rc;
-    // sum over sub-buckets of ceil(nb / tile) <= (nr + ns) / tile + 2^bits
-    pl.item_cap = (uint64_t)pl.max_slices * ((pl.nr + pl.ns) / pl.tile + (1ull << total)) + 16;
+    // few sub-buckets: their probe sides are cut finer, so that there is an item for
+    // each of the PROBE_ITEMS_MIN workgroups the chip runs at once
+    if ((1u << total) < PROBE_ITEMS_MIN) {
+        const uint32_t per = PROBE_ITEMS_MIN >> total;
+        pl.max_slices = std::max(pl.max_slices, per);
+        const uint64_t np = std::max(pl.nr, pl.ns) >> total;
+        pl.slice = (uint32_t)std::min<uint64_t>(pl.slice, std::max<uint64_t>(MIN_SLICE, (np + per - 1) / per));
+    }
+    // a sub-bucket larger than a tile on its build side builds from its smaller
+    // side: sum of ceil(nb / tile) <= min(nr, ns) / tile + 2^bits
+    pl.item_cap = (uint64_t)pl.max_slices * (std::min(pl.nr, pl.ns) / pl.tile + (1ull << total)) + 16;
     return BJ_OK;
+}
+
+// One side of a partition in the context's buffers (second: the second set, for
+// launches that take R and S together), p1 bits in the first pass, the sub-bucket
+// starts in start[0 .. 2^bits].  l1_only: only the first pass runs.
+static PartSide make_side(bj_ctx* c, const Plan& pl, int p1, const uint32_t* key, const uint32_t* val, uint64_t n,
+                          const uint64_t* n_dev, int G, uint32_t* out_key, uint32_t* out_val, uint64_t out_cap,
+                          uint64_t* start, bool l1_only, bool second)
+{
+    PartSide s{};
+    s.key = key;
+    s.val = val;
+    s.n = n;
+    s.n_dev = n_dev;
+    s.G = G;
+    s.bits = pl.bits;
+    s.p1 = p1;
+    // second-pass workgroups: four tiles each, up to about 1024 in total (3M x
+    // 4.5M's second pass: 58 us with 1024 per side, 33 so, 39 with eight tiles each)
+    s.W2 = std::min(std::max(1, std::min(64, (int)std::min<uint64_t>(1024, (n + CHUNK_TUPLES - 1) / CHUNK_TUPLES) >> p1)), G);
+    // chunk groups of the column sums: the second pass's groups, else up to 8
+    s.W = p1 < pl.bits && !l1_only ? s.W2 : std::min(8, G);
+    s.part = P<uint32_t>(second ? c->part2 : c->part);
+    s.l1h = P<uint32_t>(second ? c->l1h2 : c->l1h);
+    s.l1rel = P<uint32_t>(second ? c->l1off2 : c->l1off);
+    s.l1tot = s.l1rel + ((size_t)G << p1);
+    s.colsum = P<uint32_t>(second ? c->colsum2 : c->colsum);
+    s.totals = P<uint32_t>(second ? c->totals2 : c->totals);
+    s.start = start;
+    DevBuf& tmp = second ? c->tmp2 : c->tmp;
+    s.tmp = P<uint32_t>(tmp);
+    s.tmp_cap = tmp.bytes / 8;
+    s.okey = out_key;
+    s.oval = out_val;
+    s.out_cap = out_cap;
+    return s;
 }
 
 // Radix partition of one relation into out_key/out_val with sub-bucket starts
 // in start[0 .. 2^bits], in one or two physical scatter passes (p1 bits, then
 // the rest).  With l1_only, only the first pass runs and its output (whole tuples
 // grouped by first-pass bucket, in the final positions' ranges) is left in c->tmp.
+// first_of_join: the histogram also clears the join's counters.  plan (nullable):
+// the probe's work items, planned in the second pass; *planned tells whether it ran.
 int run_partition(bj_ctx* c, const Plan& pl, int p1, const uint32_t* key, const uint32_t* val,
                   uint64_t n_host, const uint64_t* n_dev, int G, bool solo, uint32_t* out_key,
-                  uint32_t* out_val, uint64_t out_cap, uint64_t* start, int k_hist, bool l1_only = false)
+                  uint32_t* out_val, uint64_t out_cap, uint64_t* start, int k_hist, bool l1_only = false,
+                  bool first_of_join = false, uint32_t* zero32 = nullptr, const PlanArgs* plan = nullptr,
+                  bool* planned = nullptr)
 {
     // more than half of the CU's LDS: one scatter workgroup per CU
     const size_t min_lds = solo ? (size_t)c->max_lds / 2 + 1024 : 0;
@@ -340,35 +413,27 @@ int run_partition(bj_ctx* c, const Plan& pl, int p1, const uint32_t* key, const 
     auto beg = [&](int slot) { return tl_begin(c, slot); };
     auto end = [&](int slot) { return tl_end(c, slot); };
     hipStream_t st = c->stream;
-    const int b2 = pl.bits - p1;
-    uint64_t* err = P<uint64_t>(c->counters) + CTR_ERR;
-    uint32_t* part = P<uint32_t>(c->part);
+    uint64_t* ctr = P<uint64_t>(c->counters);
+    uint64_t* err = ctr + CTR_ERR;
+    const PartSide s = make_side(c, pl, p1, key, val, n_host, n_dev, G, out_key, out_val, out_cap, start, l1_only,
+                                 false);
+    // a first pass that another kernel reads writes whole tuples into c->tmp
+    const bool two_pass = p1 < pl.bits && !l1_only;
+    const bool first = two_pass || l1_only;
     BJ_HIP(beg(k_hist));
-    BJ_HIP(launch_hist(key, n_host, n_dev, G, pl.bits, part, P<uint32_t>(c->totals), b2, P<uint32_t>(c->l1h), st));
+    BJ_HIP(launch_hist(&s, 1, first_of_join ? ctr : nullptr, CTR_N, zero32, zero32 ? 1 << pl.bits : 0, st));
     BJ_HIP(end(k_hist));
     BJ_HIP(beg(k_hist + 1));
-    const bool two_pass = b2 > 0 && !l1_only;
-    // enough second-pass workgroups to fill the chip: about 1024 in total
-    const int W2 = std::min(std::max(1, std::min(64, 1024 >> p1)), G);
-    // chunk groups of the column sums: the second pass's groups, else up to 8
-    const int W = two_pass ? W2 : std::min(8, G);
-    BJ_HIP(launch_offsets(part, G, pl.bits, b2, W, P<uint32_t>(c->colsum), P<uint32_t>(c->totals),
-                          P<uint32_t>(c->l1h), start,
-                          P<uint64_t>(c->l1off), st));
+    BJ_HIP(launch_cols(&s, 1, st));
     BJ_HIP(end(k_hist + 1));
-    // a first pass that another kernel reads writes whole tuples into c->tmp
-    const bool first = two_pass || l1_only;
-    uint32_t* k1 = first ? P<uint32_t>(c->tmp) : out_key;
-    const uint64_t cap1 = first ? c->tmp.bytes / 8 : out_cap;
     BJ_HIP(beg(k_hist + 2));
-    BJ_HIP(launch_scatter(first ? SCATTER_FIRST : SCATTER_ONLY, key, val, k1, first ? nullptr : out_val, cap1, n_host,
-                          n_dev, G, pl.bits, p1, W2,
-                          P<uint64_t>(c->l1off), start, P<uint32_t>(c->colsum), err, pl.scatter_wg, min_lds, st));
+    BJ_HIP(launch_scatter(first ? SCATTER_FIRST : SCATTER_ONLY, &s, 1, nullptr, err, pl.scatter_wg, min_lds, st));
     BJ_HIP(end(k_hist + 2));
     BJ_HIP(beg(k_hist + 3));
-    if (two_pass)
-        BJ_HIP(launch_scatter(SCATTER_SECOND, k1, nullptr, out_key, out_val, out_cap, n_host, n_dev, G, pl.bits, p1, W2,
-                              P<uint64_t>(c->l1off), start, P<uint32_t>(c->colsum), err, pl.scatter_wg, min_lds, st));
+    if (two_pass) {
+        BJ_HIP(launch_scatter(SCATTER_SECOND, &s, 1, plan, err, pl.scatter_wg, min_lds, st));
+        if (planned) *planned = plan != nullptr;
+    }
     BJ_HIP(end(k_hist + 3));
     return BJ_OK;
 }
@@ -404,8 +469,15 @@ int workspace_items(const Plan& pl, bool with_r, bool with_out,
     if ((rc = need(&bj_ctx::l1off, n_l1 * 8))) return rc;
     if ((rc = need(&bj_ctx::totals, nbins * 4))) return rc;
     if ((rc = need(&bj_ctx::colsum, std::max<uint64_t>(w2max, 8) * nbins * 4))) return rc;
-    if ((rc = need(&bj_ctx::plan_cnt, nbins * 4))) return rc;
-    if ((rc = need(&bj_ctx::item_start, (nbins + 1) * 8))) return rc;
+    if (pl.merge && with_r) {
+        // S's own set beside R's
+        const uint64_t s_l1 = (1ull << pl.p1_s) * (uint64_t)pl.G_s;
+        if ((rc = need(&bj_ctx::part2, (uint64_t)pl.G_s * nbins * 4)) || (rc = need(&bj_ctx::l1h2, s_l1 * 4)) ||
+            (rc = need(&bj_ctx::l1off2, s_l1 * 8)) || (rc = need(&bj_ctx::totals2, nbins * 4)) ||
+            (rc = need(&bj_ctx::colsum2, std::max<uint64_t>(w2max, 8) * nbins * 4)))
+            return rc;
+        if ((pl.p1_s < pl.bits || pl.bf) && (rc = need(&bj_ctx::tmp2, ns * 8))) return rc;
+    }
     if ((rc = need(&bj_ctx::s_start, (nbins + 1) * 8))) return rc;
     if ((rc = need(&bj_ctx::partials, scan_partials_needed(nbins) * 8 + 64))) return rc;
     if ((rc = need(&bj_ctx::items, pl.item_cap * sizeof(HeavyItem)))) return rc;
@@ -502,24 +574,103 @@ float tl_ms(bj_ctx* c, int slot) { return ev_ms(c, c->tl_b[slot], c->tl_e[slot])
 
 float tl_span_ms(bj_ctx* c, int first, int last) { return ev_ms(c, c->tl_b[first], c->tl_e[last]); }
 
-int enqueue_r(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* r_val)
+static int enqueue_bloom_build(bj_ctx* c, const Plan& pl)
 {
-    int rc;
-    if ((rc = run_partition(c, pl, pl.p1, r_key, r_val, pl.nr, nullptr, pl.G_r, pl.solo_r, P<uint32_t>(c->r_key),
-                            P<uint32_t>(c->r_val), c->r_key.bytes / 4, P<uint64_t>(c->r_start), BJ_K_HIST_R)))
-        return rc;
-    if (pl.bf) {
-        BJ_HIP(tl_begin(c, BJ_K_BF_BUILD));
-        BJ_HIP(launch_bloom_build(P<uint32_t>(c->r_key), P<uint64_t>(c->r_start), pl.bits, pl.geom,
-                                  P<uint64_t>(c->filter), c->stream));
-        BJ_HIP(tl_end(c, BJ_K_BF_BUILD));
-    }
+    BJ_HIP(tl_begin(c, BJ_K_BF_BUILD));
+    BJ_HIP(launch_bloom_build(P<uint32_t>(c->r_key), P<uint64_t>(c->r_start), pl.bits, pl.geom,
+                              P<uint64_t>(c->filter), c->stream));
+    BJ_HIP(tl_end(c, BJ_K_BF_BUILD));
     return BJ_OK;
 }
 
-int enqueue_s(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, const uint32_t* s_val,
-              const uint32_t** s_cnt_out, uint32_t* o_key, uint32_t* o_val, uint64_t o_cap)
+int enqueue_r(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* r_val, bool first_of_join)
 {
+    int rc;
+    if ((rc = run_partition(c, pl, pl.p1, r_key, r_val, pl.nr, nullptr, pl.G_r, pl.solo_r, P<uint32_t>(c->r_key),
+                            P<uint32_t>(c->r_val), c->r_key.bytes / 4, P<uint64_t>(c->r_start), BJ_K_HIST_R, false,
+                            first_of_join)))
+        return rc;
+    return pl.bf ? enqueue_bloom_build(c, pl) : BJ_OK;
+}
+
+// The filter after S's first pass (c->tmp or, merged, c->tmp2): its survivors,
+// compacted, in the sub-bucket regions of o_key / o_val; s_fill cleared before.
+static int enqueue_filter_l1(bj_ctx* c, const Plan& pl, const RSide& R, const DevBuf& tmp, uint32_t* o_key,
+                             uint32_t* o_val, uint64_t o_cap)
+{
+    uint64_t* ctr = P<uint64_t>(c->counters);
+    BJ_HIP(tl_begin(c, BJ_K_BF_FILTER));
+    BJ_HIP(launch_filter_l1(P<uint32_t>(tmp), P<uint64_t>(c->s_start), pl.bits, pl.bits - pl.p1_s, R.filter, pl.geom,
+                            o_key, o_val, o_cap, P<uint32_t>(c->s_fill), ctr + CTR_SPRIME, ctr + CTR_XCD,
+                            ctr + CTR_ERR, c->num_cu, c->stream));
+    BJ_HIP(tl_end(c, BJ_K_BF_FILTER));
+    return BJ_OK;
+}
+
+static PlanArgs plan_args(bj_ctx* c, const Plan& pl, const uint64_t* r_start, const uint64_t* s_start,
+                          const uint32_t* s_cnt)
+{
+    uint64_t* ctr = P<uint64_t>(c->counters);
+    PlanArgs a;
+    a.r_start = r_start;
+    a.s_start = s_start;
+    a.s_cnt = s_cnt;
+    a.bits = pl.bits;
+    a.tile = (uint32_t)pl.tile;
+    a.slice = pl.slice;
+    a.max_slices = pl.max_slices;
+    a.n_items = ctr + CTR_ITEMS;
+    a.items = P<HeavyItem>(c->items);
+    a.item_cap = pl.item_cap;
+    a.err = ctr + CTR_ERR;
+    return a;
+}
+
+// Plan::merge: R and S through the partition together, then (with a filter) R's
+// filter and the filter of S.  *s_cnt / *planned as in enqueue_s.
+static int enqueue_rs(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* r_val, const uint32_t* s_key,
+                      const uint32_t* s_val, const uint32_t** s_cnt, bool* planned)
+{
+    hipStream_t st = c->stream;
+    uint64_t* ctr = P<uint64_t>(c->counters);
+    uint64_t* err = ctr + CTR_ERR;
+    uint64_t *r_start = P<uint64_t>(c->r_start), *s_start = P<uint64_t>(c->s_start);
+    uint32_t* s_fill = pl.bf ? P<uint32_t>(c->s_fill) : nullptr;
+    const PartSide sides[2] = {
+        make_side(c, pl, pl.p1, r_key, r_val, pl.nr, nullptr, pl.G_r, P<uint32_t>(c->r_key), P<uint32_t>(c->r_val),
+                  c->r_key.bytes / 4, r_start, false, false),
+        make_side(c, pl, pl.p1_s, s_key, s_val, pl.ns, nullptr, pl.G_s, P<uint32_t>(c->s_key), P<uint32_t>(c->s_val),
+                  c->s_key.bytes / 4, s_start, pl.bf, true)};
+    const bool two = pl.p1 < pl.bits;
+    BJ_HIP(tl_begin(c, BJ_K_HIST_R));
+    BJ_HIP(launch_hist(sides, 2, ctr, CTR_N, s_fill, pl.bf ? 1 << pl.bits : 0, st));
+    BJ_HIP(tl_end(c, BJ_K_HIST_R));
+    BJ_HIP(tl_begin(c, BJ_K_SCAN_R));
+    BJ_HIP(launch_cols(sides, 2, st));
+    BJ_HIP(tl_end(c, BJ_K_SCAN_R));
+    BJ_HIP(tl_begin(c, BJ_K_SCATTER1_R));
+    BJ_HIP(launch_scatter(two ? SCATTER_FIRST : SCATTER_ONLY, sides, 2, nullptr, err, pl.scatter_wg, 0, st));
+    BJ_HIP(tl_end(c, BJ_K_SCATTER1_R));
+    *planned = two && !pl.bf;
+    if (two) {
+        const PlanArgs plan = plan_args(c, pl, r_start, s_start, nullptr);
+        BJ_HIP(tl_begin(c, BJ_K_SCATTER2_R));
+        BJ_HIP(launch_scatter(SCATTER_SECOND, sides, pl.bf ? 1 : 2, *planned ? &plan : nullptr, err, pl.scatter_wg, 0,
+                              st));
+        BJ_HIP(tl_end(c, BJ_K_SCATTER2_R));
+    }
+    *s_cnt = s_fill;
+    if (!pl.bf) return BJ_OK;
+    int rc = enqueue_bloom_build(c, pl);
+    if (rc) return rc;
+    const RSide R{P<uint32_t>(c->r_key), P<uint32_t>(c->r_val), r_start, P<uint64_t>(c->filter)};
+    return enqueue_filter_l1(c, pl, R, c->tmp2, P<uint32_t>(c->s_key), P<uint32_t>(c->s_val), c->s_key.bytes / 4);
+}
+
+int enqueue_s(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, const uint32_t* s_val,
+              const uint32_t** s_cnt_out, uint32_t* o_key, uint32_t* o_val, uint64_t o_cap, bool* planned)
+{
+    if (planned) *planned = false;
     if (!o_key) {
         o_key = P<uint32_t>(c->s_key);
         o_val = P<uint32_t>(c->s_val);
@@ -527,62 +678,51 @@ int enqueue_s(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, 
     }
     hipStream_t st = c->stream;
     uint64_t* ctr = P<uint64_t>(c->counters);
-    auto beg = [&](int slot) { return tl_begin(c, slot); };
-    auto end = [&](int slot) { return tl_end(c, slot); };
+    uint64_t* s_start = P<uint64_t>(c->s_start);
+    const PlanArgs plan = plan_args(c, pl, R.start, s_start, nullptr);
+    const PlanArgs* in_pass = planned ? &plan : nullptr;
+    *s_cnt_out = nullptr;
     int rc;
-    const uint32_t* s_cnt = nullptr;
-    if (pl.bf) {
-        if (pl.bf_stage == 1) {
-            // the reference's order: filter S, then partition the survivors
-            BJ_HIP(beg(BJ_K_BF_FILTER));
-            BJ_HIP(launch_bloom_prefilter(s_key, s_val, pl.ns, R.filter, pl.geom, P<uint32_t>(c->sp_key),
-                                          P<uint32_t>(c->sp_val), c->sp_key.bytes / 4, ctr + CTR_SPRIME,
-                                          ctr + CTR_ERR, c->num_cu, st));
-            BJ_HIP(end(BJ_K_BF_FILTER));
-            if ((rc = run_partition(c, pl, pl.p1_s, P<uint32_t>(c->sp_key), P<uint32_t>(c->sp_val), pl.ns,
-                                    ctr + CTR_SPRIME,
-                                    pl.G_s, pl.solo_s, o_key, o_val, o_cap, P<uint64_t>(c->s_start), BJ_K_HIST_S)))
-                return rc;
-        } else {
-            // first-level pass of S, then filter each bucket against its L2-resident
-            // filter slice while placing the survivors into their sub-buckets
-            if ((rc = run_partition(c, pl, pl.p1_s, s_key, s_val, pl.ns, nullptr, pl.G_s, pl.solo_s, nullptr,
-                                    nullptr, 0, P<uint64_t>(c->s_start), BJ_K_HIST_S, true)))
-                return rc;
-            BJ_HIP(beg(BJ_K_BF_FILTER));
-            BJ_HIP(launch_zero_u32(P<uint32_t>(c->s_fill), 1ull << pl.bits, st));
-            BJ_HIP(launch_filter_l1(P<uint32_t>(c->tmp), P<uint64_t>(c->s_start),
-                                    pl.bits, pl.bits - pl.p1_s, R.filter, pl.geom, o_key, o_val, o_cap,
-                                    P<uint32_t>(c->s_fill),
-                                    ctr + CTR_SPRIME, ctr + CTR_XCD, ctr + CTR_ERR, c->num_cu, st));
-            s_cnt = P<uint32_t>(c->s_fill);
-            BJ_HIP(end(BJ_K_BF_FILTER));
-        }
-    } else {
-        if ((rc = run_partition(c, pl, pl.p1_s, s_key, s_val, pl.ns, nullptr, pl.G_s, pl.solo_s, o_key, o_val, o_cap,
-                                P<uint64_t>(c->s_start), BJ_K_HIST_S)))
+    if (pl.bf && pl.bf_stage == 2) {
+        // first-level pass of S, then filter each bucket against its L2-resident
+        // filter slice while placing the survivors into their sub-buckets
+        uint32_t* s_fill = P<uint32_t>(c->s_fill);
+        if ((rc = run_partition(c, pl, pl.p1_s, s_key, s_val, pl.ns, nullptr, pl.G_s, pl.solo_s, nullptr, nullptr, 0,
+                                s_start, BJ_K_HIST_S, true, false, s_fill)))
             return rc;
+        *s_cnt_out = s_fill;
+        return enqueue_filter_l1(c, pl, R, c->tmp, o_key, o_val, o_cap);
     }
-    *s_cnt_out = s_cnt;
-    return BJ_OK;
+    const uint64_t* n_dev = nullptr;
+    if (pl.bf) {
+        // the reference's order: filter S, then partition the survivors
+        BJ_HIP(tl_begin(c, BJ_K_BF_FILTER));
+        BJ_HIP(launch_bloom_prefilter(s_key, s_val, pl.ns, R.filter, pl.geom, P<uint32_t>(c->sp_key),
+                                      P<uint32_t>(c->sp_val), c->sp_key.bytes / 4, ctr + CTR_SPRIME, ctr + CTR_ERR,
+                                      c->num_cu, st));
+        BJ_HIP(tl_end(c, BJ_K_BF_FILTER));
+        s_key = P<uint32_t>(c->sp_key);
+        s_val = P<uint32_t>(c->sp_val);
+        n_dev = ctr + CTR_SPRIME;
+    }
+    return run_partition(c, pl, pl.p1_s, s_key, s_val, pl.ns, n_dev, pl.G_s, pl.solo_s, o_key, o_val, o_cap, s_start,
+                         BJ_K_HIST_S, false, false, nullptr, in_pass, planned);
 }
 
 int enqueue_plan_probe(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* sk, const uint32_t* sv,
                        const uint64_t* s_start, const uint32_t* s_cnt, uint32_t* o_key, uint32_t* o_rval,
-                       uint32_t* o_sval, uint64_t cap)
+                       uint32_t* o_sval, uint64_t cap, bool planned)
 {
     hipStream_t st = c->stream;
     uint64_t* ctr = P<uint64_t>(c->counters);
-    const int nbins = 1 << pl.bits;
-    uint64_t* item_start = P<uint64_t>(c->item_start);
-    BJ_HIP(tl_begin(c, BJ_K_PLAN));
-    BJ_HIP(launch_plan(R.start, s_start, s_cnt, pl.bits, (uint32_t)pl.tile, pl.slice,
-                       pl.max_slices, P<uint32_t>(c->plan_cnt), item_start, ctr + CTR_ITEMS,
-                       P<HeavyItem>(c->items), pl.item_cap, ctr + CTR_ERR, st));
-    BJ_HIP(tl_end(c, BJ_K_PLAN));
+    if (!planned) {
+        BJ_HIP(tl_begin(c, BJ_K_PLAN));
+        BJ_HIP(launch_plan(plan_args(c, pl, R.start, s_start, s_cnt), st));
+        BJ_HIP(tl_end(c, BJ_K_PLAN));
+    }
     BJ_HIP(tl_begin(c, BJ_K_PROBE));
     BJ_HIP(launch_probe(pl.tile, R.key, R.val, R.start, sk, sv, s_start, s_cnt, pl.bits, pl.slice,
-                        P<HeavyItem>(c->items), item_start + nbins, pl.item_cap, ctr + CTR_WORK, ctr + CTR_OUT,
+                        P<HeavyItem>(c->items), ctr + CTR_ITEMS, pl.item_cap, ctr + CTR_WORK, ctr + CTR_OUT,
                         cap, o_key, o_rval, o_sval, c->num_cu,
                         pl.probe_breakdown ? P<uint64_t>(c->ptimers) : nullptr, st));
     BJ_HIP(tl_end(c, BJ_K_PROBE));
@@ -624,10 +764,11 @@ int enqueue_s_probe(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s
                     uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, uint64_t cap)
 {
     const uint32_t* s_cnt = nullptr;
-    int rc = enqueue_s(c, pl, R, s_key, s_val, &s_cnt);
+    bool planned = false;
+    int rc = enqueue_s(c, pl, R, s_key, s_val, &s_cnt, nullptr, nullptr, 0, &planned);
     if (rc) return rc;
     return enqueue_plan_probe(c, pl, R, P<uint32_t>(c->s_key), P<uint32_t>(c->s_val), P<uint64_t>(c->s_start),
-                              s_cnt, o_key, o_rval, o_sval, cap);
+                              s_cnt, o_key, o_rval, o_sval, cap, planned);
 }
 
 }  // namespace bj
@@ -740,7 +881,8 @@ int bj_destroy(bj_ctx* c)
                       &c->s_key,  &c->s_val,    &c->tmp,  &c->sp_key,  &c->sp_val,
                       &c->filter, &c->part,     &c->totals,  &c->l1h,      &c->l1off,   &c->colsum,  &c->r_start,
                       &c->s_start, &c->s_fill,  &c->partials, &c->items,  &c->counters, &c->out_key,
-                      &c->out_rval, &c->out_sval, &c->dtmp,  &c->plan_cnt, &c->item_start, &c->ptimers,
+                      &c->out_rval, &c->out_sval, &c->dtmp,  &c->ptimers,
+                      &c->part2, &c->totals2, &c->l1h2, &c->l1off2, &c->colsum2, &c->tmp2,
                       &c->pool_key, &c->pool_val, &c->pool_cnt, &c->pool_off, &c->fin_key, &c->fin_val,
                       &c->fin_start};
     for (DevBuf* b : bufs) release(*b);
@@ -774,6 +916,7 @@ int bj_plan(const bj_params* p, bj_plan_info* out)
         int rc = make_plan(*p, pl);
         if (rc) return rc;
         uint64_t ws = 0;
+        pl.merge = choose_merge(pl);
         ensure_workspace(nullptr, pl, &ws);
         if (!p->inputs_on_device) ws += (pl.nr + pl.ns) * 8;
         out->bits1 = pl.bits1;
@@ -881,6 +1024,10 @@ static int chunk_plan(const bj_params& p, const Plan& full, uint64_t chunk, Plan
                      cp.geom.k != full.geom.k || cp.bf_stage != full.bf_stage)))
         return fail(BJ_ERR_INTERNAL, "chunk plan differs from the join's");
     cp.cap = full.cap;
+    // the pooled probe joins all chunks' S' at once: work items as for all of S
+    cp.slice = full.slice;
+    cp.max_slices = full.max_slices;
+    cp.item_cap = full.item_cap;
     return BJ_OK;
 }
 
@@ -892,8 +1039,8 @@ static uint64_t held_bytes(bj_ctx* c)
                             &c->s_key,  &c->s_val,  &c->tmp, &c->sp_key, &c->sp_val,
                             &c->filter, &c->part,   &c->totals,  &c->l1h,     &c->l1off,  &c->colsum,
                             &c->r_start, &c->s_start, &c->s_fill, &c->partials, &c->items, &c->counters,
-                            &c->out_key, &c->out_rval, &c->out_sval, &c->dtmp, &c->plan_cnt, &c->item_start,
-                            &c->ptimers, &c->pool_key, &c->pool_val, &c->pool_cnt, &c->pool_off, &c->fin_key,
+                            &c->out_key, &c->out_rval, &c->out_sval, &c->dtmp, &c->part2, &c->totals2,
+                            &c->l1h2, &c->l1off2, &c->colsum2, &c->tmp2, &c->ptimers, &c->pool_key, &c->pool_val, &c->pool_cnt, &c->pool_off, &c->fin_key,
                             &c->fin_val, &c->fin_start};
     for (const DevBuf* b : bufs) t += b->bytes;
     return t;
@@ -1004,7 +1151,6 @@ static int join_s_chunks(bj_ctx* c, const bj_params* p, const Plan& full, int ch
     if ((rc = probe_timers_begin(c, cp))) return rc;
     if ((rc = enqueue_r(c, cp, r_key, r_val))) return rc;
     const RSide R{P<uint32_t>(c->r_key), P<uint32_t>(c->r_val), P<uint64_t>(c->r_start), P<uint64_t>(c->filter)};
-    uint64_t* item_start = P<uint64_t>(c->item_start);
 
     // buffer b of the two holds chunks b, b + 2, ...; its next copy waits until
     // the join of the chunk before has enqueued everything that reads it
@@ -1071,7 +1217,7 @@ static int join_s_chunks(bj_ctx* c, const bj_params* p, const Plan& full, int ch
             return rc;
         // |S'| and work items of the chunk, summed on the device (a copy to the
         // host here would queue behind the next chunk's copy)
-        BJ_HIP(launch_add2_u64(ctr + CTR_SPRIME, item_start + nbins, ctr + CTR_ACC_SPRIME, st));
+        BJ_HIP(launch_add2_u64(ctr + CTR_SPRIME, ctr + CTR_ITEMS, ctr + CTR_ACC_SPRIME, st));
         if (host) {
             BJ_HIP(hipEventRecord(c->ev_used[b], st));
             if (i + 1 < nch && (rc = copy_chunk(i + 1))) return rc;
@@ -1143,11 +1289,20 @@ int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uin
         first_slot = pl.bf ? BJ_K_BF_BUILD : BJ_K_PROBE;
         if ((rc = enqueue_direct(c, pl, r_key, r_val, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
     } else {
-        BJ_HIP(launch_zero_u64(ctr, CTR_N, st));
+        // the first launch, R's histogram, clears the counters
         if ((rc = probe_timers_begin(c, pl))) return rc;
-        if ((rc = enqueue_r(c, pl, r_key, r_val))) return rc;
         const RSide R{P<uint32_t>(c->r_key), P<uint32_t>(c->r_val), P<uint64_t>(c->r_start), P<uint64_t>(c->filter)};
-        if ((rc = enqueue_s_probe(c, pl, R, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
+        if (pl.merge) {
+            const uint32_t* s_cnt = nullptr;
+            bool planned = false;
+            if ((rc = enqueue_rs(c, pl, r_key, r_val, s_key, s_val, &s_cnt, &planned))) return rc;
+            if ((rc = enqueue_plan_probe(c, pl, R, P<uint32_t>(c->s_key), P<uint32_t>(c->s_val),
+                                         P<uint64_t>(c->s_start), s_cnt, o_key, o_rval, o_sval, pl.cap, planned)))
+                return rc;
+        } else {
+            if ((rc = enqueue_r(c, pl, r_key, r_val, true))) return rc;
+            if ((rc = enqueue_s_probe(c, pl, R, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
+        }
     }
 
     BJ_HIP(hipMemcpyAsync(c->h_counters, ctr, CTR_N * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
@@ -1163,6 +1318,15 @@ int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uin
     if (timing) {
         double* k = out->kernel_ms;
         for (int i = 0; i < BJ_NUM_KERNELS; i++) k[i] = tl_ms(c, i);
+        if (pl.merge) {
+            // launches that took both sides: their time by each side's tuples
+            const double of_s = (double)pl.ns / (double)std::max<uint64_t>(1, pl.nr + pl.ns);
+            const int last = pl.bf ? BJ_K_SCATTER1_R : BJ_K_SCATTER2_R;
+            for (int i = BJ_K_HIST_R; i <= last; i++) {
+                k[i - BJ_K_HIST_R + BJ_K_HIST_S] = k[i] * of_s;
+                k[i] -= k[i] * of_s;
+            }
+        }
         fill_phases(out, h2d_ms < 0 ? ev_ms(c, EV_H2D0, EV_H2D1) : h2d_ms,
                     tl_span_ms(c, first_slot, BJ_K_PROBE));
     }
@@ -1189,7 +1353,15 @@ static int join_once(bj_ctx* c, const bj_params* p, const uint32_t* r_key, const
     if (chunks == 0 && (rc = auto_s_chunks(c, *p, pl, chunks))) return rc;
     if (chunks > 1 && pl.ns > 1) return join_s_chunks(c, p, pl, chunks, r_key, r_val, s_key, s_val, out);
     pl.direct = choose_direct(*p, pl);
-    if ((rc = ensure_workspace(c, pl))) return rc;
+    pl.merge = !pl.direct && choose_merge(pl);
+    rc = ensure_workspace(c, pl);
+    if (rc == BJ_ERR_NOMEM && pl.merge) {
+        // without S's own set of partition buffers
+        for (DevBuf* b : {&c->part2, &c->totals2, &c->l1h2, &c->l1off2, &c->colsum2, &c->tmp2}) release(*b);
+        pl.merge = false;
+        rc = ensure_workspace(c, pl);
+    }
+    if (rc) return rc;
     hipStream_t st = c->stream;
 
     // Kernel-slot events only when the caller collects phase times: each event

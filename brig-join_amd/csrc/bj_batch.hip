@@ -195,12 +195,6 @@ __global__ __launch_bounds__(1024) void kb_binscan(BatchDev B, int side, const u
 // than 2^WIDE_B1 buckets, 1: the others).  ITEMS 4: two workgroups per CU,
 // 4096-tuple tiles; ITEMS 8: one per CU, 8192-tuple tiles and whole-line carries
 // up to 256 buckets (the wide class, and large second passes).
-__device__ __forceinline__ int kb_carry_log2(int nbk, bool big, bool opair)
-{
-    if (big && !opair && nbk <= 256) return 5;
-    return nbk <= 512 ? 4 : (nbk <= 1024 ? 3 : 2);  // scatter_carry
-}
-
 template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 4 ? 8 : 4, 8))) void kb_scatter(BatchDev B, int side, int cls, const uint32_t* __restrict__ sp_key,
                                                     const uint32_t* __restrict__ sp_val,
@@ -220,7 +214,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
     const int bits = side_bits(J, side), b1 = side_b1(J, side);
     const int b2 = bits - b1;
     const int nbk = 1 << b1;
-    const int cs_log2 = kb_carry_log2(nbk, ITEMS == 8, b2 > 0 || side == 2);
+    const int cs_log2 = scatter_carry_log2(nbk, ITEMS == 8, b2 > 0 || side == 2);
     const ScatterLds L = scatter_lds<BLOCK, ITEMS>(lds64, nbk, cs_log2);
     const uint32_t* cr = cur_rel + (side ? J.part_s : J.part_r) + ((size_t)c << bits);
     const uint64_t* st = start + J.sb_base;
@@ -288,7 +282,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 
     const int nbk = 1 << b2;
     const int G = (int)side_chunks(J, side);
     const int g0 = (int)(((int64_t)w * G) / W2), g1 = (int)(((int64_t)(w + 1) * G) / W2);
-    const int cs_log2 = kb_carry_log2(nbk, ITEMS == 8, false);
+    const int cs_log2 = scatter_carry_log2(nbk, ITEMS == 8, false);
     const ScatterLds L = scatter_lds<BLOCK, ITEMS>(lds64, nbk, cs_log2);
     const size_t f0 = (size_t)bb << b2;  // first sub-bucket of the bucket, within the join
     const uint32_t* base = cur_rel + (side ? J.part_s : J.part_r);

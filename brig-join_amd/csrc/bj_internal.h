@@ -103,6 +103,7 @@ struct Plan {
     int G_r = 1, G_s = 1;                // histogram / first-pass scatter workgroups
     bool solo_r = false, solo_s = false; // one scatter workgroup per CU (large relations)
     bool direct = false;                 // joined without a partition (small build side)
+    bool merge = false;                  // R and S partitioned by the same launches
     int tile = 8192;
     uint32_t slice = 65536;
     uint32_t max_slices = 16;
@@ -128,6 +129,11 @@ int make_plan(const bj_params& p, Plan& pl);
 // Whether the one-pass join of this plan runs without a partition (Plan::direct,
 // which make_plan leaves false: only join_device knows the direct join).
 bool choose_direct(const bj_params& p, const Plan& pl);
+// Whether a one-pass join may partition R and S in the same launches (Plan::merge,
+// left false by make_plan; S then needs partition buffers of its own).
+bool choose_merge(const Plan& pl);
+// Chunks twice as long: half the per-chunk histograms, for a tight workspace.
+void coarse_chunks(Plan& pl);
 
 }  // namespace bj
 
@@ -151,7 +157,8 @@ struct bj_ctx {
     bj::DevBuf r_key, r_val, s_key, s_val, sp_key, sp_val;
     bj::DevBuf tmp;  // whole 8-byte tuples between a first pass and the kernel that reads it
     bj::DevBuf filter, part, totals, l1h, l1off, colsum, r_start, s_start, s_fill, partials, items, counters;
-    bj::DevBuf plan_cnt, item_start;
+    // the second set of partition buffers, S's when R and S are partitioned together
+    bj::DevBuf part2, totals2, l1h2, l1off2, colsum2, tmp2;
     bj::DevBuf out_key, out_rval, out_sval, dtmp;
     bj::DevBuf ptimers;  // probe phase timers (probe_breakdown)
     // S in chunks with one probe: every chunk's S' (pool_key / pool_val), the
@@ -178,19 +185,22 @@ int workspace_items(const Plan& pl, bool with_r, bool with_out,
 // Allocates (or, with c == nullptr, only sums) the device workspace of a join.
 int ensure_workspace(bj_ctx* c, const Plan& pl, uint64_t* total_bytes = nullptr);
 // R partition (and the filter built from it) into c's r_key / r_val / r_start / filter.
-int enqueue_r(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* r_val);
+// first_of_join: its first launch also clears the counters.
+int enqueue_r(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* r_val, bool first_of_join = false);
 // S (filtered against R's filter when the plan has one) partitioned with R's
 // radix bits into o_key / o_val (capacity o_cap; null: c's s_key / s_val) at
 // the sub-bucket starts c->s_start; *s_cnt is the survivors per sub-bucket
 // where the regions are not full (filter after the first pass, c->s_fill),
-// else null.
+// else null.  planned (nullable): the probe may be planned in S's second pass;
+// *planned tells whether it was.
 int enqueue_s(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, const uint32_t* s_val,
-              const uint32_t** s_cnt, uint32_t* o_key = nullptr, uint32_t* o_val = nullptr, uint64_t o_cap = 0);
+              const uint32_t** s_cnt, uint32_t* o_key = nullptr, uint32_t* o_val = nullptr, uint64_t o_cap = 0,
+              bool* planned = nullptr);
 // Work items and the build + probe of a partitioned S (sk / sv at s_start, with
 // s_cnt tuples per sub-bucket when not null) against R; rows to o_* (capacity cap).
 int enqueue_plan_probe(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* sk, const uint32_t* sv,
                        const uint64_t* s_start, const uint32_t* s_cnt, uint32_t* o_key, uint32_t* o_rval,
-                       uint32_t* o_sval, uint64_t cap);
+                       uint32_t* o_sval, uint64_t cap, bool planned = false);
 // enqueue_s, then enqueue_plan_probe on its output.
 int enqueue_s_probe(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, const uint32_t* s_val,
                     uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, uint64_t cap);

@@ -34,37 +34,60 @@ hipError_t launch_gen_refdist_r(uint32_t* key, uint64_t n, uint64_t k, const Per
 hipError_t launch_gen_refdist_s(uint32_t* key, uint64_t n, uint64_t m, uint64_t mc0, uint64_t sj0, uint64_t n_r,
                                 const PermKeys& K, hipStream_t st);
 
-// Also zeroes totals (2^bits entries) for launch_offsets when not null, and
-// with bits2 > 0 writes each chunk's first-level counts l1h[g][b1] (the sums
-// over the low bits2 bits).
-hipError_t launch_hist(const uint32_t* key, uint64_t n_host, const uint64_t* n_dev, int G, int bits,
-                       uint32_t* part, uint32_t* totals, int bits2, uint32_t* l1h, hipStream_t st);
+// One side of a partition launch: a relation and where its partition goes.
+struct PartSide {
+    const uint32_t *key, *val;  // source
+    uint64_t n;                 // tuples, or n_dev (not null): on the device
+    const uint64_t* n_dev;
+    int G;                      // chunks (histogram and first-pass workgroups)
+    int bits, p1;               // radix bits, and those of the first pass
+    int W, W2;                  // chunk groups of the column sums, second-pass workgroups per bucket (W = W2)
+    uint32_t* part;             // [G][2^bits] chunk histograms
+    uint32_t* l1h;              // [G][2^p1] first-level counts (p1 < bits)
+    uint32_t* l1rel;            // [G][2^p1] first-level counts of the chunks before
+    uint32_t* l1tot;            // [2^p1] first-level totals
+    uint32_t* colsum;           // [W][2^bits]
+    uint32_t* totals;           // [2^bits]
+    uint64_t* start;            // [2^bits + 1] sub-bucket starts
+    uint32_t* tmp;              // whole tuples between the passes (8-byte aligned)
+    uint64_t tmp_cap;           // in tuples
+    uint32_t *okey, *oval;      // the partitioned relation
+    uint64_t out_cap;
+};
+// The launches of a partition, for one side or for two in one launch (the same
+// radix bits): histograms (which also clear totals, the n_ctr counters at ctr and
+// n_zero32 words at zero32, either may be null), column sums, the scatter passes.
+hipError_t launch_hist(const PartSide* sides, int n, uint64_t* ctr, int n_ctr, uint32_t* zero32, int n_zero32,
+                       hipStream_t st);
+hipError_t launch_cols(const PartSide* sides, int n, hipStream_t st);
+// The vlsplit work items of a probe (bits <= 15): items, and their number at *n_items.
+struct PlanArgs {
+    const uint64_t *r_start = nullptr, *s_start = nullptr;
+    const uint32_t* s_cnt = nullptr;
+    int bits = 0;
+    uint32_t tile = 0, slice = 0, max_slices = 0;
+    uint64_t* n_items = nullptr;
+    HeavyItem* items = nullptr;
+    uint64_t item_cap = 0;
+    uint64_t* err = nullptr;
+};
 hipError_t launch_zero_u32(uint32_t* p, uint64_t n, hipStream_t st);
-// Sub-bucket starts, pass-1 cursors l1off[g][b1] and per-group column sums
-// colsum[w][b] (W groups of chunks) from the per-chunk histograms and, when
-// bits2 > 0, the first-level counts l1h (both from launch_hist; bits <= 15);
-// totals (zeroed by launch_hist) is scratch.
-hipError_t launch_offsets(const uint32_t* part, int G, int bits, int bits2, int W, uint32_t* colsum,
-                          uint32_t* totals, uint32_t* l1h, uint64_t* sb_start, uint64_t* l1off, hipStream_t st);
 size_t scan_partials_needed(uint64_t n);
 hipError_t launch_scan(const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* partial,
                        hipStream_t st);
-int scatter_carry(int nbk);
 size_t scatter_lds_bytes(int nbk);
-// LDS of a 1024-thread, 8192-tuple tile with the carries of scatter_carry_big
+// LDS of a 1024-thread, 8192-tuple tile with whole-line carries
 size_t scatter_lds_bytes_big(int nbk);
 // One pass of a partition.  SCATTER_ONLY: the partition's only pass (p1 = bits),
 // keys and values in two arrays on both sides.  SCATTER_FIRST: by the top p1
-// bits, into whole 8-byte tuples (key, value) at okey (8-byte aligned, oval
-// unused).  SCATTER_SECOND: those tuples (ikey, ival unused) by the remaining
-// bits, W2 workgroups per first-pass bucket, cursors from sb_start and colsum,
-// into two arrays.  out_cap is in tuples.  The launch reserves at least min_lds
-// bytes of LDS per workgroup (a way to cap workgroups per CU).
+// bits, into whole 8-byte tuples (key, value) at tmp.  SCATTER_SECOND: those by the
+// remaining bits, W2 workgroups per first-pass bucket, into two arrays.  The first
+// two also write the sub-bucket starts; SCATTER_SECOND plans the probe when plan
+// is not null (both sides' starts are known then).  The launch reserves at least
+// min_lds bytes of LDS per workgroup (a way to cap workgroups per CU).
 enum { SCATTER_ONLY = 0, SCATTER_FIRST, SCATTER_SECOND };
-hipError_t launch_scatter(int pass, const uint32_t* ikey, const uint32_t* ival, uint32_t* okey, uint32_t* oval,
-                          uint64_t out_cap, uint64_t n_host, const uint64_t* n_dev, int G, int bits, int p1, int W2,
-                          const uint64_t* l1off, const uint64_t* sb_start, const uint32_t* colsum, uint64_t* err,
-                          int wg, size_t min_lds, hipStream_t st);
+hipError_t launch_scatter(int pass, const PartSide* sides, int n, const PlanArgs* plan, uint64_t* err, int wg,
+                          size_t min_lds, hipStream_t st);
 hipError_t launch_bloom_build(const uint32_t* rkey, const uint64_t* r_start, int bits,
                               const BloomGeom& g, uint64_t* filter, hipStream_t st);
 hipError_t launch_bloom_prefilter(const uint32_t* skey, const uint32_t* sval, uint64_t n,
@@ -92,10 +115,7 @@ hipError_t launch_pool_start(const uint32_t* cnt, int nch, int nbins, uint32_t* 
 hipError_t launch_pool_merge(const uint32_t* pk, const uint32_t* pv, const uint32_t* cnt, const uint64_t* off,
                              int nch, int nbins, const uint64_t* start, uint32_t* ok, uint32_t* ov,
                              uint64_t out_cap, uint64_t* err, hipStream_t st);
-hipError_t launch_plan(const uint64_t* r_start, const uint64_t* s_start, const uint32_t* s_cnt, int bits,
-                       uint32_t tile, uint32_t slice, uint32_t max_slices, uint32_t* counts,
-                       uint64_t* item_start, uint64_t* total_out, HeavyItem* items, uint64_t item_cap,
-                       uint64_t* err, hipStream_t st);  // total_out: item count (nullable)
+hipError_t launch_plan(const PlanArgs& plan, hipStream_t st);
 hipError_t launch_probe(int tile, const uint32_t* rk, const uint32_t* rv, const uint64_t* r_start,
                         const uint32_t* sk, const uint32_t* sv, const uint64_t* s_start,
                         const uint32_t* s_cnt, int bits, uint32_t slice, const HeavyItem* items,

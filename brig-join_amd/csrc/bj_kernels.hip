@@ -1,16 +1,17 @@
 // bj_kernels.hip -- gfx950 kernels of the radix hash join, and their launchers.
 //
 // Pipeline (one GPU; all integer, all exact):
-//   R:  k_hist -> k_colsums, k_starts, k_l1_offsets -> k_scatter(pass 1) -> k_scatter(pass 2)
+//   R:  k_hist -> k_cols -> k_scatter(pass 1, sub-bucket starts) -> k_scatter(pass 2)
 //   BF: k_bloom_build (one workgroup per filter segment, built in LDS)
 //   S:  bf_stage 2: k_hist + pass 1 of S, then k_filter_l1 (per first-level
 //       bucket, XCD-aware, filter slice L2-resident) places the survivors;
 //       bf_stage 1: k_bloom_prefilter (S -> S') then the two-level partition
-//   J:  k_plan_count, k_plan_fill (vlsplit work items) -> k_probe (persistent;
-//       LDS chained hash table on the build side, stream the other side)
+//   J:  k_plan (vlsplit work items; in S's second pass where that is last) ->
+//       k_probe (persistent; LDS hash table on the build side, stream the other side)
+//   Below 32M tuples per side one launch takes R and S together (Sides).
 //
 // Reference counterparts (Chanho-LEE-SNU/BRIG-Join):
-//   k_hist / k_colsums / k_starts    gpu_run_hist_for_both, gpu_make_simple_prefix,
+//   k_hist / k_cols                  gpu_run_hist_for_both, gpu_make_simple_prefix,
 //                                    gpu_run_hist_second_pass
 //                                    (src/kernel_functions.cu:22-90, 461-492, 163-207)
 //   k_scatter                        gpu_make_sorted_table_for_both, gpu_build_table_second_pass
@@ -163,167 +164,175 @@ __global__ void k_zipf_Hn(double* out, uint32_t n, double s)
     if (threadIdx.x == 0 && blockIdx.x == 0) out[0] = zipf_H((double)n, s);
 }
 
-// ============================================================== histogram
+// ============================================================== partition
+// The launches of a partition take one side (R or S) or both: workgroups
+// [0, na) belong to side a, the rest to side b.  Joins below some tens of
+// millions of tuples per side spend as long between launches as in them.
+struct Sides {
+    PartSide a, b;
+    int na;  // workgroups of side a
+};
+__device__ __forceinline__ PartSide side_of(const Sides& S, uint32_t& x)
+{
+    if ((int)x < S.na) return S.a;
+    x -= (uint32_t)S.na;
+    return S.b;
+}
+__device__ __forceinline__ uint64_t side_len(const PartSide& s) { return s.n_dev ? *s.n_dev : s.n; }
+
 // Per-workgroup histogram of the full radix (2^bits bins) over a contiguous
 // chunk.  Chunking: chunk = ceil(n / G), workgroup g owns [g*chunk, (g+1)*chunk).
 // k_scatter pass 1 uses exactly the same chunks, so the per-(bucket, group)
 // offsets derived from these histograms place every tuple without atomics.
+// Also clears what the later launches accumulate into: the bin totals, the
+// join's counters (ctr, in the first launch of a join) and zero32.
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_hist(const uint32_t* __restrict__ key, uint64_t n_host,
-                                                const uint64_t* __restrict__ n_dev, int G,
-                                                int bits, uint32_t* __restrict__ part,
-                                                uint32_t* __restrict__ totals, int bits2,
-                                                uint32_t* __restrict__ l1h)
+__global__ __launch_bounds__(BLOCK) void k_hist(Sides S, uint64_t* __restrict__ ctr, int n_ctr,
+                                                uint32_t* __restrict__ zero32, int n_zero32)
 {
     extern __shared__ uint32_t h[];
-    const int nbins = 1 << bits;
+    if (ctr && blockIdx.x == 0 && (int)threadIdx.x < n_ctr) ctr[threadIdx.x] = 0ull;
+    if (zero32)
+        for (int i = blockIdx.x * BLOCK + threadIdx.x; i < n_zero32; i += gridDim.x * BLOCK) zero32[i] = 0u;
+    uint32_t x = blockIdx.x;
+    const PartSide s = side_of(S, x);
+    const int nbins = 1 << s.bits;
     for (int i = threadIdx.x; i < nbins; i += BLOCK) h[i] = 0u;
-    // the bin totals that k_colsums accumulates start at zero
-    if (totals)
-        for (int i = blockIdx.x * BLOCK + threadIdx.x; i < nbins; i += G * BLOCK) totals[i] = 0u;
+    for (int i = x * BLOCK + threadIdx.x; i < nbins; i += s.G * BLOCK) s.totals[i] = 0u;
     __syncthreads();
-    const uint64_t n = n_dev ? *n_dev : n_host;
-    const uint64_t chunk = (n + (uint64_t)G - 1) / (uint64_t)G;
-    const uint64_t lo = min((uint64_t)blockIdx.x * chunk, n);
+    const uint64_t n = side_len(s);
+    const uint64_t chunk = (n + (uint64_t)s.G - 1) / (uint64_t)s.G;
+    const uint64_t lo = min((uint64_t)x * chunk, n);
     const uint64_t hi = min(lo + chunk, n);
-    hist_range<BLOCK>(key, lo, hi, 32 - bits, h);
+    hist_range<BLOCK>(s.key, lo, hi, 32 - s.bits, h);
     __syncthreads();
-    uint32_t* dst = part + (size_t)blockIdx.x * nbins;
+    uint32_t* dst = s.part + (size_t)x * nbins;
     for (int b = threadIdx.x; b < nbins; b += BLOCK) dst[b] = h[b];
-    // this chunk's first-level counts (bits2 > 0): thread b1 sums its 2^bits2
+    // this chunk's first-level counts (two levels): thread b1 sums its 2^b2
     // bins from LDS, starting at a rotated offset so that threads hit different
     // banks at each step
-    if (bits2 > 0) {
-        const int P1 = nbins >> bits2, seg = 1 << bits2;
+    const int b2 = s.bits - s.p1;
+    if (b2 > 0) {
+        const int P1 = 1 << s.p1, seg = 1 << b2;
         for (int b1 = threadIdx.x; b1 < P1; b1 += BLOCK) {
-            const uint32_t* hb = h + ((size_t)b1 << bits2);
+            const uint32_t* hb = h + ((size_t)b1 << b2);
             uint32_t sum = 0;
             for (int j = 0; j < seg; j++) sum += hb[(j + b1) & (seg - 1)];
-            l1h[(size_t)blockIdx.x * P1 + b1] = sum;
+            s.l1h[(size_t)x * P1 + b1] = sum;
         }
     }
 }
 
-// Offsets of a partition, three launches.
-// k_colsums: workgroups [0, ncb * W) sum column block cb (1024 bins) of the
-// per-chunk histograms over chunk group w (chunks [w*G/W, (w+1)*G/W)) into
-// colsum[w][b] and, by atomics, into totals[b] (zeroed by k_hist).  k_hist
-// writes each chunk's first-level counts l1h[g][b1] when the first pass has
-// fewer bits than the partition.
-// Pass 2 derives its cursors from sb_start and colsum itself.
-__global__ __launch_bounds__(1024) void k_colsums(const uint32_t* __restrict__ part, int G, int bits, int W,
-                                                  uint32_t* __restrict__ colsum, uint32_t* __restrict__ totals)
-{
-    constexpr int B = 1024;
-    const int nbins = 1 << bits;
-    const int ncb = (nbins + B - 1) / B;
-    {
-        const int cb = blockIdx.x % ncb, w = blockIdx.x / ncb;
-        const int c = cb * B + threadIdx.x;
-        const int g0 = (int)((int64_t)w * G / W), g1 = (int)((int64_t)(w + 1) * G / W);
-        if (c < nbins) {
-            uint32_t sum = 0;
-#pragma unroll 8
-            for (int g = g0; g < g1; g++) sum += part[(size_t)g * nbins + c];
-            colsum[(size_t)w * nbins + c] = sum;
-            if (sum) atomicAdd(&totals[c], sum);
-        }
-    }
-}
-
-// k_starts: one workgroup scans the bin totals into the sub-bucket starts
-// (sb_start[nbins] = number of tuples).  nbins is a power of two up to 2^15:
-// thread t owns bins [t * per, (t + 1) * per), per = nbins / 1024 (at least 1),
-// read as 16-byte vectors and written as pairs of starts from 4 bins on.
-__global__ __launch_bounds__(1024) void k_starts(const uint32_t* __restrict__ totals, int nbins,
-                                                 uint64_t* __restrict__ sb_start)
-{
-    constexpr int MAXPER = 32;
-    __shared__ uint64_t wtmp[1024 / WAVE + 1];
-    const int per = max(1, nbins >> 10);
-    const int b0 = (int)threadIdx.x * per;
-    uint32_t v[MAXPER];
-    if (per >= 4) {
-        const uint4* t4 = (const uint4*)(totals + b0);
-#pragma unroll
-        for (int j = 0; j < MAXPER / 4; j++) {
-            const uint4 q = (4 * j < per) ? t4[j] : make_uint4(0u, 0u, 0u, 0u);
-            v[4 * j] = q.x;
-            v[4 * j + 1] = q.y;
-            v[4 * j + 2] = q.z;
-            v[4 * j + 3] = q.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = (i < per && b0 + i < nbins) ? totals[b0 + i] : 0u;
-#pragma unroll
-        for (int i = 4; i < MAXPER; i++) v[i] = 0u;
-    }
-    uint64_t sum = 0;
-#pragma unroll
-    for (int i = 0; i < MAXPER; i++) sum += v[i];
-    uint64_t tot;
-    uint64_t ex = block_exclusive_scan<1024, uint64_t>(sum, wtmp, &tot);
-    if (per >= 4) {
-        ulonglong2* o2 = (ulonglong2*)(sb_start + b0);
-#pragma unroll
-        for (int j = 0; j < MAXPER / 2; j++) {
-            const uint64_t e0 = ex, e1 = ex + v[2 * j];
-            ex = e1 + v[2 * j + 1];
-            if (2 * j < per) o2[j] = make_ulonglong2(e0, e1);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            if (i < per && b0 + i < nbins) sb_start[b0 + i] = ex;
-            ex += v[i];
-        }
-    }
-    if (threadIdx.x == 0) sb_start[nbins] = tot;
-}
-
-// First-level cursors of the pass-1 scatter: l1off[g][b1] = start of bucket b1
-// (sb_start[b1 << bits2]) + sum_{g' < g} l1h[g'][b1].  A column scan: each
-// workgroup owns 16 columns; 64 row ranges per column are summed, scanned by
-// one wave per column, then rescanned row by row.  Short row ranges keep the
-// serial chains short when there are few columns (128 first-level buckets give
-// 8 workgroups); loads and stores are coalesced over a row's 16 columns.
+// k_cols, the column sums of a side's histograms, in two kinds of workgroups:
+// - [0, ncb * W): column block cb (1024 bins) of the per-chunk histograms summed
+//   over chunk group w (chunks [w*G/W, (w+1)*G/W)) into colsum[w][b] and, by
+//   atomics, into totals[b] (zeroed by k_hist);
+// - then ceil(2^p1 / L1_COLS): a column scan of the first-level counts,
+//   l1rel[g][b1] = sum_{g' < g} l1h[g'][b1] and the column's total l1tot[b1].  Each
+//   workgroup owns 16 columns; 64 row ranges per column are summed, scanned by
+//   one wave per column, then rescanned row by row (short row ranges keep the
+//   serial chains short when there are few columns).
 constexpr int L1_COLS = 16, L1_ROWS = 1024 / L1_COLS;
 static_assert(L1_ROWS == WAVE && 1024 / WAVE == L1_COLS, "one wave scans one column");
 
-__global__ __launch_bounds__(1024) void k_l1_offsets(const uint32_t* __restrict__ l1h, int G, int P1,
-                                                     int bits2, const uint64_t* __restrict__ sb_start,
-                                                     uint64_t* __restrict__ l1off)
+__host__ __device__ __forceinline__ int cols_sum_wgs(const PartSide& s) { return ((1 << s.bits) + 1023) / 1024 * s.W; }
+__host__ __device__ __forceinline__ int cols_wgs(const PartSide& s)
 {
-    __shared__ uint64_t part_sum[L1_ROWS][L1_COLS + 1];
+    return cols_sum_wgs(s) + ((1 << s.p1) + L1_COLS - 1) / L1_COLS;
+}
+
+__global__ __launch_bounds__(1024) void k_cols(Sides S)
+{
+    __shared__ uint32_t part_sum[L1_ROWS][L1_COLS + 1];
+    uint32_t x = blockIdx.x;
+    const PartSide s = side_of(S, x);
+    const int nbins = 1 << s.bits, nsum = cols_sum_wgs(s);
+    if ((int)x < nsum) {
+        const int ncb = (nbins + 1023) / 1024;
+        const int cb = (int)x % ncb, w = (int)x / ncb;
+        const int c = cb * 1024 + threadIdx.x;
+        const int g0 = (int)((int64_t)w * s.G / s.W), g1 = (int)((int64_t)(w + 1) * s.G / s.W);
+        if (c < nbins) {
+            uint32_t sum = 0;
+#pragma unroll 8
+            for (int g = g0; g < g1; g++) sum += s.part[(size_t)g * nbins + c];
+            s.colsum[(size_t)w * nbins + c] = sum;
+            if (sum) atomicAdd(&s.totals[c], sum);
+        }
+        return;
+    }
+    x -= (uint32_t)nsum;
+    const int P1 = 1 << s.p1;
+    const uint32_t* l1h = s.p1 < s.bits ? s.l1h : s.part;
     const int c = threadIdx.x % L1_COLS, r = threadIdx.x / L1_COLS;
-    const int b1 = blockIdx.x * L1_COLS + c;
-    const int rows = (G + L1_ROWS - 1) / L1_ROWS;
-    const int g0 = min(r * rows, G), g1 = min(g0 + rows, G);
-    uint64_t s = 0;
+    const int b1 = (int)x * L1_COLS + c;
+    const int rows = (s.G + L1_ROWS - 1) / L1_ROWS;
+    const int g0 = min(r * rows, s.G), g1 = min(g0 + rows, s.G);
+    uint32_t sum = 0;
     if (b1 < P1)
-        for (int g = g0; g < g1; g++) s += l1h[(size_t)g * P1 + b1];
-    part_sum[r][c] = s;
+        for (int g = g0; g < g1; g++) sum += l1h[(size_t)g * P1 + b1];
+    part_sum[r][c] = sum;
     __syncthreads();
     {
         // wave w: column w, lane = row range (the branch is uniform per wave)
         const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-        const int col = blockIdx.x * L1_COLS + w;
+        const int col = (int)x * L1_COLS + w;
         if (col < P1) {
-            const uint64_t v = part_sum[lane][w];
-            part_sum[lane][w] = sb_start[(size_t)col << bits2] + wave_inclusive_scan<uint64_t>(v) - v;
+            const uint32_t v = part_sum[lane][w];
+            const uint32_t inc = wave_inclusive_scan<uint32_t>(v);
+            part_sum[lane][w] = inc - v;
+            if (lane == WAVE - 1) s.l1tot[col] = inc;
         }
     }
     __syncthreads();
     if (b1 < P1) {
-        uint64_t acc = part_sum[r][c];
+        uint32_t acc = part_sum[r][c];
         for (int g = g0; g < g1; g++) {
-            l1off[(size_t)g * P1 + b1] = acc;
+            s.l1rel[(size_t)g * P1 + b1] = acc;
             acc += l1h[(size_t)g * P1 + b1];
         }
     }
 }
 
+// One workgroup: exclusive scan of v[0, n) (n a power of two) into out[0, n], as
+// a thread's run of max(1, n / BLOCK) entries, read twice (the second time from
+// the cache), 16 bytes at a time from 4 entries on.  lds: BLOCK/64 + 1 words.
+template <int BLOCK>
+__device__ __forceinline__ void starts_block(const uint32_t* __restrict__ v, int n, uint64_t* __restrict__ out,
+                                             uint64_t* lds)
+{
+    const int per = max(1, n / BLOCK);
+    const int b0 = (int)threadIdx.x * per;
+    uint64_t sum = 0;
+    if (per >= 4) {
+        for (int j = 0; j < per; j += 4) {
+            const uint4 q = *(const uint4*)&v[b0 + j];
+            sum += (uint64_t)q.x + q.y + q.z + q.w;
+        }
+    } else {
+        for (int j = 0; j < per; j++)
+            if (b0 + j < n) sum += v[b0 + j];
+    }
+    uint64_t tot;
+    uint64_t ex = block_exclusive_scan<BLOCK, uint64_t>(sum, lds, &tot);
+    if (per >= 4) {
+        for (int j = 0; j < per; j += 4) {
+            const uint4 q = *(const uint4*)&v[b0 + j];
+            ulonglong2* o = (ulonglong2*)(out + b0 + j);
+            const uint64_t e1 = ex + q.x, e2 = e1 + q.y, e3 = e2 + q.z;
+            o[0] = make_ulonglong2(ex, e1);
+            o[1] = make_ulonglong2(e2, e3);
+            ex = e3 + q.w;
+        }
+    } else {
+        for (int j = 0; j < per; j++)
+            if (b0 + j < n) {
+                out[b0 + j] = ex;
+                ex += v[b0 + j];
+            }
+    }
+    if (threadIdx.x == 0) out[n] = tot;
+}
 
 __global__ void k_zero_u32(uint32_t* __restrict__ p, uint64_t n)
 {
@@ -398,60 +407,181 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(const uint32_t* __rest
     if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = partial[W];
 }
 
+// ============================================================== probe planning
+// A sub-bucket whose build side (build_from_r: R when it fits one LDS tile,
+// else the smaller side) fits one LDS tile and whose probe side fits one slice
+// is "regular": one work item, indexed by the sub-bucket itself.
+// Larger ones are split (vlsplit): the build side into ceil(nb / tile) chunks,
+// the probe side into min(ceil(np / slice), max_slices) slices, one explicit
+// work item per (chunk, slice).  Count, scan, fill: no contention, and the
+// item buffer bound max_slices * (sum ceil(nb / tile)) always holds.
+__device__ __forceinline__ void sb_sizes(const uint64_t* r_start, const uint64_t* s_start,
+                                         const uint32_t* s_cnt, int sb, uint64_t& r0, uint64_t& nr,
+                                         uint64_t& s0, uint64_t& ns)
+{
+    r0 = r_start[sb];
+    nr = r_start[sb + 1] - r0;
+    s0 = s_start[sb];
+    ns = s_cnt ? (uint64_t)s_cnt[sb] : (s_start[sb + 1] - s0);
+}
+
+// One workgroup: every thread takes sub-buckets t, t + BLOCK, ... in groups of
+// PG, counts their items, and a block scan per group places them.  lds: BLOCK/64
+// + 1 words.  In a launch of its own it is latency-bound; where both sides end in
+// a second scatter pass it runs in that launch, whose other workgroups do not
+// need it.
+template <int BLOCK>
+__device__ void plan_block(const PlanArgs& A, uint64_t* lds)
+{
+    constexpr int PG = 8;
+    const int nbins = 1 << A.bits;
+    uint64_t base = 0;
+    bool over = false;
+    for (int sb0 = 0; sb0 < nbins; sb0 += BLOCK * PG) {
+        uint32_t v[PG], sum = 0;
+#pragma unroll
+        for (int j = 0; j < PG; j++) {
+            const int sb = sb0 + j * BLOCK + (int)threadIdx.x;
+            v[j] = 0;
+            if (sb < nbins) {
+                uint64_t r0, nr, s0, ns;
+                sb_sizes(A.r_start, A.s_start, A.s_cnt, sb, r0, nr, s0, ns);
+                uint32_t c, sl;
+                v[j] = plan_items(nr, ns, A.tile, A.slice, A.max_slices, c, sl);
+            }
+            sum += v[j];
+        }
+        uint64_t tot;
+        uint64_t at = base + block_exclusive_scan<BLOCK, uint64_t>((uint64_t)sum, lds, &tot);
+        base += tot;
+        if (tot == 0) continue;  // uniform: no split sub-bucket in the group
+#pragma unroll
+        for (int j = 0; j < PG; j++) {
+            if (v[j] == 0) continue;
+            const int sb = sb0 + j * BLOCK + (int)threadIdx.x;
+            uint64_t r0, nr, s0, ns;
+            sb_sizes(A.r_start, A.s_start, A.s_cnt, sb, r0, nr, s0, ns);
+            uint32_t chunks, slices;
+            plan_items(nr, ns, A.tile, A.slice, A.max_slices, chunks, slices);
+            if (at + v[j] > A.item_cap) {
+                over = true;
+            } else {
+                for (uint32_t c = 0; c < chunks; c++)
+                    for (uint32_t q = 0; q < slices; q++) {
+                        HeavyItem it;
+                        it.sb = (uint32_t)sb;
+                        it.chunk = c;
+                        it.slice = q;
+                        it.nslices = slices;
+                        A.items[at + (uint64_t)c * slices + q] = it;
+                    }
+            }
+            at += v[j];
+        }
+    }
+    if (threadIdx.x == 0) *A.n_items = base;
+    if (over) atomicOr((unsigned long long*)A.err, 4ull);
+}
+
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_plan(PlanArgs A)
+{
+    __shared__ uint64_t lds[BLOCK / WAVE + 1];
+    plan_block<BLOCK>(A, lds);
+}
+
 // ============================================================== scatter
 // Write-combining scatter of one range (scatter_range, bj_tiles.h).  What a
-// workgroup owns:
-//   mode 0 (pass 1, p1 bits): workgroup g owns the same chunk as k_hist's group
-//       g; bucket = h >> (32 - p1); cur[b] = l1off[g * nbk + b].
-//   mode 1 (pass 2, bits - p1 bits): workgroup (b1, w) owns the pass-1 output of
-//       bucket b1 written by pass-1 groups [w*G/W2, (w+1)*G/W2); bucket =
-//       (h >> (32 - bits)) & (2^(bits-p1) - 1); cur[b] = sb_start[sb] +
-//       sum_{v < w} colsum[v][sb] with sb = (b1 << (bits-p1)) + b.
-// Writes are bounds-checked against out_cap and flag err on violation.
+// workgroup of a side owns:
+//   pass 1 (p1 bits): workgroup 1 + g owns the same chunk as k_hist's group g;
+//       bucket = h >> (32 - p1); cur[b] = the bucket's start (a scan of l1tot) +
+//       l1rel[g][b].  Workgroup 0 meanwhile turns the bin totals into the
+//       sub-bucket starts, which only later launches read.
+//   pass 2 (bits - p1 bits): workgroup (b1, w) owns the pass-1 output of bucket
+//       b1 written by pass-1 groups [w*G/W2, (w+1)*G/W2); bucket = (h >> (32 -
+//       bits)) & (2^(bits-p1) - 1); cur[b] = start[sb] + sum_{v < w} colsum[v][sb]
+//       with sb = (b1 << (bits-p1)) + b.
+// IPAIR / OPAIR: whole tuples in one array (TupleIn / TupleOut) on that side:
+// pass 1 writes them unless it is the only pass, pass 2 (IPAIR) reads them.
+// Writes are bounds-checked against the capacity and flag err on violation.
+// plan.items not null: workgroup 0 of the launch plans the probe (plan_block).
 // Occupancy targets: two 1024-thread workgroups per CU for the 4096-tuple tile,
 // one for the 8192-tuple tile (launched one per CU), three 512-thread ones.
 constexpr int sc_min_waves(int block, int items) { return block == 1024 ? (items == 4 ? 8 : 4) : 6; }
 
-// IPAIR / OPAIR: whole tuples in one array (TupleIn / TupleOut) on that side.
 template <int BLOCK, int ITEMS, bool IPAIR, bool OPAIR>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sc_min_waves(BLOCK, ITEMS), 8))) void k_scatter(
-    TupleIn<IPAIR> in, TupleOut<OPAIR> out, uint64_t out_cap,
-    uint64_t n_host, const uint64_t* __restrict__ n_dev, int G, int mode, int bits, int p1, int W2,
-    int cs_log2, const uint64_t* __restrict__ l1off, const uint64_t* __restrict__ sb_start,
-    const uint32_t* __restrict__ colsum, uint64_t* __restrict__ err)
+    Sides S, PlanArgs plan, uint64_t* __restrict__ err)
 {
-    const int b2 = bits - p1;
-    const int nbk = (mode == 0) ? (1 << p1) : (1 << b2);
-    const int shift = (mode == 0) ? (32 - p1) : (32 - bits);
-    const uint32_t bmask = (uint32_t)nbk - 1u;
     extern __shared__ uint64_t lds64[];
+    uint32_t x = blockIdx.x;
+    if (IPAIR && plan.items) {
+        if (x == 0) {
+            plan_block<BLOCK>(plan, lds64);
+            return;
+        }
+        x--;
+    }
+    const PartSide s = side_of(S, x);
+    const int b2 = s.bits - s.p1;
+    const int nbk = IPAIR ? (1 << b2) : (1 << s.p1);
+    const int shift = IPAIR ? (32 - s.bits) : (32 - s.p1);
+    const int cs_log2 = scatter_carry_log2(nbk, ITEMS == 8 && BLOCK == 1024, OPAIR);
     const ScatterLds L = scatter_lds<BLOCK, ITEMS>(lds64, nbk, cs_log2);
-
+    const int P1 = 1 << s.p1;
     uint64_t lo, hi;
-    if (mode == 0) {
-        const uint64_t n = n_dev ? *n_dev : n_host;
-        const uint64_t chunk = (n + (uint64_t)G - 1) / (uint64_t)G;
-        lo = min((uint64_t)blockIdx.x * chunk, n);
+    TupleIn<IPAIR> in;
+    TupleOut<OPAIR> out;
+    uint64_t cap;
+    if constexpr (!IPAIR) {
+        if (x == 0) {
+            starts_block<BLOCK>(s.totals, 1 << s.bits, s.start, lds64);
+            return;
+        }
+        const uint32_t g = x - 1u;
+        const uint64_t n = side_len(s);
+        const uint64_t chunk = (n + (uint64_t)s.G - 1) / (uint64_t)s.G;
+        lo = min((uint64_t)g * chunk, n);
         hi = min(lo + chunk, n);
-        for (int b = threadIdx.x; b < nbk; b += BLOCK) L.cur[b] = l1off[(size_t)blockIdx.x * nbk + b];
+        // the buckets' starts: thread t scans buckets [t * per, (t + 1) * per)
+        const int per = max(1, nbk / BLOCK), q0 = (int)threadIdx.x * per;
+        uint32_t sum = 0, tot;
+        for (int j = 0; j < per; j++)
+            if (q0 + j < nbk) sum += s.l1tot[q0 + j];
+        uint32_t ex = block_exclusive_scan<BLOCK, uint32_t>(sum, L.wtmp, &tot);
+        for (int j = 0; j < per; j++)
+            if (q0 + j < nbk) {
+                L.cur[q0 + j] = (uint64_t)ex + s.l1rel[(size_t)g * P1 + q0 + j];
+                ex += s.l1tot[q0 + j];
+            }
+        in = {s.key, s.val};
     } else {
-        const int P1 = 1 << p1;
-        const int b1 = blockIdx.x / W2, w = blockIdx.x % W2;
-        const int g0 = (int)(((int64_t)w * G) / W2), g1 = (int)(((int64_t)(w + 1) * G) / W2);
-        lo = (g0 < G) ? l1off[(size_t)g0 * P1 + b1] : sb_start[(uint64_t)(b1 + 1) << b2];
-        hi = (g1 < G) ? l1off[(size_t)g1 * P1 + b1] : sb_start[(uint64_t)(b1 + 1) << b2];
+        const int b1 = (int)x / s.W2, w = (int)x % s.W2;
+        const int g0 = (int)(((int64_t)w * s.G) / s.W2), g1 = (int)(((int64_t)(w + 1) * s.G) / s.W2);
+        const uint64_t b_lo = s.start[(uint64_t)b1 << b2], b_hi = s.start[(uint64_t)(b1 + 1) << b2];
+        lo = (g0 < s.G) ? b_lo + s.l1rel[(size_t)g0 * P1 + b1] : b_hi;
+        hi = (g1 < s.G) ? b_lo + s.l1rel[(size_t)g1 * P1 + b1] : b_hi;
         // cursor of sub-bucket sb: its start plus what the earlier groups hold of it
-        const uint64_t nbins = 1ull << bits;
+        const uint64_t nbins = 1ull << s.bits;
         for (int b = threadIdx.x; b < nbk; b += BLOCK) {
             const uint64_t sb = ((uint64_t)b1 << b2) + b;
-            uint64_t cur = sb_start[sb];
-            for (int v = 0; v < w; v++) cur += colsum[(size_t)v * nbins + sb];
+            uint64_t cur = s.start[sb];
+#pragma unroll 8
+            for (int v = 0; v < w; v++) cur += s.colsum[(size_t)v * nbins + sb];
             L.cur[b] = cur;
         }
+        in = {(const Tuple*)s.tmp};
+    }
+    if constexpr (OPAIR) {
+        out = {(Tuple*)s.tmp};
+        cap = s.tmp_cap;
+    } else {
+        out = {s.okey, s.oval};
+        cap = s.out_cap;
     }
     // ranges are below 2^31 tuples
-    const bool bad = scatter_range<BLOCK, ITEMS, IPAIR, OPAIR>(L, in.from(lo), (uint32_t)(hi - lo), nbk, shift, bmask,
-                                                               cs_log2, out, out_cap);
+    const bool bad = scatter_range<BLOCK, ITEMS, IPAIR, OPAIR>(L, in.from(lo), (uint32_t)(hi - lo), nbk, shift,
+                                                               (uint32_t)nbk - 1u, cs_log2, out, cap);
     if (bad) atomicOr((unsigned long long*)err, 1ull);
 }
 
@@ -807,122 +937,6 @@ __global__ __launch_bounds__(POOL_BLOCK) void k_pool_merge(
     }
 }
 
-// ============================================================== probe planning
-// A sub-bucket whose build side (build_from_r: R when it fits one LDS tile,
-// else the smaller side) fits one LDS tile and whose probe side fits one slice
-// is "regular": one work item, indexed by the sub-bucket itself.
-// Larger ones are split (vlsplit): the build side into ceil(nb / tile) chunks,
-// the probe side into min(ceil(np / slice), max_slices) slices, one explicit
-// work item per (chunk, slice).  Count, scan, fill: no contention, and the
-// item buffer bound max_slices * (sum ceil(nb / tile)) always holds.
-__device__ __forceinline__ void sb_sizes(const uint64_t* r_start, const uint64_t* s_start,
-                                         const uint32_t* s_cnt, int sb, uint64_t& r0, uint64_t& nr,
-                                         uint64_t& s0, uint64_t& ns)
-{
-    r0 = r_start[sb];
-    nr = r_start[sb + 1] - r0;
-    s0 = s_start[sb];
-    ns = s_cnt ? (uint64_t)s_cnt[sb] : (s_start[sb + 1] - s0);
-}
-
-__global__ void k_plan_count(const uint64_t* __restrict__ r_start, const uint64_t* __restrict__ s_start,
-                             const uint32_t* __restrict__ s_cnt, int nbins, uint32_t tile,
-                             uint32_t slice, uint32_t max_slices, uint32_t* __restrict__ n_items)
-{
-    const int sb = blockIdx.x * blockDim.x + threadIdx.x;
-    if (sb >= nbins) return;
-    uint64_t r0, nr, s0, ns;
-    sb_sizes(r_start, s_start, s_cnt, sb, r0, nr, s0, ns);
-    uint32_t c, sl;
-    n_items[sb] = plan_items(nr, ns, tile, slice, max_slices, c, sl);
-}
-
-// One workgroup: thread t owns a run of at most 32 sub-buckets; one block scan
-// of the counts into item_start (item_start[nbins] = total, also stored at
-// *total_out when given), then the items of the (few) split sub-buckets.
-__global__ __launch_bounds__(1024) void k_plan_fill(const uint64_t* __restrict__ r_start,
-                                                    const uint64_t* __restrict__ s_start,
-                                                    const uint32_t* __restrict__ s_cnt, int nbins, uint32_t tile,
-                                                    uint32_t slice, uint32_t max_slices,
-                                                    const uint32_t* __restrict__ n_items,
-                                                    uint64_t* __restrict__ item_start, uint64_t item_cap,
-                                                    HeavyItem* __restrict__ items, uint64_t* __restrict__ err,
-                                                    uint64_t* __restrict__ total_out)
-{
-    // nbins is a power of two up to 2^15: thread t owns sub-buckets
-    // [t * per, (t + 1) * per), per = nbins / 1024 (at least 1); counts read as
-    // 16-byte vectors and starts written in pairs from 4 sub-buckets on
-    constexpr int MAXPER = 32;
-    __shared__ uint64_t wtmp[1024 / WAVE + 1];
-    const int per = max(1, nbins >> 10);
-    const int b0 = (int)threadIdx.x * per, b1 = min(b0 + per, nbins);
-    uint32_t v[MAXPER];
-    if (per >= 4) {
-        const uint4* n4 = (const uint4*)(n_items + b0);
-#pragma unroll
-        for (int j = 0; j < MAXPER / 4; j++) {
-            const uint4 q = (4 * j < per) ? n4[j] : make_uint4(0u, 0u, 0u, 0u);
-            v[4 * j] = q.x;
-            v[4 * j + 1] = q.y;
-            v[4 * j + 2] = q.z;
-            v[4 * j + 3] = q.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = (b0 + i < b1) ? n_items[b0 + i] : 0u;
-#pragma unroll
-        for (int i = 4; i < MAXPER; i++) v[i] = 0u;
-    }
-    uint64_t sum = 0;
-#pragma unroll
-    for (int i = 0; i < MAXPER; i++) sum += v[i];
-    uint64_t total;
-    uint64_t base = block_exclusive_scan<1024, uint64_t>(sum, wtmp, &total);
-    if (threadIdx.x == 0) {
-        item_start[nbins] = total;
-        if (total_out) *total_out = total;
-    }
-    if (per >= 4) {
-        ulonglong2* o2 = (ulonglong2*)(item_start + b0);
-        uint64_t e = base;
-#pragma unroll
-        for (int j = 0; j < MAXPER / 2; j++) {
-            const uint64_t e0 = e, e1 = e + v[2 * j];
-            e = e1 + v[2 * j + 1];
-            if (2 * j < per) o2[j] = make_ulonglong2(e0, e1);
-        }
-    }
-    bool over = false;
-#pragma unroll
-    for (int i = 0; i < MAXPER; i++) {
-        const int sb = b0 + i;
-        if (sb < b1) {
-            if (per < 4) item_start[sb] = base;
-            if (v[i]) {
-                uint64_t r0, nr, s0, ns;
-                sb_sizes(r_start, s_start, s_cnt, sb, r0, nr, s0, ns);
-                uint32_t chunks, slices;
-                plan_items(nr, ns, tile, slice, max_slices, chunks, slices);
-                if (base + v[i] > item_cap) {
-                    over = true;
-                } else {
-                    for (uint32_t c = 0; c < chunks; c++)
-                        for (uint32_t q = 0; q < slices; q++) {
-                            HeavyItem it;
-                            it.sb = (uint32_t)sb;
-                            it.chunk = c;
-                            it.slice = q;
-                            it.nslices = slices;
-                            items[base + (uint64_t)c * slices + q] = it;
-                        }
-                }
-            }
-            base += v[i];
-        }
-    }
-    if (over) atomicOr((unsigned long long*)err, 4ull);
-}
-
 // ============================================================== build + probe
 // Persistent workgroups pull work items from a global counter (the next item
 // is fetched while the current one runs): first the vlsplit items (the
@@ -1191,11 +1205,32 @@ hipError_t kernels_init(int max_lds_bytes)
     return hipSuccess;
 }
 
-hipError_t launch_hist(const uint32_t* key, uint64_t n_host, const uint64_t* n_dev, int G, int bits,
-                       uint32_t* part, uint32_t* totals, int bits2, uint32_t* l1h, hipStream_t st)
+static Sides sides_of(const PartSide* sides, int n, int (*wgs)(const PartSide&), int& grid)
 {
-    const size_t lds = sizeof(uint32_t) << bits;
-    k_hist<HIST_BLOCK><<<G, HIST_BLOCK, lds, st>>>(key, n_host, n_dev, G, bits, part, totals, bits2, l1h);
+    Sides S;
+    S.a = sides[0];
+    S.b = sides[n - 1];
+    S.na = wgs(sides[0]);
+    grid = S.na + (n > 1 ? wgs(sides[1]) : 0);
+    return S;
+}
+
+hipError_t launch_hist(const PartSide* sides, int n, uint64_t* ctr, int n_ctr, uint32_t* zero32, int n_zero32,
+                       hipStream_t st)
+{
+    int grid;
+    const Sides S = sides_of(sides, n, [](const PartSide& s) { return s.G; }, grid);
+    const size_t lds = sizeof(uint32_t) << std::max(S.a.bits, S.b.bits);
+    k_hist<HIST_BLOCK><<<grid, HIST_BLOCK, lds, st>>>(S, ctr, n_ctr, zero32, n_zero32);
+    return hipGetLastError();
+}
+
+hipError_t launch_cols(const PartSide* sides, int n, hipStream_t st)
+{
+    int grid;
+    const Sides S = sides_of(sides, n, [](const PartSide& s) { return cols_wgs(s); }, grid);
+    if (S.a.bits > 15 || S.b.bits > 15) return hipErrorInvalidValue;
+    k_cols<<<grid, 1024, 0, st>>>(S);
     return hipGetLastError();
 }
 
@@ -1204,17 +1239,6 @@ hipError_t launch_zero_u32(uint32_t* p, uint64_t n, hipStream_t st)
     if (n == 0) return hipSuccess;
     const int grid = (int)std::min<uint64_t>(4096, (n + 255) / 256);
     k_zero_u32<<<grid, 256, 0, st>>>(p, n);
-    return hipGetLastError();
-}
-
-hipError_t launch_offsets(const uint32_t* part, int G, int bits, int bits2, int W, uint32_t* colsum,
-                          uint32_t* totals, uint32_t* l1h, uint64_t* sb_start, uint64_t* l1off, hipStream_t st)
-{
-    if (bits > 15) return hipErrorInvalidValue;
-    const int nbins = 1 << bits, P1 = 1 << (bits - bits2);
-    k_colsums<<<ceil_div_i(nbins, 1024) * W, 1024, 0, st>>>(part, G, bits, W, colsum, totals);
-    k_starts<<<1, 1024, 0, st>>>(totals, nbins, sb_start);
-    k_l1_offsets<<<ceil_div_i(P1, L1_COLS), 1024, 0, st>>>(bits2 ? l1h : part, G, P1, bits2, sb_start, l1off);
     return hipGetLastError();
 }
 
@@ -1231,77 +1255,59 @@ hipError_t launch_scan(const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* 
     return hipGetLastError();
 }
 
-// Write-combining geometry: tile T = SC_BLOCK * SC_ITEMS tuples, carry chunk
-// cs tuples (64 B up to 512 buckets, then 32 B / 16 B so the carry stays at
-// 64 KB of LDS).
-int scatter_carry(int nbk) { return nbk <= 512 ? 16 : (nbk <= 1024 ? 8 : 4); }
-
-static int log2i(int x)
+static size_t scatter_lds_tile(int nbk, int tile, int cs_log2)
 {
-    int l = 0;
-    while ((1 << l) < x) l++;
-    return l;
+    return (size_t)nbk * SCATTER_BUCKET_BYTES + ((size_t)nbk << cs_log2) * 8 + (size_t)tile * 8 +
+           (SC_BLOCK / WAVE + 1) * 4;
 }
 
-// One-workgroup-per-CU launches have the CU's LDS to themselves: whole 128-byte
-// lines of keys and of values per carried chunk up to 256 buckets.  (Tuples
-// written whole fill a 128-byte line with a chunk of 16.)
-static int scatter_carry_big(int nbk, bool opair) { return !opair && nbk <= 256 ? 32 : scatter_carry(nbk); }
-
-static size_t scatter_lds_tile(int nbk, int tile, int cs)
+size_t scatter_lds_bytes(int nbk)
 {
-    return (size_t)nbk * SCATTER_BUCKET_BYTES + (size_t)nbk * cs * 8 + (size_t)tile * 8 + (SC_BLOCK / WAVE + 1) * 4;
+    return scatter_lds_tile(nbk, SC_BLOCK * SC_ITEMS, scatter_carry_log2(nbk, false, false));
 }
-
-size_t scatter_lds_bytes(int nbk) { return scatter_lds_tile(nbk, SC_BLOCK * SC_ITEMS, scatter_carry(nbk)); }
 
 size_t scatter_lds_bytes_big(int nbk)
 {
-    return scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, scatter_carry_big(nbk, false));
+    return scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, scatter_carry_log2(nbk, true, false));
 }
 
 template <bool IPAIR, bool OPAIR>
-static hipError_t scatter_pass(TupleIn<IPAIR> in, TupleOut<OPAIR> out, uint64_t out_cap, uint64_t n_host,
-                               const uint64_t* n_dev, int G, int mode, int bits, int p1, int W2,
-                               const uint64_t* l1off, const uint64_t* sb_start, const uint32_t* colsum, uint64_t* err,
-                               int wg, size_t min_lds, hipStream_t st)
+static hipError_t scatter_pass(const PartSide* sides, int n, const PlanArgs& plan, uint64_t* err, int wg,
+                               size_t min_lds, hipStream_t st)
 {
-    const int nbk = (mode == 0) ? (1 << p1) : (1 << (bits - p1));
-    const int grid = (mode == 0) ? G : (1 << p1) * W2;
-    const int cs = log2i(scatter_carry(nbk));
-    const size_t lds = std::max(scatter_lds_bytes(nbk), min_lds);
-    const int cs_big = scatter_carry_big(nbk, OPAIR);
-    const size_t lds_big = std::max(scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, cs_big), min_lds);
+    int grid;
+    const Sides S = sides_of(
+        sides, n, [](const PartSide& s) { return IPAIR ? (1 << s.p1) * s.W2 : s.G + 1; }, grid);
+    if (IPAIR && plan.items) grid++;
+    size_t lds = 0, lds_big = 0;
+    for (int i = 0; i < n; i++) {
+        const int nbk = IPAIR ? 1 << (sides[i].bits - sides[i].p1) : 1 << sides[i].p1;
+        lds = std::max(lds, scatter_lds_tile(nbk, SC_BLOCK * SC_ITEMS, scatter_carry_log2(nbk, false, OPAIR)));
+        lds_big =
+            std::max(lds_big, scatter_lds_tile(nbk, SC_BLOCK * SC_BIG_ITEMS, scatter_carry_log2(nbk, true, OPAIR)));
+    }
+    lds = std::max(lds, min_lds);
+    lds_big = std::max(lds_big, min_lds);
     if (wg != 512 && min_lds > 0 && lds_big <= g_max_lds) {
         // one workgroup per CU: twice the tile, twice the loads in flight, whole-line carries
-        k_scatter<SC_BLOCK, SC_BIG_ITEMS, IPAIR, OPAIR><<<grid, SC_BLOCK, lds_big, st>>>(
-            in, out, out_cap, n_host, n_dev, G, mode, bits, p1, W2, log2i(cs_big), l1off, sb_start, colsum, err);
+        k_scatter<SC_BLOCK, SC_BIG_ITEMS, IPAIR, OPAIR><<<grid, SC_BLOCK, lds_big, st>>>(S, plan, err);
     } else if (wg == 512) {
         // same tile (4096 tuples), half the threads: more workgroups per CU
-        k_scatter<SC_BLOCK / 2, SC_ITEMS * 2, IPAIR, OPAIR><<<grid, SC_BLOCK / 2, lds, st>>>(
-            in, out, out_cap, n_host, n_dev, G, mode, bits, p1, W2, cs, l1off, sb_start, colsum, err);
+        k_scatter<SC_BLOCK / 2, SC_ITEMS * 2, IPAIR, OPAIR><<<grid, SC_BLOCK / 2, lds, st>>>(S, plan, err);
     } else {
-        k_scatter<SC_BLOCK, SC_ITEMS, IPAIR, OPAIR><<<grid, SC_BLOCK, lds, st>>>(
-            in, out, out_cap, n_host, n_dev, G, mode, bits, p1, W2, cs, l1off, sb_start, colsum, err);
+        k_scatter<SC_BLOCK, SC_ITEMS, IPAIR, OPAIR><<<grid, SC_BLOCK, lds, st>>>(S, plan, err);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_scatter(int pass, const uint32_t* ikey, const uint32_t* ival, uint32_t* okey, uint32_t* oval,
-                          uint64_t out_cap, uint64_t n_host, const uint64_t* n_dev, int G, int bits, int p1, int W2,
-                          const uint64_t* l1off, const uint64_t* sb_start, const uint32_t* colsum, uint64_t* err,
-                          int wg, size_t min_lds, hipStream_t st)
+hipError_t launch_scatter(int pass, const PartSide* sides, int n, const PlanArgs* plan, uint64_t* err, int wg,
+                          size_t min_lds, hipStream_t st)
 {
+    const PlanArgs p = plan ? *plan : PlanArgs{};
     switch (pass) {
-    case SCATTER_ONLY:
-        return scatter_pass<false, false>({ikey, ival}, {okey, oval}, out_cap, n_host, n_dev, G, 0, bits, p1, W2,
-                                          l1off, sb_start, colsum, err, wg, min_lds, st);
-    case SCATTER_FIRST:
-        return scatter_pass<false, true>({ikey, ival}, {(Tuple*)okey}, out_cap, n_host, n_dev, G, 0, bits, p1, W2,
-                                         l1off, sb_start, colsum, err, wg, min_lds, st);
-    case SCATTER_SECOND:
-        return scatter_pass<true, false>({(const Tuple*)ikey}, {okey, oval}, out_cap, n_host, n_dev, G, 1, bits, p1,
-                                         W2, l1off, sb_start, colsum, err, wg, min_lds, st);
+    case SCATTER_ONLY: return scatter_pass<false, false>(sides, n, p, err, wg, min_lds, st);
+    case SCATTER_FIRST: return scatter_pass<false, true>(sides, n, p, err, wg, min_lds, st);
+    case SCATTER_SECOND: return scatter_pass<true, false>(sides, n, p, err, wg, min_lds, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -1379,17 +1385,10 @@ hipError_t launch_pool_merge(const uint32_t* pk, const uint32_t* pv, const uint3
     return hipGetLastError();
 }
 
-hipError_t launch_plan(const uint64_t* r_start, const uint64_t* s_start, const uint32_t* s_cnt, int bits,
-                       uint32_t tile, uint32_t slice, uint32_t max_slices, uint32_t* counts,
-                       uint64_t* item_start, uint64_t* total_out, HeavyItem* items, uint64_t item_cap,
-                       uint64_t* err, hipStream_t st)
+hipError_t launch_plan(const PlanArgs& plan, hipStream_t st)
 {
-    if (bits > 15) return hipErrorInvalidValue;
-    const int nbins = 1 << bits;
-    k_plan_count<<<ceil_div_i(nbins, 256), 256, 0, st>>>(r_start, s_start, s_cnt, nbins, tile, slice, max_slices,
-                                                         counts);
-    k_plan_fill<<<1, 1024, 0, st>>>(r_start, s_start, s_cnt, nbins, tile, slice, max_slices, counts, item_start,
-                                    item_cap, items, err, total_out);
+    if (plan.bits > 15) return hipErrorInvalidValue;
+    k_plan<1024><<<1, 1024, 0, st>>>(plan);
     return hipGetLastError();
 }
 

@@ -89,16 +89,28 @@ int bj_join_noalloc(bj_ctx* c, const bj_params* p, const uint32_t* r_key, const 
     }
     if (!base) return fail(BJ_ERR_HIP, "the scratch array's device address is not known for this device");
 
-    // the workspace, carved from the scratch array (the counters stay the context's)
+    // the workspace, carved from the scratch array (the counters stay the
+    // context's); R and S in the same launches only where that fits too
     std::vector<std::pair<DevBuf bj_ctx::*, uint64_t>> items;
     uint64_t total = 0;
-    workspace_items(pl, true, false, [&](DevBuf bj_ctx::*m, uint64_t bytes) -> int {
-        if (m != &bj_ctx::counters) {
-            items.emplace_back(m, align_up(bytes));
-            total += align_up(bytes);
-        }
-        return BJ_OK;
-    });
+    pl.direct = choose_direct(*p, pl);
+    pl.merge = !pl.direct && choose_merge(pl);
+    for (bool coarse = false;;) {
+        items.clear();
+        total = 0;
+        workspace_items(pl, true, false, [&](DevBuf bj_ctx::*m, uint64_t bytes) -> int {
+            if (m != &bj_ctx::counters) {
+                items.emplace_back(m, align_up(bytes));
+                total += align_up(bytes);
+            }
+            return BJ_OK;
+        });
+        if (total <= BJ_NOALLOC_SCRATCH_BYTES) break;
+        // without S's own set of partition buffers, then with longer chunks
+        if (pl.merge) pl.merge = false;
+        else if (!coarse) coarse_chunks(pl), coarse = true;
+        else break;
+    }
     if (total > BJ_NOALLOC_SCRATCH_BYTES)
         return fail(BJ_ERR_SIZE, "the join's workspace (" + std::to_string(total) + " B) exceeds the " +
                                      std::to_string((unsigned long long)BJ_NOALLOC_SCRATCH_BYTES) +
@@ -115,7 +127,6 @@ int bj_join_noalloc(bj_ctx* c, const bj_params* p, const uint32_t* r_key, const 
         off += it.second;
     }
     pl.cap = out_cap;
-    pl.direct = choose_direct(*p, pl);
     const bool timing = p->collect_phase_times != 0;
     tl_reset(c, timing);
     g_no_alloc = true;

@@ -104,6 +104,16 @@ struct ScatterLds {
 };
 constexpr int SCATTER_BUCKET_BYTES = 28;  // cur, dst, cnt, ol, nc
 
+// Carry chunk (log2 tuples) of an nbk-way pass.  big: one workgroup per CU, which
+// has the CU's LDS to itself.  Whole tuples fill a 128-byte line with 16; two
+// arrays need 32 for whole lines of each, affordable in big up to 256 buckets.
+// Above 512 buckets smaller chunks keep the carry at 64 KB.
+__host__ __device__ __forceinline__ int scatter_carry_log2(int nbk, bool big, bool opair)
+{
+    if (big && !opair && nbk <= 256) return 5;
+    return nbk <= 512 ? 4 : (nbk <= 1024 ? 3 : 2);
+}
+
 template <int BLOCK, int ITEMS>
 __device__ __forceinline__ ScatterLds scatter_lds(uint64_t* lds64, int nbk, int cs_log2)
 {
