@@ -166,28 +166,43 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan<uint32_t>(uint32_t x)
     return x;
 }
 
-// Block-wide exclusive scan of one value per thread.  `wtmp` holds
-// BLOCK/64 + 1 entries of LDS.  Returns the exclusive prefix; *total = sum.
+// Block-wide exclusive scan of one value per thread.  `wtmp` holds BLOCK/64 + 1
+// entries of LDS.  Returns the exclusive prefix; *total = sum.  Every wave sums the
+// waves' totals by itself, so there are two barriers: one before the totals are
+// read, one before they are rewritten.
 template <int BLOCK, typename T>
 __device__ __forceinline__ T block_exclusive_scan(T v, T* wtmp, T* total)
 {
     constexpr int NW = BLOCK / WAVE;
+    static_assert((NW & (NW - 1)) == 0 && NW <= 16, "wave totals in a row of lanes");
     const int wid = threadIdx.x / WAVE;
     const uint32_t lane = lane_id();
     const T inc = wave_inclusive_scan<T>(v);
     if (lane == WAVE - 1) wtmp[wid] = inc;
     __syncthreads();
-    if (wid == 0) {
-        T w = (lane < (uint32_t)NW) ? wtmp[lane] : (T)0;
-        T wi = wave_inclusive_scan<T>(w);
-        if (lane < (uint32_t)NW) wtmp[lane] = wi - w;
-        if (lane == (uint32_t)(NW - 1)) wtmp[NW] = wi;
+    T before, all;
+    if constexpr (sizeof(T) == 4) {
+        // the totals in every row of 16 lanes, summed by row shifts
+        T x = wtmp[lane & (NW - 1)];
+        x += (T)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+        x += (T)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+        if (NW > 4) x += (T)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+        if (NW > 8) x += (T)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+        const int w = __builtin_amdgcn_readfirstlane(wid);
+        before = w ? (T)__builtin_amdgcn_readlane((int)x, w - 1) : (T)0;
+        all = (T)__builtin_amdgcn_readlane((int)x, NW - 1);
+    } else {
+        before = all = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const T x = wtmp[w];
+            before += w < wid ? x : (T)0;
+            all += x;
+        }
     }
     __syncthreads();
-    const T res = wtmp[wid] + inc - v;
-    *total = wtmp[NW];
-    __syncthreads();
-    return res;
+    *total = all;
+    return before + inc - v;
 }
 
 // Exclusive scan of an LDS array in[0..n) into out[0..n) (may alias).

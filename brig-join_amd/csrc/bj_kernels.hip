@@ -938,9 +938,9 @@ __global__ __launch_bounds__(POOL_BLOCK) void k_pool_merge(
 }
 
 // ============================================================== build + probe
-// Persistent workgroups pull work items from a global counter (the next item
-// is fetched while the current one runs): first the vlsplit items (the
-// largest), then one item per regular sub-bucket.  Each item builds the
+// Persistent workgroups take work items in order, first the vlsplit items (the
+// largest), then one item per regular sub-bucket: the first by workgroup number,
+// the others from a global counter (claimed while the current one runs).  Each item builds the
 // build side's chunk into an LDS table and streams the other side's slice
 // past it (probe_item, bj_tiles.h).
 // COLLECT (the reference's COLLECT / --fused_probe_breakdown): thread 0 of
@@ -962,7 +962,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     uint64_t* __restrict__ timers)
 {
     __shared__ ProbeLds<BLOCK, CAP> L;
-    __shared__ uint64_t s_item, s_next;
+    __shared__ uint64_t s_next;
     uint64_t tacc[PT_N] = {}, tmark = 0;
     if (COLLECT && threadIdx.x == 0) tmark = phase_clock();
 
@@ -970,17 +970,20 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     const uint64_t n_heavy = min(*n_items_p, item_cap);
     const uint64_t n_work = n_heavy + (uint64_t)nbins;
 
-    // items are claimed PROBE_GRAB at a time: thread 0 waits for the queue's
-    // atomic once per claim instead of once per item
-    if (threadIdx.x == 0) s_item = atomicAdd((unsigned long long*)work_ctr, (unsigned long long)PROBE_GRAB);
-    __syncthreads();
-    uint64_t item = s_item;
-    int left = PROBE_GRAB;  // items of the current claim, this one included
-    __syncthreads();
+    // Items are claimed PROBE_GRAB at a time (the counter's answer is waited for
+    // once per claim), but one by one when there is no more than one claim for each
+    // workgroup: 3M x 4.5M has 512 items, which pairs would give to half of the 512
+    // workgroups (46.6 -> 32.2 us with the next line; 16M x 16M, 2048 items: 99-102 us
+    // in pairs, 105 us one by one).  The first claim is the workgroup's number: from
+    // the counter, the last of 512 answers would be several us away.
+    const int grab = n_work <= (uint64_t)gridDim.x * PROBE_GRAB ? 1 : PROBE_GRAB;
+    uint64_t item = (uint64_t)blockIdx.x * grab;
+    const uint64_t claimed = (uint64_t)gridDim.x * grab;
+    int left = grab;  // items of the current claim, this one included
 
     while (item < n_work) {
         if (left == 1 && threadIdx.x == 0)
-            s_next = atomicAdd((unsigned long long*)work_ctr, (unsigned long long)PROBE_GRAB);
+            s_next = atomicAdd((unsigned long long*)work_ctr, (unsigned long long)grab);
 
         uint32_t sb, chunk = 0, sl = 0, nsl = 1;
         const bool heavy = item < n_heavy;
@@ -1015,8 +1018,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
             item++;
             left--;
         } else {
-            item = s_next;
-            left = PROBE_GRAB;
+            item = claimed + s_next;
+            left = grab;
         }
         __syncthreads();
     }

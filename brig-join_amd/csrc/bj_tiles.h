@@ -586,7 +586,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     __syncthreads();
     phase_tick<COLLECT>(tacc, tmark, PT_CLEAR);
     // build: rank each tuple in its bucket, scan the counts, place;
-    // bucket (< 2^15) and rank (< 2^16) of each build tuple, packed
+    // bucket (< 2^15) and rank (< 2^16) of each build tuple, packed, then its slot
     uint32_t bkey[BPT], btr[BPT];
 #pragma unroll
     for (int u = 0; u < BPT; u++) {
@@ -596,6 +596,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
 #pragma unroll
     for (int u = 0; u < BPT; u++) {
         const int i = u * BLOCK + threadIdx.x;
+        btr[u] = 0;
         if (i < bn) {
             const uint32_t t = bucket(bkey[u]);
             btr[u] = (atomicAdd(&cnt[t], 1u) << 16) | t;
@@ -635,13 +636,16 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         if (threadIdx.x == 0) L.bst[nbk] = (uint16_t)bn;
     }
     __syncthreads();
+    // every tuple's bucket start is read before the first is placed (reads inside
+    // the branches below would be waited for one by one)
+#pragma unroll
+    for (int u = 0; u < BPT; u++) btr[u] = (uint32_t)L.bst[btr[u] & 0xFFFFu] + (btr[u] >> 16);
 #pragma unroll
     for (int u = 0; u < BPT; u++) {
         const int i = u * BLOCK + threadIdx.x;
         if (i < bn) {
-            const uint32_t q = (uint32_t)L.bst[btr[u] & 0xFFFFu] + (btr[u] >> 16);
-            L.hkey[q] = bkey[u];
-            L.hidx[q] = (uint16_t)i;
+            L.hkey[btr[u]] = bkey[u];
+            L.hidx[btr[u]] = (uint16_t)i;
         }
     }
     __syncthreads();
