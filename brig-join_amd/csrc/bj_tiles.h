@@ -180,9 +180,9 @@ __device__ __forceinline__ void scatter_offsets(const ScatterLds& L, int b0, boo
 // barrier).  Writes are bounds-checked against out_cap; returns true on a
 // violation.
 //
-// Per tile three barriers: ranks (LDS atomics) | offsets (scan of the counts,
-// retiring the previous tile's buckets and sizing this tile's writes) | staging +
-// next tile's loads + carried tuples out | the tile's tuples out or into the carry
+// Per tile three barriers: (next tile's loads) ranks (LDS atomics) | offsets (scan of
+// the counts, retiring the previous tile's buckets and sizing this tile's writes) |
+// staging + (or here the loads) + carried tuples out | the tile's tuples out or into the carry
 // (which runs into the next tile's ranks).  Counts alternate between the halves of
 // a word so the next tile's ranks need no clearing barrier.
 //
@@ -191,8 +191,8 @@ __device__ __forceinline__ void scatter_offsets(const ScatterLds& L, int b0, boo
 // loads are unconditional (clamped to the last tuple): with a branch per tuple the
 // compiler waited for each load, and for each LDS read, before it issued the next.
 // HBM bandwidth bounds large passes: 640M tuples by 128 buckets into whole tuples
-// 2.43 -> 2.25 ms (4.5 TB/s; a plain copy reaches 4.96), by 256 buckets 2.88 -> 2.47,
-// a second pass 2.67 -> 2.53; 100M tuples 0.45 -> 0.33 ms.  Whole tuples halve a
+// 2.43 -> 2.24 ms (4.6 TB/s; a plain copy reaches 4.96), by 256 buckets 2.88 -> 2.41,
+// a second pass 2.67 -> 2.43; 100M tuples 0.45 -> 0.33 ms.  Whole tuples halve a
 // bucket's carry (16 tuples fill a 128-byte line) and the store instructions.
 template <int BLOCK, int ITEMS, bool IPAIR, bool OPAIR>
 __device__ __forceinline__ bool scatter_range(const ScatterLds& L, const TupleIn<IPAIR>& in, uint32_t len, int nbk,
@@ -211,17 +211,21 @@ __device__ __forceinline__ bool scatter_range(const ScatterLds& L, const TupleIn
     __syncthreads();  // cur is read by other threads
     if (len == 0) return false;
 
-    Tuple kv[ITEMS];
-    auto load_tile = [&](uint32_t at) {
+    Tuple kv[ITEMS], nx[ITEMS];
+    auto load_tile = [&](Tuple* x, uint32_t at) {
 #pragma unroll
-        for (int it = 0; it < ITEMS; it++) kv[it] = in.load(min(at + (uint32_t)it * BLOCK + threadIdx.x, len - 1u));
+        for (int it = 0; it < ITEMS; it++) x[it] = in.load(min(at + (uint32_t)it * BLOCK + threadIdx.x, len - 1u));
     };
-    load_tile(0);
+    load_tile(kv, 0);
     bool bad = false;
     uint32_t par = 0;
 
     auto run_tile = [&](auto whole, uint32_t tile, uint32_t tn) {
         constexpr bool WHOLE = decltype(whole)::value;
+        // one workgroup per CU: no other workgroup's loads fill the time until this
+        // tile is staged, and there are registers for a second tile
+        constexpr bool EARLY = WHOLE && ITEMS == 8 && BLOCK == 1024;
+        if (EARLY) load_tile(nx, tile + T);
         uint32_t br[ITEMS];  // bucket | rank << 16
         const uint32_t one = par ? 1u << 16 : 1u, half = par ? 16u : 0u;
 #pragma unroll
@@ -257,8 +261,9 @@ __device__ __forceinline__ bool scatter_range(const ScatterLds& L, const TupleIn
 #pragma unroll
         for (int it = 0; it < ITEMS; it++)
             if (WHOLE || (uint32_t)it * BLOCK + threadIdx.x < tn) L.stage[q[it]] = kv[it];
-        // the next tile, in flight while this one is written out
-        if (WHOLE && tile + T < len) load_tile(tile + T);
+        // (two workgroups per CU: the next tile takes the registers of the staged one;
+        // its own registers spill, 3M x 4.5M's second pass 33 -> 40 us)
+        if (WHOLE && !EARLY && tile + T < len) load_tile(kv, tile + T);
         // carried tuples of the buckets that are written go out
         for (uint32_t i0 = threadIdx.x; i0 < ncarry; i0 += U * BLOCK) {
             uint32_t nc[U];
@@ -309,6 +314,10 @@ __device__ __forceinline__ bool scatter_range(const ScatterLds& L, const TupleIn
                     L.carry[(b[u] << cs_log2) + s - (ol[u] >> 16) + ((nc & 0xFFFFu) ? 0u : nc >> 16)] = x[u];
                 }
             }
+        }
+        if (EARLY) {
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) kv[it] = nx[it];
         }
         par ^= 1u;
     };
