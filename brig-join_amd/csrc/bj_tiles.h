@@ -511,25 +511,25 @@ __device__ __forceinline__ bool filter_run(uint32_t end, Next&& next, Desc&& des
 // The probe side (pn keys) streams through in rounds of BLOCK*PITEMS keys (the
 // next round is loaded while the current one is processed).  Each round counts
 // its matches and block-scans the counts.  A round with at most STAGE rows
-// stages them in LDS as (probe row, build row) pairs and reserves them with one
-// global atomic; the next round loads their keys and values, one or two rows
-// per thread, and the round after stores them after its own count (stores by
-// consecutive threads).  Larger rounds reserve and write from the lanes at
-// once.  Both
+// stages them in LDS as (probe row, table slot) pairs, reserved together with
+// those of the round before or after by one global atomic; the keys and values
+// are loaded two rounds later, one or two rows per thread, and stored after the
+// third round's count (stores by consecutive threads).  Larger rounds reserve and
+// write from the lanes at once.  Both
 // values of a row are read only for matches: the build side's from its
 // (cache-resident) chunk, the probe side's from its slice.  Rows past out_cap
 // are counted, not written.
 template <int BLOCK, int CAP>
 struct alignas(16) ProbeLds {
-    static constexpr int STAGE = 2 * BLOCK;  // rows of one round staged in LDS
-    uint32_t stage_p[2][STAGE];  // probe-side row of each of a round's rows, two
-                                 // rounds (first: short LDS offsets)
-    uint16_t stage_b[2][STAGE];  // table slot of the build tuple (its key and row)
+    static constexpr int STAGE = CAP / 8;  // rows of one round staged in LDS: one or two per thread
+    // a round's rows, three rounds (first: short LDS offsets): probe-side row of the
+    // round | table slot of the build tuple (its key and row) << 16
+    uint32_t stage[3][STAGE];
     uint32_t hkey[CAP];        // keys by bucket (bucket counts while the table is built)
     uint16_t hidx[CAP];
     uint16_t bst[CAP + 2];     // bucket starts, CAP buckets at most
     uint32_t wtmp[BLOCK / WAVE + 1];
-    unsigned long long s_base[2];  // reservations of staged rounds being stored
+    unsigned long long s_base[3];  // reservations of staged rounds being stored
     unsigned long long s_direct;  // reservation of a round written from the lanes
 };
 
@@ -664,62 +664,72 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     uint32_t nk[PITEMS];
 #pragma unroll
     for (int it = 0; it < PITEMS; it++) nk[it] = pkp[min((uint32_t)it * BLOCK + threadIdx.x, pn - 1u)];
-    // Rows are written two rounds late, with two barriers per round (those of
-    // the count scan): round r stages the (probe row, build row) pairs of its
-    // matches in stage[r & 1] and reserves their places (one atomic by thread 0);
-    // round r + 1 loads the key and values of rows tid and tid + BLOCK; round
-    // r + 2 stores them after its count, at the reservation thread 0 published
-    // in s_base[r & 1] before that round's scan.  The scan barriers of the round
-    // in between separate every LDS write from the reads of the same slot.  No
-    // wait for a reservation or a value load is on a round's path.
-    uint32_t wk0, wp0, wb0, wk1, wp1, wb1;  // loaded rows: key, probe / build value
+    // Rows are written three rounds late, with two barriers per round (those of the
+    // count scan): round r stages the (probe row, table slot) pairs of its matches in
+    // stage[r % 3]; round r + 2 loads the key and values of rows tid, tid + BLOCK, ...;
+    // round r + 3 stores them after its count, at the place thread 0 published before
+    // that round's scan.  The scan barriers of the rounds between separate every LDS
+    // write from the reads of the same slot.  No wait for a reservation or a value
+    // load is on a round's path.
+    // One atomic reserves the rows of two rounds (an odd one and the one before): the
+    // chip does about 70 atomics on one address per us, and one per round of 5120 keys
+    // was as many (640M x 640M: 125K in 1.94 ms; rounds of 4096 keys took 2.24 ms, of
+    // 6144 keys 1.76).  Now 1.69 ms; 16M x 16M's probe 100 -> 93 us.
+    constexpr int NR = STAGE / BLOCK;
+    uint32_t wk[NR], wp[NR], wb[NR];  // loaded rows: key, probe / build value
     uint32_t n_loaded = 0;          // rows in the registers, stored this round (uniform)
-    uint32_t n_staged = 0;          // rows staged last round, loaded this round (uniform)
-    unsigned long long sb_loaded = 0, sb_staged = 0;  // thread 0: their reservations
-    uint32_t par = 0;               // round parity
+    uint32_t n_last = 0, n_prev = 0;  // rows staged last round and in the one before (uniform)
+    // thread 0: the reservations of the loaded rows and of those of the pairs of
+    // rounds that the last two belong to; a pair's second round lies behind its first
+    unsigned long long sb_loaded = 0, sb_pair = 0;
+    uint32_t off_loaded = 0, off_prev = 0, off_last = 0;
+    uint32_t r3 = 0;                // round number mod 3
+    bool odd = false;               // of the round
     // The key and build row come from the table (LDS), the values from global
     // memory.  The four loads are issued in every round, also where nothing is
     // staged (row 0 of the probe side and table slot 0, unused): the loads in
     // flight at the top of a round are then the same on every path (the next
     // keys, then these four), so waiting for the keys never waits for these.
-    auto load_rows = [&](uint32_t n, int buf) {
-        uint32_t p0 = 0, q0s = 0, p1 = 0, q1s = 0;
-        if (n) {  // uniform; rows tid and tid + BLOCK, clamped to the last row
-            const uint32_t j0 = min((uint32_t)threadIdx.x, n - 1u);
-            const uint32_t j1 = min((uint32_t)threadIdx.x + BLOCK, n - 1u);
-            p0 = L.stage_p[buf][j0];
-            q0s = L.stage_b[buf][j0];
-            p1 = L.stage_p[buf][j1];
-            q1s = L.stage_b[buf][j1];
+    auto load_rows = [&](uint32_t n, uint32_t buf, uint32_t base, uint32_t* wk, uint32_t* wp, uint32_t* wb) {
+        uint32_t p[NR], q[NR], b[NR];
+#pragma unroll
+        for (int u = 0; u < NR; u++) {
+            p[u] = q[u] = 0;
+            if (n) {  // uniform; rows tid, tid + BLOCK, clamped to the last row
+                const uint32_t j = min((uint32_t)(u * BLOCK) + threadIdx.x, n - 1u);
+                const uint32_t x = L.stage[buf][j];
+                p[u] = base + (x & 0xFFFFu);
+                q[u] = x >> 16;
+            }
         }
-        wk0 = L.hkey[q0s];
-        wk1 = L.hkey[q1s];
-        uint32_t b0 = L.hidx[q0s], b1 = L.hidx[q1s];
-        // per-lane rows: vector loads on every path (a known row 0 would become
-        // a scalar load, which the vector load counter does not see)
-        asm volatile("" : "+v"(p0), "+v"(b0), "+v"(p1), "+v"(b1));
-        wp0 = pvp[p0];
-        wp1 = pvp[p1];
-        wb0 = bvp[b0];
-        wb1 = bvp[b1];
+#pragma unroll
+        for (int u = 0; u < NR; u++) {
+            wk[u] = L.hkey[q[u]];
+            b[u] = L.hidx[q[u]];
+            // per-lane rows: vector loads on every path (a known row 0 would become
+            // a scalar load, which the vector load counter does not see)
+            asm volatile("" : "+v"(p[u]), "+v"(b[u]));
+        }
+#pragma unroll
+        for (int u = 0; u < NR; u++) wp[u] = pvp[p[u]];
+#pragma unroll
+        for (int u = 0; u < NR; u++) wb[u] = bvp[b[u]];
     };
-    auto flush = [&](uint32_t n, int slot) {  // after a barrier that published L.s_base[slot]
+    auto flush = [&](uint32_t n, uint32_t slot, const uint32_t* wk, const uint32_t* wp, const uint32_t* wb) {  // after a barrier that published L.s_base[slot]
         const uint64_t sb = uniform_u64(L.s_base[slot]);
         const uint32_t nw = sb >= out_cap ? 0u : (uint32_t)min<uint64_t>(n, out_cap - sb);
-        const uint32_t j0 = threadIdx.x, j1 = threadIdx.x + BLOCK;
-        if (j0 < nw) {
-            o_key[sb + j0] = wk0;
-            o_rval[sb + j0] = build_r ? wb0 : wp0;
-            o_sval[sb + j0] = build_r ? wp0 : wb0;
-        }
-        if (j1 < nw) {
-            o_key[sb + j1] = wk1;
-            o_rval[sb + j1] = build_r ? wb1 : wp1;
-            o_sval[sb + j1] = build_r ? wp1 : wb1;
+#pragma unroll
+        for (int u = 0; u < NR; u++) {
+            const uint32_t j = (uint32_t)(u * BLOCK) + threadIdx.x;
+            if (j < nw) {
+                o_key[sb + j] = wk[u];
+                o_rval[sb + j] = build_r ? wb[u] : wp[u];
+                o_sval[sb + j] = build_r ? wp[u] : wb[u];
+            }
         }
     };
-    load_rows(0, 0);
-    for (uint32_t base = 0; base < pn; base += ROUND, par ^= 1u) {
+    load_rows(0, 0, 0, wk, wp, wb);
+    for (uint32_t base = 0; base < pn; base += ROUND, r3 = r3 == 2u ? 0u : r3 + 1u, odd = !odd) {
         uint32_t kk[PITEMS], qs[PITEMS], qe[PITEMS];
 #pragma unroll
         for (int it = 0; it < PITEMS; it++) kk[it] = nk[it];
@@ -760,46 +770,50 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             hitmask |= (m ? 1u : 0u) << it;
             multi |= (m > 1 ? 1u : 0u) << it;
         }
-        // the reservation of the rows stored this round (staged two rounds ago,
-        // in slot par; its last reader was that round's store, before the last
-        // round's scan barriers)
-        if (threadIdx.x == 0 && n_loaded) L.s_base[par] = sb_loaded;
+        // the place of the rows stored this round (the slot's last reader was the
+        // store three rounds ago)
+        if (threadIdx.x == 0 && n_loaded) L.s_base[r3] = sb_loaded + off_loaded;
         uint32_t total;
         const uint32_t pre = block_exclusive_scan<BLOCK, uint32_t>(c, L.wtmp, &total);
         phase_tick<COLLECT>(tacc, tmark, PT_COUNT);
-        if (n_loaded) flush(n_loaded, (int)par);
-        // last round's staged rows into the registers (stage[par ^ 1] was
-        // written before this round's scan barriers)
-        load_rows(n_staged, (int)(par ^ 1u));
-        n_loaded = n_staged;
-        sb_loaded = sb_staged;
-        n_staged = 0;
+        if (n_loaded) flush(n_loaded, r3, wk, wp, wb);
+        // the rows of the round before the last into the registers (stage[r3 + 1 mod 3])
+        load_rows(n_prev, r3 == 2u ? 0u : r3 + 1u, base - 2u * ROUND, wk, wp, wb);
+        const bool wrote = n_loaded != 0u;
+        n_loaded = n_prev;
+        sb_loaded = sb_pair;
+        off_loaded = off_prev;
+        n_prev = n_last;
+        off_prev = off_last;
+        const bool large = total > (uint32_t)STAGE;  // uniform
+        n_last = large ? 0u : total;
+        off_last = odd ? n_prev : 0u;
+        // this round's rows, and those of the round before where it opened a pair
+        const uint32_t res = n_last + off_last;
+        const bool last = pn - base <= (uint32_t)ROUND;
+        if (threadIdx.x == 0 && (odd || last)) {
+            // (a last round without a second: the round before belongs to the pair before)
+            if (last && !odd) L.s_base[r3 == 0u ? 2u : r3 - 1u] = sb_pair + off_prev;
+            if (res) sb_pair = atomicAdd((unsigned long long*)out_count, (unsigned long long)res);
+        }
         if (total == 0) {  // uniform
-            if (n_loaded) phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
+            if (wrote) phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
             continue;
         }
-        if (total <= (uint32_t)STAGE) {  // uniform
-            if (threadIdx.x == 0) sb_staged = atomicAdd((unsigned long long*)out_count, (unsigned long long)total);
+        if (!large) {
             uint32_t w = pre;
+            uint32_t* const st = L.stage[r3];
 #pragma unroll
             for (int it = 0; it < PITEMS; it++) {
                 if (hitmask & (1u << it)) {
-                    const uint32_t prow = base + (uint32_t)it * BLOCK + threadIdx.x;
-                    L.stage_p[par][w] = prow;
-                    L.stage_b[par][w] = (uint16_t)qm[it];
-                    w++;
+                    const uint32_t prow = (uint32_t)it * BLOCK + threadIdx.x;
+                    st[w++] = prow | qm[it] << 16;
                     if (multi & (1u << it)) {
-                        for (uint32_t q = (qm[it] & 0xFFFFu) + 1; q < qm[it] >> 16; q++) {
-                            if (L.hkey[q] == kk[it]) {
-                                L.stage_p[par][w] = prow;
-                                L.stage_b[par][w] = (uint16_t)q;
-                                w++;
-                            }
-                        }
+                        for (uint32_t q = (qm[it] & 0xFFFFu) + 1; q < qm[it] >> 16; q++)
+                            if (L.hkey[q] == kk[it]) st[w++] = prow | q << 16;
                     }
                 }
             }
-            n_staged = total;
             phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
             continue;
         }
@@ -847,33 +861,36 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             }
         } else {
             // duplicate build keys: the wave's rows go through its share of the
-            // round's stage (free: stage[par] was last read a round ago), two rows
-            // per lane at a time, so the values of up to 128 rows are in flight
-            // instead of one per match of a lane
+            // round's stage (free: stage[r3] was last read a round ago), so the
+            // values of all its rows are in flight instead of one per match of a lane
             __syncthreads();
             constexpr uint32_t FIFO = STAGE / (BLOCK / WAVE);
-            static_assert(FIFO == 2 * WAVE, "two rows per lane");
+            static_assert(FIFO == 2 * WAVE || FIFO == WAVE, "one or two rows per lane");
             const uint32_t lane = lane_id();
-            uint32_t* fp = &L.stage_p[par][threadIdx.x / WAVE * FIFO];
-            uint16_t* fb = &L.stage_b[par][threadIdx.x / WAVE * FIFO];
+            uint32_t* fifo = &L.stage[r3][threadIdx.x / WAVE * FIFO];
             uint64_t w = uniform_u64(L.s_direct + pre);
             uint32_t n = 0;  // rows in the wave's FIFO (uniform)
             auto drain = [&]() {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                const uint32_t j0 = min(lane, n - 1u), j1 = min(lane + WAVE, n - 1u);
-                const uint32_t p0 = fp[j0], s0 = fb[j0], p1 = fp[j1], s1 = fb[j1];
-                const uint32_t k0 = L.hkey[s0], b0 = L.hidx[s0], k1 = L.hkey[s1], b1 = L.hidx[s1];
-                const uint32_t pv0 = pvp[p0], pv1 = pvp[p1], bv0 = bvp[b0], bv1 = bvp[b1];
-                const uint32_t nw = min(n, room(w));
-                if (lane < nw) {
-                    (o_key + w)[lane] = k0;
-                    (o_rval + w)[lane] = build_r ? bv0 : pv0;
-                    (o_sval + w)[lane] = build_r ? pv0 : bv0;
+                constexpr int NF = FIFO / WAVE;
+                uint32_t k[NF], pv[NF], bv[NF];
+#pragma unroll
+                for (int u = 0; u < NF; u++) {
+                    const uint32_t j = min(lane + u * WAVE, n - 1u);
+                    const uint32_t x = fifo[j];
+                    k[u] = L.hkey[x >> 16];
+                    pv[u] = pvp[base + (x & 0xFFFFu)];
+                    bv[u] = bvp[L.hidx[x >> 16]];
                 }
-                if (lane + WAVE < nw) {
-                    (o_key + w)[lane + WAVE] = k1;
-                    (o_rval + w)[lane + WAVE] = build_r ? bv1 : pv1;
-                    (o_sval + w)[lane + WAVE] = build_r ? pv1 : bv1;
+                const uint32_t nw = min(n, room(w));
+#pragma unroll
+                for (int u = 0; u < NF; u++) {
+                    const uint32_t j = lane + u * WAVE;
+                    if (j < nw) {
+                        (o_key + w)[j] = k[u];
+                        (o_rval + w)[j] = build_r ? bv[u] : pv[u];
+                        (o_sval + w)[j] = build_r ? pv[u] : bv[u];
+                    }
                 }
                 w += n;
                 n = 0;
@@ -883,7 +900,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             for (int it = 0; it < PITEMS; it++) {
                 // this key's matches (its rows stay next to each other), places in
                 // the wave by a scan; the FIFO takes them in windows of its free room
-                const uint32_t prow = base + (uint32_t)it * BLOCK + threadIdx.x, qend = qm[it] >> 16;
+                const uint32_t prow = (uint32_t)it * BLOCK + threadIdx.x, qend = qm[it] >> 16;
                 uint32_t q = qm[it] & 0xFFFFu;
                 uint32_t left = (hitmask >> it) & 1u;
                 if ((multi >> it) & 1u)
@@ -894,8 +911,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
                 for (uint32_t w0 = 0; w0 < rows;) {
                     const uint32_t take = min(FIFO - n, rows - w0);
                     while (left && pos < w0 + take) {
-                        fp[n + pos - w0] = prow;
-                        fb[n + pos - w0] = (uint16_t)q;
+                        fifo[n + pos - w0] = prow | q << 16;
                         pos++;
                         if (--left)
                             while (L.hkey[++q] != kk[it]) {}
@@ -910,20 +926,25 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         // L.s_direct is rewritten only after the next round's scan barriers
         phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
     }
-    // the rows still in flight: those in the registers (slot par) and those
-    // staged by the last round (stage[par ^ 1], slot par ^ 1)
-    if (n_loaded || n_staged) {  // uniform
-        __syncthreads();  // the last round's store read slot par ^ 1 after its scan
+    // the rows still in flight: those in the registers and those staged by the last
+    // two rounds (r3: the number of rounds mod 3)
+    if (n_loaded || n_prev || n_last) {  // uniform
+        const uint32_t s1 = r3 == 2u ? 0u : r3 + 1u, s2 = 3u - r3 - s1;  // stages of the last but one, the last
+        const uint32_t base1 = (pn - 1u) / ROUND * ROUND;  // the last round's
+        __syncthreads();  // the last round's store read its slot of s_base
         if (threadIdx.x == 0) {
-            if (n_loaded) L.s_base[par] = sb_loaded;
-            if (n_staged) L.s_base[par ^ 1u] = sb_staged;
+            if (n_loaded) L.s_base[r3] = sb_loaded + off_loaded;
+            // (odd: of the round after the last)
+            if (n_prev && !odd) L.s_base[s1] = sb_pair + off_prev;
+            if (n_last) L.s_base[s2] = sb_pair + off_last;
         }
         __syncthreads();
-        if (n_loaded) flush(n_loaded, (int)par);
-        if (n_staged) {
-            load_rows(n_staged, (int)(par ^ 1u));
-            flush(n_staged, (int)(par ^ 1u));
-        }
+        uint32_t xk[NR], xp[NR], xb[NR], yk[NR], yp[NR], yb[NR];
+        if (n_prev) load_rows(n_prev, s1, base1 - ROUND, xk, xp, xb);
+        if (n_last) load_rows(n_last, s2, base1, yk, yp, yb);
+        if (n_loaded) flush(n_loaded, r3, wk, wp, wb);
+        if (n_prev) flush(n_prev, s1, xk, xp, xb);
+        if (n_last) flush(n_last, s2, yk, yp, yb);
         phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
     }
     // the caller synchronises before the next item rebuilds the table
