@@ -721,7 +721,11 @@ int enqueue_plan_probe(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t
         BJ_HIP(tl_end(c, BJ_K_PLAN));
     }
     BJ_HIP(tl_begin(c, BJ_K_PROBE));
-    BJ_HIP(launch_probe(pl.tile, R.key, R.val, R.start, sk, sv, s_start, s_cnt, pl.bits, pl.slice,
+    // (with a filter only R's share is known before the join)
+    const uint64_t per_r = pl.nr >> pl.bits, per_s = pl.ns >> pl.bits;
+    const uint64_t probe_mean = pl.bf ? (per_r > (uint64_t)pl.tile ? per_r : 0)
+                                      : (build_from_r(per_r, per_s, (uint32_t)pl.tile) ? per_s : per_r);
+    BJ_HIP(launch_probe(pl.tile, probe_mean, R.key, R.val, R.start, sk, sv, s_start, s_cnt, pl.bits, pl.slice,
                         P<HeavyItem>(c->items), ctr + CTR_ITEMS, pl.item_cap, ctr + CTR_WORK, ctr + CTR_OUT,
                         cap, o_key, o_rval, o_sval, c->num_cu,
                         pl.probe_breakdown ? P<uint64_t>(c->ptimers) : nullptr, st));

@@ -116,7 +116,8 @@ hipError_t launch_pool_merge(const uint32_t* pk, const uint32_t* pv, const uint3
                              int nch, int nbins, const uint64_t* start, uint32_t* ok, uint32_t* ov,
                              uint64_t out_cap, uint64_t* err, hipStream_t st);
 hipError_t launch_plan(const PlanArgs& plan, hipStream_t st);
-hipError_t launch_probe(int tile, const uint32_t* rk, const uint32_t* rv, const uint64_t* r_start,
+// probe_mean: probe tuples of a sub-bucket on average, as far as the host knows
+hipError_t launch_probe(int tile, uint64_t probe_mean, const uint32_t* rk, const uint32_t* rv, const uint64_t* r_start,
                         const uint32_t* sk, const uint32_t* sv, const uint64_t* s_start,
                         const uint32_t* s_cnt, int bits, uint32_t slice, const HeavyItem* items,
                         const uint64_t* n_items, uint64_t item_cap, uint64_t* work_ctr, uint64_t* out_count,

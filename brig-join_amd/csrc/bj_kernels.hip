@@ -951,7 +951,7 @@ __global__ __launch_bounds__(POOL_BLOCK) void k_pool_merge(
 constexpr int PROBE_GRAB = BJ_PROBE_GRAB;
 
 template <int BLOCK, int CAP, int PITEMS, bool COLLECT>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_probe(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_waves(BLOCK, CAP), 8))) void k_probe(
     const uint32_t* __restrict__ rk, const uint32_t* __restrict__ rv,
     const uint64_t* __restrict__ r_start, const uint32_t* __restrict__ sk,
     const uint32_t* __restrict__ sv, const uint64_t* __restrict__ s_start,
@@ -1062,7 +1062,7 @@ __global__ void k_direct_bloom(const uint32_t* __restrict__ rkey, uint32_t n, Bl
 // on one XCD (slices are dealt in multiples of 8), so its keys come from that
 // XCD's L2 after the first chunk.
 template <int BLOCK, int CAP, int PITEMS>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_join_direct(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_waves(BLOCK, CAP), 8))) void k_join_direct(
     const uint32_t* __restrict__ rk, const uint32_t* __restrict__ rv, uint32_t nr,
     const uint32_t* __restrict__ sk, const uint32_t* __restrict__ sv, uint32_t ns_host,
     const uint64_t* __restrict__ ns_dev, bool build_r, uint32_t grain, uint64_t* __restrict__ out_count,
@@ -1397,10 +1397,16 @@ hipError_t launch_plan(const PlanArgs& plan, hipStream_t st)
 
 int probe_grid(int tile, int num_cu) { return tile == 8192 ? num_cu * 2 : num_cu * 4; }
 
-// Probe keys per thread per round: 10 (a round of 5120 keys at 512 threads)
-// measured 11% faster than 8 on the 640M join, 6 was 23% slower, and 12 no
-// faster than 10 while spilling registers.
-constexpr int PROBE_ITEMS = 10;
+// Probe keys per thread per round of k_probe.  The rounds are chains of LDS latencies
+// between barriers, so the CU's 160 KB of tables are worked on by as many waves as it
+// holds: 1024 threads per 8192-tuple table (8 waves per SIMD, 64 registers) against
+// 512 threads with 10 keys each: ids 100M x 130M 742 -> 678 us, 9M x 24M with four
+// copies of each key 315 -> 259, 64M x 1.28B 289 -> 263, 3M x 4.5M 33.4 -> 29.7.  Rounds
+// of 3 keys per thread leave less of a short probe side's last round empty (ids with 4:
+// 693 us, 3M x 4.5M 35.2); from PROBE_LONG probe tuples per sub-bucket on 4 are better,
+// with fewer reservations (640M x 640M, 39K per sub-bucket: 1.52 ms, 3 keys 1.74).
+constexpr int PROBE_ITEMS = 3, PROBE_ITEMS_LONG = 4;
+constexpr uint64_t PROBE_LONG = 16384;
 
 static_assert(PT_N == PROBE_TIMER_SLOTS, "probe timer slots");
 
@@ -1431,43 +1437,46 @@ hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t n
     const uint64_t C = (nb + CAP - 1) / CAP;
     const uint64_t wgs = (uint64_t)probe_grid(CAP, num_cu);
     // one short round (2 keys per thread) per workgroup while that fills at most
-    // one wave of workgroups, else rounds of PROBE_ITEMS keys per thread
-    constexpr int SMALL_ITEMS = 2;
+    // one wave of workgroups, else rounds of DIRECT_ITEMS keys per thread
+    // (1024 threads of 3 keys as in k_probe: 6001 x 20M 159 -> 162 us)
+    constexpr int SMALL_ITEMS = 2, DIRECT_ITEMS = 10;
     const uint64_t small_slices = (np + B * SMALL_ITEMS - 1) / (B * SMALL_ITEMS);
     const bool small = C * small_slices <= wgs;
-    const uint32_t grain = B * (small ? SMALL_ITEMS : PROBE_ITEMS);
+    const uint32_t grain = B * (small ? SMALL_ITEMS : DIRECT_ITEMS);
     const int grid = (int)std::min<uint64_t>(wgs, C * std::max<uint64_t>(1, (np + grain - 1) / grain));
     if (small)
         k_join_direct<B, CAP, SMALL_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
                                                                build_r, grain, out_count, out_cap, o_key, o_rval,
                                                                o_sval);
     else
-        k_join_direct<B, CAP, PROBE_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
+        k_join_direct<B, CAP, DIRECT_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
                                                                build_r, grain, out_count, out_cap, o_key, o_rval,
                                                                o_sval);
     return hipGetLastError();
 }
 
-hipError_t launch_probe(int tile, const uint32_t* rk, const uint32_t* rv, const uint64_t* r_start,
+hipError_t launch_probe(int tile, uint64_t probe_mean, const uint32_t* rk, const uint32_t* rv, const uint64_t* r_start,
                         const uint32_t* sk, const uint32_t* sv, const uint64_t* s_start,
                         const uint32_t* s_cnt, int bits, uint32_t slice, const HeavyItem* items,
                         const uint64_t* n_items, uint64_t item_cap, uint64_t* work_ctr, uint64_t* out_count,
                         uint64_t out_cap, uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, int num_cu,
                         uint64_t* timers, hipStream_t st)
 {
-#define BJ_PROBE(B, C, G)                                                                                  \
+#define BJ_PROBE(B, C, I, G)                                                                               \
     do {                                                                                                 \
         if (timers)                                                                                      \
-            k_probe<B, C, PROBE_ITEMS, true><<<(G), B, 0, st>>>(rk, rv, r_start, sk, sv, s_start, s_cnt, bits, slice, \
+            k_probe<B, C, I, true><<<(G), B, 0, st>>>(rk, rv, r_start, sk, sv, s_start, s_cnt, bits, slice, \
                                                       items, n_items, item_cap, work_ctr, out_count,     \
                                                       out_cap, o_key, o_rval, o_sval, timers);           \
         else                                                                                             \
-            k_probe<B, C, PROBE_ITEMS, false><<<(G), B, 0, st>>>(rk, rv, r_start, sk, sv, s_start, s_cnt, bits,    \
+            k_probe<B, C, I, false><<<(G), B, 0, st>>>(rk, rv, r_start, sk, sv, s_start, s_cnt, bits,    \
                                                        slice, items, n_items, item_cap, work_ctr,        \
                                                        out_count, out_cap, o_key, o_rval, o_sval, nullptr); \
     } while (0)
-    if (tile == 8192) BJ_PROBE(512, 8192, probe_grid(8192, num_cu));
-    else if (tile == 4096) BJ_PROBE(256, 4096, probe_grid(4096, num_cu));
+    const bool long_probe = probe_mean >= PROBE_LONG;
+    if (tile == 8192 && long_probe) BJ_PROBE(1024, 8192, PROBE_ITEMS_LONG, probe_grid(8192, num_cu));
+    else if (tile == 8192) BJ_PROBE(1024, 8192, PROBE_ITEMS, probe_grid(8192, num_cu));
+    else if (tile == 4096) BJ_PROBE(512, 4096, PROBE_ITEMS, probe_grid(4096, num_cu));
     else return hipErrorInvalidValue;
 #undef BJ_PROBE
     return hipGetLastError();

@@ -533,6 +533,9 @@ struct alignas(16) ProbeLds {
     unsigned long long s_direct;  // reservation of a round written from the lanes
 };
 
+// waves per SIMD of a probe kernel: 8192-tuple tables two to a CU, 4096-tuple ones four
+constexpr int probe_waves(int block, int cap) { return block / WAVE * (cap == 8192 ? 2 : 4) / 4; }
+
 // Probe phase timers (one accumulator per workgroup, kept by thread 0, in
 // ticks of the constant-rate wall clock): fetching work items, clearing the
 // table, building it, counting the rounds' matches (through the reservation),
@@ -931,7 +934,11 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     if (n_loaded || n_prev || n_last) {  // uniform
         const uint32_t s1 = r3 == 2u ? 0u : r3 + 1u, s2 = 3u - r3 - s1;  // stages of the last but one, the last
         const uint32_t base1 = (pn - 1u) / ROUND * ROUND;  // the last round's
-        __syncthreads();  // the last round's store read its slot of s_base
+        __syncthreads();  // the last round's rows are staged, its store has read s_base
+        // the values are under way while thread 0 waits for the reservation
+        uint32_t xk[NR], xp[NR], xb[NR], yk[NR], yp[NR], yb[NR];
+        if (n_prev) load_rows(n_prev, s1, base1 - ROUND, xk, xp, xb);
+        if (n_last) load_rows(n_last, s2, base1, yk, yp, yb);
         if (threadIdx.x == 0) {
             if (n_loaded) L.s_base[r3] = sb_loaded + off_loaded;
             // (odd: of the round after the last)
@@ -939,9 +946,6 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             if (n_last) L.s_base[s2] = sb_pair + off_last;
         }
         __syncthreads();
-        uint32_t xk[NR], xp[NR], xb[NR], yk[NR], yp[NR], yb[NR];
-        if (n_prev) load_rows(n_prev, s1, base1 - ROUND, xk, xp, xb);
-        if (n_last) load_rows(n_last, s2, base1, yk, yp, yb);
         if (n_loaded) flush(n_loaded, r3, wk, wp, wb);
         if (n_prev) flush(n_prev, s1, xk, xp, xb);
         if (n_last) flush(n_last, s2, yk, yp, yb);
