@@ -973,7 +973,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_wav
     // Items are claimed PROBE_GRAB at a time (the counter's answer is waited for
     // once per claim), but one by one when there is no more than one claim for each
     // workgroup: 3M x 4.5M has 512 items, which pairs would give to half of the 512
-    // workgroups (46.6 -> 32.2 us with the next line; 16M x 16M, 2048 items: 99-102 us
+    // workgroups (46.6 -> 32.2 us with the next line, by 512 threads per table; 16M x 16M, 2048 items: 99-102 us
     // in pairs, 105 us one by one).  The first claim is the workgroup's number: from
     // the counter, the last of 512 answers would be several us away.
     const int grab = n_work <= (uint64_t)gridDim.x * PROBE_GRAB ? 1 : PROBE_GRAB;
