@@ -169,16 +169,17 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan<uint32_t>(uint32_t x)
 // Block-wide exclusive scan of one value per thread.  `wtmp` holds BLOCK/64 + 1
 // entries of LDS.  Returns the exclusive prefix; *total = sum.  Every wave sums the
 // waves' totals by itself, so there are two barriers: one before the totals are
-// read, one before they are rewritten.
+// read, one before they are rewritten.  wave_extra is added to the calling wave's
+// total (and so to *total and the later waves' prefixes).
 template <int BLOCK, typename T>
-__device__ __forceinline__ T block_exclusive_scan(T v, T* wtmp, T* total)
+__device__ __forceinline__ T block_exclusive_scan(T v, T* wtmp, T* total, T wave_extra = 0)
 {
     constexpr int NW = BLOCK / WAVE;
     static_assert((NW & (NW - 1)) == 0 && NW <= 16, "wave totals in a row of lanes");
     const int wid = threadIdx.x / WAVE;
     const uint32_t lane = lane_id();
     const T inc = wave_inclusive_scan<T>(v);
-    if (lane == WAVE - 1) wtmp[wid] = inc;
+    if (lane == WAVE - 1) wtmp[wid] = inc + wave_extra;
     __syncthreads();
     T before, all;
     if constexpr (sizeof(T) == 4) {

@@ -570,6 +570,9 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     constexpr int ROUND = BLOCK * PITEMS;
     constexpr int BPT = CAP / BLOCK;  // build tuples per thread
     constexpr int STAGE = ProbeLds<BLOCK, CAP>::STAGE;
+    // a wave's mark in its round's row count (at most 16 waves, 2^27 rows)
+    constexpr uint32_t DUPS = 1u << 27;
+    static_assert((uint64_t)ROUND * CAP < DUPS && BLOCK / WAVE <= 16, "row count and waves' marks in one word");
     static_assert(CAP % BLOCK == 0 && CAP <= 32768, "bucket and rank pack into 16 bits each");
     if (pn == 0) return;  // an empty slice (uniform)
 
@@ -777,7 +780,10 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         // store three rounds ago)
         if (threadIdx.x == 0 && n_loaded) L.s_base[r3] = sb_loaded + off_loaded;
         uint32_t total;
-        const uint32_t pre = block_exclusive_scan<BLOCK, uint32_t>(c, L.wtmp, &total);
+        uint32_t pre = block_exclusive_scan<BLOCK, uint32_t>(c, L.wtmp, &total, __ballot(multi != 0u) ? DUPS : 0u);
+        pre &= DUPS - 1u;
+        const bool dups = total >= DUPS;  // uniform: some key of the round has several matches
+        total &= DUPS - 1u;
         phase_tick<COLLECT>(tacc, tmark, PT_COUNT);
         if (n_loaded) flush(n_loaded, r3, wk, wp, wb);
         // the rows of the round before the last into the registers (stage[r3 + 1 mod 3])
@@ -827,31 +833,31 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         // took 0.29 ms in the direct join, now 0.16, and the probe of 9M x 24M with
         // four copies of each key (19.2M rows) 434 us, now 337.  The first values are
         // loaded while thread 0 waits for the reservation: 6001 x 20M 159 -> 149 us, 12M x
-        // 50M with every tuple matching 461 -> 428.
+        // 50M with every tuple matching 461 -> 428.  Waves with duplicate matches write in
+        // another form than waves without; a barrier only stands where the whole workgroup
+        // goes the same way (dups), and a round without any keeps its loads ahead of it (one
+        // barrier before a branch per wave, loads under that branch: 6001 x 20M 158 us, 12M x
+        // 50M 455 against 151 and 418 so).
         unsigned long long sd = 0;
         if (threadIdx.x == 0) sd = atomicAdd((unsigned long long*)out_count, (unsigned long long)total);
         // rows that fit from place w on (uniform)
         auto room = [&](uint64_t w) { return w >= out_cap ? 0u : (uint32_t)min<uint64_t>(out_cap - w, 4u * WAVE); };
-        if (__ballot(multi != 0u) == 0ull) {
-            // one row per matching key: key group by key group, so that the lanes of
-            // a store write consecutive rows (in lane order a lane's keys would lie
-            // up to PITEMS rows apart); the values of HALF groups in flight together
-            // (of all groups: spills)
-            constexpr int HALF = (PITEMS + 1) / 2;
-            uint32_t pv[HALF], bv[HALF];
-            auto load_values = [&](int h) {
+        // One row per matching key: key group by key group, so that the lanes of a
+        // store write consecutive rows (in lane order a lane's keys would lie up to
+        // PITEMS rows apart); the values of HALF groups in flight together (of all
+        // groups: spills).
+        constexpr int HALF = (PITEMS + 1) / 2;
+        uint32_t pv[HALF], bv[HALF];
+        auto load_values = [&](int h) {
 #pragma unroll
-                for (int u = 0; u < HALF; u++) {
-                    if (h + u >= PITEMS) continue;
-                    const bool hit = (hitmask >> (h + u)) & 1u;
-                    pv[u] = pvp[hit ? base + (uint32_t)(h + u) * BLOCK + threadIdx.x : 0u];
-                    bv[u] = bvp[L.hidx[qm[h + u] & 0xFFFFu]];
-                }
-            };
-            load_values(0);  // under way while thread 0 waits for the reservation
-            if (threadIdx.x == 0) L.s_direct = sd;
-            __syncthreads();
-            uint64_t w = uniform_u64(L.s_direct + pre);
+            for (int u = 0; u < HALF; u++) {
+                if (h + u >= PITEMS) continue;
+                const bool hit = (hitmask >> (h + u)) & 1u;
+                pv[u] = pvp[hit ? base + (uint32_t)(h + u) * BLOCK + threadIdx.x : 0u];
+                bv[u] = bvp[L.hidx[qm[h + u] & 0xFFFFu]];
+            }
+        };
+        auto write_single = [&](uint64_t w) {  // the values of the first HALF groups are loaded
 #pragma unroll
             for (int h = 0; h < PITEMS; h += HALF) {
                 if (h) load_values(h);
@@ -869,29 +875,41 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
                     w += (uint32_t)__popcll(m);
                 }
             }
+        };
+        if (!dups) {  // no key of the round has several matches (the same for all waves)
+            load_values(0);  // under way while thread 0 waits for the reservation
+            if (threadIdx.x == 0) L.s_direct = sd;
+            __syncthreads();
+            write_single(uniform_u64(L.s_direct + pre));
+            phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
+            continue;
+        }
+        if (threadIdx.x == 0) L.s_direct = sd;
+        __syncthreads();
+        uint64_t w = uniform_u64(L.s_direct + pre);
+        if (__ballot(multi != 0u) == 0ull) {  // this wave has none
+            load_values(0);
+            write_single(w);
         } else {
             // duplicate build keys: the wave's rows go through its share of the
             // round's stage (free: stage[r3] was last read a round ago), so the
             // values of all its rows are in flight instead of one per match of a lane
-            if (threadIdx.x == 0) L.s_direct = sd;
-            __syncthreads();
             constexpr uint32_t FIFO = STAGE / (BLOCK / WAVE);
             static_assert(FIFO == 2 * WAVE || FIFO == WAVE, "one or two rows per lane");
             const uint32_t lane = lane_id();
             uint32_t* fifo = &L.stage[r3][threadIdx.x / WAVE * FIFO];
-            uint64_t w = uniform_u64(L.s_direct + pre);
             uint32_t n = 0;  // rows in the wave's FIFO (uniform)
             auto drain = [&]() {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 constexpr int NF = FIFO / WAVE;
-                uint32_t k[NF], pv[NF], bv[NF];
+                uint32_t k[NF], fp[NF], fb[NF];
 #pragma unroll
                 for (int u = 0; u < NF; u++) {
                     const uint32_t j = min(lane + u * WAVE, n - 1u);
                     const uint32_t x = fifo[j];
                     k[u] = L.hkey[x >> 16];
-                    pv[u] = pvp[base + (x & 0xFFFFu)];
-                    bv[u] = bvp[L.hidx[x >> 16]];
+                    fp[u] = pvp[base + (x & 0xFFFFu)];
+                    fb[u] = bvp[L.hidx[x >> 16]];
                 }
                 const uint32_t nw = min(n, room(w));
 #pragma unroll
@@ -899,8 +917,8 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
                     const uint32_t j = lane + u * WAVE;
                     if (j < nw) {
                         (o_key + w)[j] = k[u];
-                        (o_rval + w)[j] = build_r ? bv[u] : pv[u];
-                        (o_sval + w)[j] = build_r ? pv[u] : bv[u];
+                        (o_rval + w)[j] = build_r ? fb[u] : fp[u];
+                        (o_sval + w)[j] = build_r ? fp[u] : fb[u];
                     }
                 }
                 w += n;
