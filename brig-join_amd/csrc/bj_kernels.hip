@@ -1038,16 +1038,40 @@ __global__ void k_direct_begin(uint64_t* __restrict__ ctr, int n_ctr, uint64_t* 
     for (uint64_t i = i0; i < nf; i += (uint64_t)gridDim.x * blockDim.x) filter[i] = 0ull;
 }
 
-// The filter of an unpartitioned R: one 64-bit atomic OR per key (cleared
-// before).  The same bits as k_bloom_build's.
-__global__ void k_direct_bloom(const uint32_t* __restrict__ rkey, uint32_t n, BloomGeom g,
-                               uint64_t* __restrict__ filter)
+// The filter of an unpartitioned R (cleared before); the same bits as k_bloom_build's.
+// Every workgroup gathers its keys' bits block by block in an LDS hash table, then ORs
+// each block into the filter with one 64-bit atomic: the chip does some 70 atomics on
+// one address per us, so that with an atomic per key equal keys, or a filter of few
+// blocks, set the pace (100K equal keys 1.14 ms, 2.5M 28.3 ms, 200K keys in 256 bits
+// 1.08 ms; so 7, 116 and 9 us).  Distinct keys are bound by the atomics either way: 2.5M
+// 97 -> 99 us, 200K 12 -> 13 (two or four keys per thread 16-19).
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_direct_bloom(const uint32_t* __restrict__ rkey, uint32_t n, BloomGeom g,
+                                                        uint64_t* __restrict__ filter)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const uint32_t k = rkey[i];
-        atomicOr((unsigned long long*)&filter[bloom_block(k, g)], (unsigned long long)bloom_mask(k, g.k));
+    constexpr uint32_t SLOTS = 2 * BLOCK, EMPTY = 0xFFFFFFFFu;  // at most half full
+    static_assert((SLOTS & (SLOTS - 1)) == 0, "slots are found by a mask");
+    __shared__ uint32_t blk[SLOTS];
+    __shared__ unsigned long long bits[SLOTS];
+    for (uint32_t i = threadIdx.x; i < SLOTS; i += BLOCK) {
+        blk[i] = EMPTY;
+        bits[i] = 0ull;
     }
+    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
+    const uint32_t k = rkey[min(i, n - 1u)];
+    __syncthreads();
+    if (i < n) {
+        const uint32_t b = (uint32_t)bloom_block(k, g);
+        uint32_t s = b & (SLOTS - 1);
+        for (;; s = (s + 1) & (SLOTS - 1)) {  // ends: there are more slots than keys
+            const uint32_t was = atomicCAS(&blk[s], EMPTY, b);
+            if (was == EMPTY || was == b) break;
+        }
+        atomicOr(&bits[s], (unsigned long long)bloom_mask(k, g.k));
+    }
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s < SLOTS; s += BLOCK)
+        if (blk[s] != EMPTY) atomicOr((unsigned long long*)&filter[blk[s]], bits[s]);
 }
 
 // Joins unpartitioned relations: the build side in C chunks of at most CAP
@@ -1420,8 +1444,10 @@ hipError_t launch_direct_begin(uint64_t* ctr, int n_ctr, uint64_t* filter, uint6
 hipError_t launch_direct_bloom(const uint32_t* rkey, uint64_t n, const BloomGeom& g, uint64_t* filter,
                                hipStream_t st)
 {
+    constexpr int B = 256;
     if (n == 0) return hipSuccess;
-    k_direct_bloom<<<ceil_div_i(n, 256), 256, 0, st>>>(rkey, (uint32_t)n, g, filter);
+    if (((uint64_t)g.wps << g.seg_bits) >= 0xFFFFFFFFull) return hipErrorInvalidValue;  // block numbers in 32 bits
+    k_direct_bloom<B><<<ceil_div_i(n, B), B, 0, st>>>(rkey, (uint32_t)n, g, filter);
     return hipGetLastError();
 }
 
