@@ -572,8 +572,6 @@ hipError_t tl_end(bj_ctx* c, int slot)
 
 float tl_ms(bj_ctx* c, int slot) { return ev_ms(c, c->tl_b[slot], c->tl_e[slot]); }
 
-float tl_span_ms(bj_ctx* c, int first, int last) { return ev_ms(c, c->tl_b[first], c->tl_e[last]); }
-
 static int enqueue_bloom_build(bj_ctx* c, const Plan& pl)
 {
     BJ_HIP(tl_begin(c, BJ_K_BF_BUILD));
@@ -590,7 +588,7 @@ int enqueue_r(bj_ctx* c, const Plan& pl, const uint32_t* r_key, const uint32_t* 
                             P<uint32_t>(c->r_val), c->r_key.bytes / 4, P<uint64_t>(c->r_start), BJ_K_HIST_R, false,
                             first_of_join)))
         return rc;
-    return pl.bf ? enqueue_bloom_build(c, pl) : BJ_OK;
+    return pl.bf && !pl.filtered ? enqueue_bloom_build(c, pl) : BJ_OK;
 }
 
 // The filter after S's first pass (c->tmp or, merged, c->tmp2): its survivors,
@@ -696,11 +694,13 @@ int enqueue_s(bj_ctx* c, const Plan& pl, const RSide& R, const uint32_t* s_key, 
     const uint64_t* n_dev = nullptr;
     if (pl.bf) {
         // the reference's order: filter S, then partition the survivors
-        BJ_HIP(tl_begin(c, BJ_K_BF_FILTER));
-        BJ_HIP(launch_bloom_prefilter(s_key, s_val, pl.ns, R.filter, pl.geom, P<uint32_t>(c->sp_key),
-                                      P<uint32_t>(c->sp_val), c->sp_key.bytes / 4, ctr + CTR_SPRIME, ctr + CTR_ERR,
-                                      c->num_cu, st));
-        BJ_HIP(tl_end(c, BJ_K_BF_FILTER));
+        if (!pl.filtered) {
+            BJ_HIP(tl_begin(c, BJ_K_BF_FILTER));
+            BJ_HIP(launch_bloom_prefilter(s_key, s_val, pl.ns, R.filter, pl.geom, P<uint32_t>(c->sp_key),
+                                          P<uint32_t>(c->sp_val), c->sp_key.bytes / 4, ctr + CTR_SPRIME,
+                                          ctr + CTR_ERR, c->num_cu, st));
+            BJ_HIP(tl_end(c, BJ_K_BF_FILTER));
+        }
         s_key = P<uint32_t>(c->sp_key);
         s_val = P<uint32_t>(c->sp_val);
         n_dev = ctr + CTR_SPRIME;
@@ -758,8 +758,8 @@ static int enqueue_direct(bj_ctx* c, const Plan& pl, const uint32_t* r_key, cons
         ns_dev = ctr + CTR_SPRIME;
     }
     BJ_HIP(tl_begin(c, BJ_K_PROBE));
-    BJ_HIP(launch_join_direct(r_key, r_val, pl.nr, s_key, s_val, pl.ns, ns_dev, ctr + CTR_OUT, cap, o_key, o_rval,
-                              o_sval, c->num_cu, st));
+    BJ_HIP(launch_join_direct(r_key, r_val, pl.nr, s_key, s_val, pl.ns, ns_dev, pl.bits, ctr + CTR_LONG_RUN,
+                              ctr + CTR_OUT, cap, o_key, o_rval, o_sval, c->num_cu, st));
     BJ_HIP(tl_end(c, BJ_K_PROBE));
     return BJ_OK;
 }
@@ -1280,19 +1280,36 @@ static int join_s_chunks(bj_ctx* c, const bj_params* p, const Plan& full, int ch
 // The join of device-resident inputs in one pass, into the row arrays o_*
 // (capacity pl.cap): the workspace must already be in place.  h2d_ms < 0: the
 // host copies before it were bracketed by EV_H2D0 / EV_H2D1.
-int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uint32_t* r_key,
+int join_device(bj_ctx* c, const Plan& plan, bool timing, double h2d_ms, const uint32_t* r_key,
                 const uint32_t* r_val, const uint32_t* s_key, const uint32_t* s_val, uint32_t* o_key,
                 uint32_t* o_rval, uint32_t* o_sval, bj_result* out)
 {
     int rc;
+    Plan pl = plan;
     hipStream_t st = c->stream;
     uint64_t* ctr = P<uint64_t>(c->counters);
-    // slots without kernels (no filter) keep no events and read as 0 ms
-    int first_slot = BJ_K_HIST_R;
+    auto read_counters = [&]() -> int {
+        BJ_HIP(hipMemcpyAsync(c->h_counters, ctr, CTR_N * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+        BJ_HIP(hipStreamSynchronize(st));
+        return BJ_OK;
+    };
+    int first = -1;  // the event before the first kernel
     if (pl.direct) {
-        first_slot = pl.bf ? BJ_K_BF_BUILD : BJ_K_PROBE;
         if ((rc = enqueue_direct(c, pl, r_key, r_val, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
-    } else {
+        if ((rc = read_counters())) return rc;
+        first = c->tl_b[pl.bf ? BJ_K_BF_BUILD : BJ_K_PROBE];
+        if (c->h_counters[CTR_LONG_RUN]) {
+            // a hot key on the build side: by partitions after all, with the filter and S'
+            // that are there.  The rows written so far are written again.
+            pl.direct = false;
+            pl.filtered = pl.bf;
+            pl.merge = !g_no_alloc && choose_merge(pl);  // (the caller's scratch holds one set of buffers)
+            if (!g_no_alloc && (rc = ensure_workspace(c, pl))) return rc;
+            if (pl.filtered) BJ_HIP(launch_zero_u64(ctr + CTR_OUT, CTR_ITEMS - CTR_OUT + 1, st));
+            c->tl_open = false;
+        }
+    }
+    if (!pl.direct) {
         // the first launch, R's histogram, clears the counters
         if ((rc = probe_timers_begin(c, pl))) return rc;
         const RSide R{P<uint32_t>(c->r_key), P<uint32_t>(c->r_val), P<uint64_t>(c->r_start), P<uint64_t>(c->filter)};
@@ -1304,13 +1321,12 @@ int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uin
                                          P<uint64_t>(c->s_start), s_cnt, o_key, o_rval, o_sval, pl.cap, planned)))
                 return rc;
         } else {
-            if ((rc = enqueue_r(c, pl, r_key, r_val, true))) return rc;
+            if ((rc = enqueue_r(c, pl, r_key, r_val, !pl.filtered))) return rc;
             if ((rc = enqueue_s_probe(c, pl, R, s_key, s_val, o_key, o_rval, o_sval, pl.cap))) return rc;
         }
+        if ((rc = read_counters())) return rc;
+        if (first < 0) first = c->tl_b[BJ_K_HIST_R];
     }
-
-    BJ_HIP(hipMemcpyAsync(c->h_counters, ctr, CTR_N * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-    BJ_HIP(hipStreamSynchronize(st));
 
     const uint64_t* h = c->h_counters;
     if (h[CTR_ERR]) return fail(BJ_ERR_INTERNAL, "device check flags " + std::to_string(h[CTR_ERR]));
@@ -1331,8 +1347,8 @@ int join_device(bj_ctx* c, const Plan& pl, bool timing, double h2d_ms, const uin
                 k[i] -= k[i] * of_s;
             }
         }
-        fill_phases(out, h2d_ms < 0 ? ev_ms(c, EV_H2D0, EV_H2D1) : h2d_ms,
-                    tl_span_ms(c, first_slot, BJ_K_PROBE));
+        // (slots without kernels keep no events and read as 0 ms)
+        fill_phases(out, h2d_ms < 0 ? ev_ms(c, EV_H2D0, EV_H2D1) : h2d_ms, ev_ms(c, first, c->tl_e[BJ_K_PROBE]));
     }
     return probe_timers_end(c, pl, out);
 }

@@ -85,8 +85,9 @@ int ceil_log2(uint64_t n);
 // CTR_XCD .. CTR_XCD + 7: tile counters of the filter kernel, one per XCD;
 // CTR_ACC_SPRIME / CTR_ACC_ITEMS: |S'| and vlsplit items summed over the chunks of S
 // CTR_POOL: tuples in the pool of S' (S in chunks with one probe)
+// CTR_LONG_RUN: the direct join (which has no work queue) left a table with a long run
 enum { CTR_SPRIME = 0, CTR_OUT, CTR_WORK, CTR_ITEMS, CTR_ERR, CTR_ACC_SPRIME, CTR_ACC_ITEMS, CTR_POOL, CTR_XCD = 8,
-       CTR_N = 16 };
+       CTR_LONG_RUN = CTR_WORK, CTR_N = 16 };
 
 // Events EV_H2D0/1 bracket the host copies; EV_KB .. are a pool for the
 // kernel-slot boundaries (tl_begin / tl_end), EV_N at creation, grown when a
@@ -104,6 +105,7 @@ struct Plan {
     bool solo_r = false, solo_s = false; // one scatter workgroup per CU (large relations)
     bool direct = false;                 // joined without a partition (small build side)
     bool merge = false;                  // R and S partitioned by the same launches
+    bool filtered = false;               // filter and S' are in place (bf_stage 1)
     int tile = 8192;
     uint32_t slice = 65536;
     uint32_t max_slices = 16;
@@ -218,6 +220,5 @@ void tl_reset(bj_ctx* c, bool timing);
 hipError_t tl_begin(bj_ctx* c, int slot);
 hipError_t tl_end(bj_ctx* c, int slot);
 float tl_ms(bj_ctx* c, int slot);
-float tl_span_ms(bj_ctx* c, int first, int last);
 
 }  // namespace bj

@@ -126,14 +126,16 @@ hipError_t launch_probe(int tile, uint64_t probe_mean, const uint32_t* rk, const
 // Direct join of unpartitioned relations (small build sides): begin clears the
 // join's counters and its filter (64-bit blocks), bloom fills the filter, join
 // emits the rows.
-// ns_dev (nullable): device-side length of S, at most ns.
+// ns_dev (nullable): device-side length of S, at most ns.  *long_run is set, and the
+// rows are not all there, when a table has a run of equal keys that makes the join by
+// partitions (of bits radix bits) the faster one.
 hipError_t launch_direct_begin(uint64_t* ctr, int n_ctr, uint64_t* filter, uint64_t blocks, hipStream_t st);
 hipError_t launch_direct_bloom(const uint32_t* rkey, uint64_t n, const BloomGeom& g, uint64_t* filter,
                                hipStream_t st);
 hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t nr, const uint32_t* sk,
-                              const uint32_t* sv, uint64_t ns, const uint64_t* ns_dev, uint64_t* out_count,
-                              uint64_t out_cap, uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, int num_cu,
-                              hipStream_t st);
+                              const uint32_t* sv, uint64_t ns, const uint64_t* ns_dev, int bits,
+                              uint64_t* long_run, uint64_t* out_count, uint64_t out_cap, uint32_t* o_key,
+                              uint32_t* o_rval, uint32_t* o_sval, int num_cu, hipStream_t st);
 // Workgroups of a probe launch (persistent: a fixed number per CU).  With
 // timers, every workgroup adds its phase times (ticks, PT_* order of bj_tiles.h,
 // PT_N = 5 per workgroup) to its slots; the caller clears them.

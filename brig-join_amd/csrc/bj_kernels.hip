@@ -1085,18 +1085,35 @@ __global__ __launch_bounds__(BLOCK) void k_direct_bloom(const uint32_t* __restri
 // device-side length of S (S' after the filter).  Workgroups of one slice run
 // on one XCD (slices are dealt in multiples of 8), so its keys come from that
 // XCD's L2 after the first chunk.
+// Every probe key of a bucket walks its whole run, so a key that fills a good part of
+// every chunk costs far more than here is saved (300K x 200K with 90% of S equal: 1.8
+// ms), where the partitioned join builds the hot sub-bucket's table from the other side.
+// A workgroup whose table has a longer run than it may have sets *long_run and leaves;
+// the host then joins by partitions (of bits radix bits).  With one chunk (C = 1) the
+// partitioned join would build the same table.  Otherwise a run may be DIRECT_MAX_RUN
+// long, or as long as a key that has it in every chunk leaves its sub-bucket of the
+// partitioned join smaller on this side than on the other, so that a C times longer
+// run would be walked there.  Both sides of the line, direct against partitioned: 200K x
+// 300K, 256 copies in a chunk 109 / 76 us (some 40 us more after the attempt), 512 138 /
+// 76, 1024 281 / 76; 300K x 100K 512 119 / 969, 1024 270 / 75; 100K x 1M 1024 398 / 660, 2M x
+// 50K 4096 1582 / 2192.
+constexpr uint32_t DIRECT_MAX_RUN = 320;
+
 template <int BLOCK, int CAP, int PITEMS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_waves(BLOCK, CAP), 8))) void k_join_direct(
     const uint32_t* __restrict__ rk, const uint32_t* __restrict__ rv, uint32_t nr,
     const uint32_t* __restrict__ sk, const uint32_t* __restrict__ sv, uint32_t ns_host,
-    const uint64_t* __restrict__ ns_dev, bool build_r, uint32_t grain, uint64_t* __restrict__ out_count,
-    uint64_t out_cap, uint32_t* __restrict__ o_key, uint32_t* __restrict__ o_rval, uint32_t* __restrict__ o_sval)
+    const uint64_t* __restrict__ ns_dev, bool build_r, uint32_t grain, int bits, uint64_t* __restrict__ long_run,
+    uint64_t* __restrict__ out_count, uint64_t out_cap, uint32_t* __restrict__ o_key, uint32_t* __restrict__ o_rval, uint32_t* __restrict__ o_sval)
 {
     __shared__ ProbeLds<BLOCK, CAP> L;
     const uint32_t ns = ns_dev ? (uint32_t)min(*ns_dev, (uint64_t)ns_host) : ns_host;
     const uint32_t nb = build_r ? nr : ns, np = build_r ? ns : nr;
     if (nb == 0 || np == 0) return;
     const uint32_t C = (nb + CAP - 1) / CAP;
+    // longest run that a table may have
+    const uint32_t per_b = nb >> bits, per_p = np >> bits;
+    const uint32_t max_run = C == 1 ? 0xFFFFFFFFu : max(DIRECT_MAX_RUN, per_p > per_b ? (per_p - per_b) / C : 0u);
     const uint32_t cper = (nb + C - 1) / C;
     uint32_t S = max(1u, min(gridDim.x / C, (np + grain - 1) / grain));
     if (S > 8) S &= ~7u;
@@ -1107,9 +1124,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_wav
         const uint32_t b0 = min(c * cper, nb), p0 = (uint32_t)min((uint64_t)sl * sper, (uint64_t)np);
         const int bn = (int)min(cper, nb - b0);
         const uint32_t pn = min(sper, np - p0);
-        probe_item<BLOCK, CAP, PITEMS>(L, (build_r ? rk : sk) + b0, (build_r ? rv : sv) + b0, bn,
-                                       (build_r ? sk : rk) + p0, (build_r ? sv : rv) + p0, pn, build_r, 0,
-                                       out_count, out_cap, o_key, o_rval, o_sval);
+        if (probe_item<BLOCK, CAP, PITEMS, false, true>(
+                L, (build_r ? rk : sk) + b0, (build_r ? rv : sv) + b0, bn, (build_r ? sk : rk) + p0,
+                (build_r ? sv : rv) + p0, pn, build_r, 0, out_count, out_cap, o_key, o_rval, o_sval, nullptr, nullptr,
+                max_run)) {
+            if (threadIdx.x == 0) *long_run = 1ull;
+            return;
+        }
         __syncthreads();  // the table is rebuilt by the next item
     }
 }
@@ -1452,9 +1473,9 @@ hipError_t launch_direct_bloom(const uint32_t* rkey, uint64_t n, const BloomGeom
 }
 
 hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t nr, const uint32_t* sk,
-                              const uint32_t* sv, uint64_t ns, const uint64_t* ns_dev, uint64_t* out_count,
-                              uint64_t out_cap, uint32_t* o_key, uint32_t* o_rval, uint32_t* o_sval, int num_cu,
-                              hipStream_t st)
+                              const uint32_t* sv, uint64_t ns, const uint64_t* ns_dev, int bits,
+                              uint64_t* long_run, uint64_t* out_count, uint64_t out_cap, uint32_t* o_key,
+                              uint32_t* o_rval, uint32_t* o_sval, int num_cu, hipStream_t st)
 {
     constexpr int CAP = 8192, B = 512;
     if (nr == 0 || ns == 0) return hipSuccess;
@@ -1472,12 +1493,12 @@ hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t n
     const int grid = (int)std::min<uint64_t>(wgs, C * std::max<uint64_t>(1, (np + grain - 1) / grain));
     if (small)
         k_join_direct<B, CAP, SMALL_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
-                                                               build_r, grain, out_count, out_cap, o_key, o_rval,
-                                                               o_sval);
+                                                               build_r, grain, bits, long_run, out_count, out_cap,
+                                                               o_key, o_rval, o_sval);
     else
         k_join_direct<B, CAP, DIRECT_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
-                                                               build_r, grain, out_count, out_cap, o_key, o_rval,
-                                                               o_sval);
+                                                               build_r, grain, bits, long_run, out_count, out_cap,
+                                                               o_key, o_rval, o_sval);
     return hipGetLastError();
 }
 

@@ -557,15 +557,17 @@ __device__ __forceinline__ void phase_tick(uint64_t* acc, uint64_t* mark, int ph
 
 // COLLECT: thread 0 adds the item's phase times to tacc[PT_CLEAR..PT_WRITE]
 // (tmark: the time the item started; left at the item's end).
-template <int BLOCK, int CAP, int PITEMS, bool COLLECT = false>
-__device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32_t* __restrict__ bkp,
+// WATCH: returns true, with nothing probed, when a bucket holds more than max_run
+// build tuples (the same for all threads); false otherwise.
+template <int BLOCK, int CAP, int PITEMS, bool COLLECT = false, bool WATCH = false>
+__device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32_t* __restrict__ bkp,
                                            const uint32_t* __restrict__ bvp, int bn,
                                            const uint32_t* __restrict__ pkp, const uint32_t* __restrict__ pvp,
                                            uint32_t pn, bool build_r, int bits,
                                            uint64_t* __restrict__ out_count, uint64_t out_cap,
                                            uint32_t* __restrict__ o_key, uint32_t* __restrict__ o_rval,
                                            uint32_t* __restrict__ o_sval, uint64_t* tacc = nullptr,
-                                           uint64_t* tmark = nullptr)
+                                           uint64_t* tmark = nullptr, uint32_t max_run = 0)
 {
     constexpr int ROUND = BLOCK * PITEMS;
     constexpr int BPT = CAP / BLOCK;  // build tuples per thread
@@ -574,7 +576,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     constexpr uint32_t DUPS = 1u << 27;
     static_assert((uint64_t)ROUND * CAP < DUPS && BLOCK / WAVE <= 16, "row count and waves' marks in one word");
     static_assert(CAP % BLOCK == 0 && CAP <= 32768, "bucket and rank pack into 16 bits each");
-    if (pn == 0) return;  // an empty slice (uniform)
+    if (pn == 0) return false;  // an empty slice (uniform)
 
     // table geometry: 2^tb buckets, about two per build tuple when the probe
     // side is at least as long as the build side (shorter runs per probe key:
@@ -598,6 +600,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     } else if (threadIdx.x < nbk) {
         cnt[threadIdx.x] = 0u;
     }
+    if (WATCH && threadIdx.x == 0) L.s_direct = 0ull;  // here: whether a bucket is too long
     __syncthreads();
     phase_tick<COLLECT>(tacc, tmark, PT_CLEAR);
     // build: rank each tuple in its bucket, scan the counts, place;
@@ -614,10 +617,13 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         btr[u] = 0;
         if (i < bn) {
             const uint32_t t = bucket(bkey[u]);
-            btr[u] = (atomicAdd(&cnt[t], 1u) << 16) | t;
+            const uint32_t r = atomicAdd(&cnt[t], 1u);
+            btr[u] = (r << 16) | t;
+            if (WATCH && r == max_run) L.s_direct = 1ull;
         }
     }
     __syncthreads();
+    if (WATCH && L.s_direct) return true;  // uniform
     {
         // exclusive scan of the counts into the bucket starts; a thread's run
         // of counts is a power of two, read and written four at a time from 4
@@ -978,6 +984,7 @@ __device__ __forceinline__ void probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         phase_tick<COLLECT>(tacc, tmark, PT_WRITE);
     }
     // the caller synchronises before the next item rebuilds the table
+    return false;
 }
 
 // Work-item split of one sub-bucket (vlsplit).  A sub-bucket whose build side
