@@ -374,9 +374,11 @@ static PartSide make_side(bj_ctx* c, const Plan& pl, int p1, const uint32_t* key
     s.G = G;
     s.bits = pl.bits;
     s.p1 = p1;
-    // second-pass workgroups: four tiles each, up to about 1024 in total (3M x
-    // 4.5M's second pass: 58 us with 1024 per side, 33 so, 39 with eight tiles each)
-    s.W2 = std::min(std::max(1, std::min(64, (int)std::min<uint64_t>(1024, (n + CHUNK_TUPLES - 1) / CHUNK_TUPLES) >> p1)), G);
+    // second-pass workgroups: up to about 1024 in total, W2 for each bucket; where four
+    // tiles for each give fewer, so many in total, shared by the buckets' sizes
+    s.W2 = std::min(std::max(1, std::min(64, 1024 >> p1)), G);
+    const uint64_t by_tuples = n / CHUNK_TUPLES + (1ull << p1);
+    s.shared2 = by_tuples < (uint64_t)s.W2 << p1 ? (int)by_tuples : 0;
     // chunk groups of the column sums: the second pass's groups, else up to 8
     s.W = p1 < pl.bits && !l1_only ? s.W2 : std::min(8, G);
     s.part = P<uint32_t>(second ? c->part2 : c->part);

@@ -42,6 +42,7 @@ struct PartSide {
     int G;                      // chunks (histogram and first-pass workgroups)
     int bits, p1;               // radix bits, and those of the first pass
     int W, W2;                  // chunk groups of the column sums, second-pass workgroups per bucket (W = W2)
+    int shared2;                // not 0: so many in all (above 2^p1), shared by the buckets' sizes, at most W2 each
     uint32_t* part;             // [G][2^bits] chunk histograms
     uint32_t* l1h;              // [G][2^p1] first-level counts (p1 < bits)
     uint32_t* l1rel;            // [G][2^p1] first-level counts of the chunks before

@@ -497,10 +497,10 @@ __global__ __launch_bounds__(BLOCK) void k_plan(PlanArgs A)
 //       bucket = h >> (32 - p1); cur[b] = the bucket's start (a scan of l1tot) +
 //       l1rel[g][b].  Workgroup 0 meanwhile turns the bin totals into the
 //       sub-bucket starts, which only later launches read.
-//   pass 2 (bits - p1 bits): workgroup (b1, w) owns the pass-1 output of bucket
-//       b1 written by pass-1 groups [w*G/W2, (w+1)*G/W2); bucket = (h >> (32 -
-//       bits)) & (2^(bits-p1) - 1); cur[b] = start[sb] + sum_{v < w} colsum[v][sb]
-//       with sb = (b1 << (bits-p1)) + b.
+//   pass 2 (bits - p1 bits): workgroup (b1, w) of the bucket's A owns the pass-1 output
+//       of bucket b1 written by pass-1 groups [w*G/A, (w+1)*G/A); bucket = (h >> (32 -
+//       bits)) & (2^(bits-p1) - 1); cur[b] = start[sb] + what the chunks before hold of
+//       sb = (b1 << (bits-p1)) + b.  A follows the bucket's size (second_share).
 // IPAIR / OPAIR: whole tuples in one array (TupleIn / TupleOut) on that side:
 // pass 1 writes them unless it is the only pass, pass 2 (IPAIR) reads them.
 // Writes are bounds-checked against the capacity and flag err on violation.
@@ -508,6 +508,46 @@ __global__ __launch_bounds__(BLOCK) void k_plan(PlanArgs A)
 // Occupancy targets: two 1024-thread workgroups per CU for the 4096-tuple tile,
 // one for the 8192-tuple tile (launched one per CU), three 512-thread ones.
 constexpr int sc_min_waves(int block, int items) { return block == 1024 ? (items == 4 ? 8 : 4) : 6; }
+
+// Workgroups launched for a side's second pass.
+static int second_wgs(const PartSide& s) { return s.shared2 ? s.shared2 : s.W2 << s.p1; }
+
+// Bucket b1 of workgroup x of a side's second pass, its place w among the bucket's A
+// workgroups; false: there is none.  With shared2 a bucket of nb tuples takes ceil(nb /
+// per), at least one and at most W2, per being such that the sum stays within shared2;
+// every wave finds its place by itself, lane l adding up 2^p1 / 64 buckets.
+// W2 workgroups each would be many for the work below some 16M tuples (3M x 4.5M: 58 us
+// with 1024 per side, 35 so), but a fixed smaller number leaves a hot key's bucket to those
+// few (eight there: half of S equal 365 us, so 110).
+__device__ __forceinline__ bool second_place(const PartSide& s, uint32_t x, int& b1, int& w, int& A)
+{
+    A = s.W2;
+    b1 = (int)x / s.W2;
+    w = (int)x % s.W2;
+    if (s.shared2 == 0) return true;
+    const int P1 = 1 << s.p1, b2 = s.bits - s.p1;
+    const uint32_t room = (uint32_t)(s.shared2 - P1);
+    const uint32_t per = max(1u, (uint32_t)((side_len(s) + room - 1u) / room));
+    auto share = [&](int b) {
+        const uint32_t nb = (uint32_t)(s.start[(uint64_t)(b + 1) << b2] - s.start[(uint64_t)b << b2]);
+        return min((uint32_t)s.W2, max(1u, (nb + per - 1u) / per));
+    };
+    const int np = (P1 + WAVE - 1) / WAVE, q0 = (int)lane_id() * np;
+    uint32_t sum = 0;
+    for (int j = 0; j < np; j++)
+        if (q0 + j < P1) sum += share(q0 + j);
+    const uint32_t inc = wave_inclusive_scan<uint32_t>(sum);
+    if (x >= __builtin_amdgcn_readlane(inc, WAVE - 1)) return false;
+    const int l = __popcll(__ballot(inc <= x));  // the lane whose buckets x falls into
+    uint32_t at = l ? __builtin_amdgcn_readlane(inc, l - 1) : 0u;
+    for (b1 = l * np;; b1++) {  // ends: x lies below the sum of the lane's shares
+        A = (int)share(b1);
+        if (x < at + (uint32_t)A) break;
+        at += (uint32_t)A;
+    }
+    w = (int)(x - at);
+    return true;
+}
 
 template <int BLOCK, int ITEMS, bool IPAIR, bool OPAIR>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sc_min_waves(BLOCK, ITEMS), 8))) void k_scatter(
@@ -556,19 +596,29 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sc_min_wa
             }
         in = {s.key, s.val};
     } else {
-        const int b1 = (int)x / s.W2, w = (int)x % s.W2;
-        const int g0 = (int)(((int64_t)w * s.G) / s.W2), g1 = (int)(((int64_t)(w + 1) * s.G) / s.W2);
+        int b1, w, A;
+        if (!second_place(s, x, b1, w, A)) return;
+        const int g0 = (int)(((int64_t)w * s.G) / A), g1 = (int)(((int64_t)(w + 1) * s.G) / A);
         const uint64_t b_lo = s.start[(uint64_t)b1 << b2], b_hi = s.start[(uint64_t)(b1 + 1) << b2];
         lo = (g0 < s.G) ? b_lo + s.l1rel[(size_t)g0 * P1 + b1] : b_hi;
         hi = (g1 < s.G) ? b_lo + s.l1rel[(size_t)g1 * P1 + b1] : b_hi;
-        // cursor of sub-bucket sb: its start plus what the earlier groups hold of it
+        // cursor of sub-bucket sb: its start plus what the earlier chunks hold of it, those
+        // of the column sums' groups before chunk g0's and the others of that group
+        const int v0 = (int)(((int64_t)(g0 + 1) * s.W2 - 1) / s.G), gs = (int)(((int64_t)v0 * s.G) / s.W2);
+        // (2^b2 threads take every K-th row of them, and the next 2^b2 the rows beside)
         const uint64_t nbins = 1ull << s.bits;
-        for (int b = threadIdx.x; b < nbk; b += BLOCK) {
-            const uint64_t sb = ((uint64_t)b1 << b2) + b;
-            uint64_t cur = s.start[sb];
-#pragma unroll 8
-            for (int v = 0; v < w; v++) cur += s.colsum[(size_t)v * nbins + sb];
-            L.cur[b] = cur;
+        for (int b = threadIdx.x; b < nbk; b += BLOCK) L.cur[b] = s.start[((uint64_t)b1 << b2) + b];
+        __syncthreads();
+        const int K = max(1, BLOCK >> b2), k = (int)threadIdx.x >> b2;
+        for (int b = threadIdx.x & (nbk - 1); b < nbk; b += BLOCK) {
+            const uint32_t* row = s.colsum + ((size_t)b1 << b2) + b;
+            uint32_t sum = 0;
+#pragma unroll 4
+            for (int v = k; v < v0; v += K) sum += row[(size_t)v * nbins];
+            row = s.part + ((size_t)b1 << b2) + b;
+#pragma unroll 4
+            for (int g = gs + k; g < g0; g += K) sum += row[(size_t)g * nbins];
+            if (sum) atomicAdd((unsigned long long*)&L.cur[b], (unsigned long long)sum);
         }
         in = {(const Tuple*)s.tmp};
     }
@@ -1325,7 +1375,7 @@ static hipError_t scatter_pass(const PartSide* sides, int n, const PlanArgs& pla
 {
     int grid;
     const Sides S = sides_of(
-        sides, n, [](const PartSide& s) { return IPAIR ? (1 << s.p1) * s.W2 : s.G + 1; }, grid);
+        sides, n, [](const PartSide& s) { return IPAIR ? second_wgs(s) : s.G + 1; }, grid);
     if (IPAIR && plan.items) grid++;
     size_t lds = 0, lds_big = 0;
     for (int i = 0; i < n; i++) {
