@@ -1135,7 +1135,7 @@ __global__ __launch_bounds__(BLOCK) void k_direct_bloom(const uint32_t* __restri
 // device-side length of S (S' after the filter).  Workgroups of one slice run
 // on one XCD (slices are dealt in multiples of 8), so its keys come from that
 // XCD's L2 after the first chunk.
-// Every probe key of a bucket walks its whole run, so a key that fills a good part of
+// WATCH (build sides of several chunks): every probe key of a bucket walks its whole run, so a key that fills a good part of
 // every chunk costs far more than here is saved (300K x 200K with 90% of S equal: 1.8
 // ms), where the partitioned join builds the hot sub-bucket's table from the other side.
 // A workgroup whose table has a longer run than it may have sets *long_run and leaves;
@@ -1149,7 +1149,7 @@ __global__ __launch_bounds__(BLOCK) void k_direct_bloom(const uint32_t* __restri
 // 50K 4096 1582 / 2192.
 constexpr uint32_t DIRECT_MAX_RUN = 320;
 
-template <int BLOCK, int CAP, int PITEMS>
+template <int BLOCK, int CAP, int PITEMS, bool WATCH>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_waves(BLOCK, CAP), 8))) void k_join_direct(
     const uint32_t* __restrict__ rk, const uint32_t* __restrict__ rv, uint32_t nr,
     const uint32_t* __restrict__ sk, const uint32_t* __restrict__ sv, uint32_t ns_host,
@@ -1174,7 +1174,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_wav
         const uint32_t b0 = min(c * cper, nb), p0 = (uint32_t)min((uint64_t)sl * sper, (uint64_t)np);
         const int bn = (int)min(cper, nb - b0);
         const uint32_t pn = min(sper, np - p0);
-        if (probe_item<BLOCK, CAP, PITEMS, false, true>(
+        if (probe_item<BLOCK, CAP, PITEMS, false, WATCH>(
                 L, (build_r ? rk : sk) + b0, (build_r ? rv : sv) + b0, bn, (build_r ? sk : rk) + p0,
                 (build_r ? sv : rv) + p0, pn, build_r, 0, out_count, out_cap, o_key, o_rval, o_sval, nullptr, nullptr,
                 max_run)) {
@@ -1541,14 +1541,14 @@ hipError_t launch_join_direct(const uint32_t* rk, const uint32_t* rv, uint64_t n
     const bool small = C * small_slices <= wgs;
     const uint32_t grain = B * (small ? SMALL_ITEMS : DIRECT_ITEMS);
     const int grid = (int)std::min<uint64_t>(wgs, C * std::max<uint64_t>(1, (np + grain - 1) / grain));
-    if (small)
-        k_join_direct<B, CAP, SMALL_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
-                                                               build_r, grain, bits, long_run, out_count, out_cap,
-                                                               o_key, o_rval, o_sval);
-    else
-        k_join_direct<B, CAP, DIRECT_ITEMS><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev,
-                                                               build_r, grain, bits, long_run, out_count, out_cap,
-                                                               o_key, o_rval, o_sval);
+#define BJ_DIRECT(I, W)                                                                                          \
+    k_join_direct<B, CAP, I, W><<<grid, B, 0, st>>>(rk, rv, (uint32_t)nr, sk, sv, (uint32_t)ns, ns_dev, build_r, grain, \
+                                                    bits, long_run, out_count, out_cap, o_key, o_rval, o_sval)
+    if (small && C > 1) BJ_DIRECT(SMALL_ITEMS, true);
+    else if (small) BJ_DIRECT(SMALL_ITEMS, false);
+    else if (C > 1) BJ_DIRECT(DIRECT_ITEMS, true);
+    else BJ_DIRECT(DIRECT_ITEMS, false);
+#undef BJ_DIRECT
     return hipGetLastError();
 }
 
