@@ -346,16 +346,20 @@ int make_plan(const bj_params& p, Plan& pl)
     pl.solo_s = pl.ns >= SOLO_TUPLES;
     if (const int rc = row_capacity(std::max(pl.nr, pl.ns), p.answer_scale, pl.cap)) return rc;
     // few sub-buckets: their probe sides are cut finer, so that there is an item for
-    // each of the PROBE_ITEMS_MIN workgroups the chip runs at once
+    // each of the PROBE_ITEMS_MIN workgroups the chip runs at once.  Where the build side
+    // makes items enough by its many chunks the slices stay few, and the items within
+    // what 16 slices of both sides' chunks would be.
+    const uint64_t build_chunks = std::min(pl.nr, pl.ns) / pl.tile + (1ull << total);
+    const uint64_t most_items = pl.max_slices * ((pl.nr + pl.ns) / pl.tile + (1ull << total));
     if ((1u << total) < PROBE_ITEMS_MIN) {
         const uint32_t per = PROBE_ITEMS_MIN >> total;
-        pl.max_slices = std::max(pl.max_slices, per);
+        pl.max_slices = std::max(pl.max_slices, (uint32_t)std::min<uint64_t>(per, most_items / build_chunks));
         const uint64_t np = std::max(pl.nr, pl.ns) >> total;
         pl.slice = (uint32_t)std::min<uint64_t>(pl.slice, std::max<uint64_t>(MIN_SLICE, (np + per - 1) / per));
     }
     // a sub-bucket larger than a tile on its build side builds from its smaller
     // side: sum of ceil(nb / tile) <= min(nr, ns) / tile + 2^bits
-    pl.item_cap = (uint64_t)pl.max_slices * (std::min(pl.nr, pl.ns) / pl.tile + (1ull << total)) + 16;
+    pl.item_cap = (uint64_t)pl.max_slices * build_chunks + 16;
     return BJ_OK;
 }
 
@@ -509,6 +513,17 @@ int ensure_workspace(bj_ctx* c, const Plan& pl, uint64_t* total_bytes)
     if (rc) return rc;
     if (total_bytes) *total_bytes = total;
     return BJ_OK;
+}
+
+// ensure_workspace, without S's own set of partition buffers where the device memory
+// does not hold both.
+static int ensure_join_workspace(bj_ctx* c, Plan& pl)
+{
+    const int rc = ensure_workspace(c, pl);
+    if (rc != BJ_ERR_NOMEM || !pl.merge) return rc;
+    for (DevBuf* b : {&c->part2, &c->totals2, &c->l1h2, &c->l1off2, &c->colsum2, &c->tmp2}) release(*b);
+    pl.merge = false;
+    return ensure_workspace(c, pl);
 }
 
 float ev_ms(bj_ctx* c, int a, int b)
@@ -1306,7 +1321,7 @@ int join_device(bj_ctx* c, const Plan& plan, bool timing, double h2d_ms, const u
             pl.direct = false;
             pl.filtered = pl.bf;
             pl.merge = !g_no_alloc && choose_merge(pl);  // (the caller's scratch holds one set of buffers)
-            if (!g_no_alloc && (rc = ensure_workspace(c, pl))) return rc;
+            if (!g_no_alloc && (rc = ensure_join_workspace(c, pl))) return rc;
             if (pl.filtered) BJ_HIP(launch_zero_u64(ctr + CTR_OUT, CTR_ITEMS - CTR_OUT + 1, st));
             c->tl_open = false;
         }
@@ -1376,14 +1391,7 @@ static int join_once(bj_ctx* c, const bj_params* p, const uint32_t* r_key, const
     if (chunks > 1 && pl.ns > 1) return join_s_chunks(c, p, pl, chunks, r_key, r_val, s_key, s_val, out);
     pl.direct = choose_direct(*p, pl);
     pl.merge = !pl.direct && choose_merge(pl);
-    rc = ensure_workspace(c, pl);
-    if (rc == BJ_ERR_NOMEM && pl.merge) {
-        // without S's own set of partition buffers
-        for (DevBuf* b : {&c->part2, &c->totals2, &c->l1h2, &c->l1off2, &c->colsum2, &c->tmp2}) release(*b);
-        pl.merge = false;
-        rc = ensure_workspace(c, pl);
-    }
-    if (rc) return rc;
+    if ((rc = ensure_join_workspace(c, pl))) return rc;
     hipStream_t st = c->stream;
 
     // Kernel-slot events only when the caller collects phase times: each event
