@@ -206,24 +206,4 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* wtmp, T* total, T wave
     return before + inc - v;
 }
 
-// Exclusive scan of an LDS array in[0..n) into out[0..n) (may alias).
-template <int BLOCK>
-__device__ __forceinline__ uint32_t lds_exclusive_scan(const uint32_t* in, uint32_t* out, int n,
-                                                      uint32_t* wtmp)
-{
-    const int per = (n + BLOCK - 1) / BLOCK;
-    const int lo = min((int)threadIdx.x * per, n);
-    const int hi = min(lo + per, n);
-    uint32_t s = 0;
-    for (int i = lo; i < hi; i++) s += in[i];
-    uint32_t tot;
-    uint32_t ex = block_exclusive_scan<BLOCK, uint32_t>(s, wtmp, &tot);
-    for (int i = lo; i < hi; i++) {
-        const uint32_t c = in[i];
-        out[i] = ex;
-        ex += c;
-    }
-    return tot;
-}
-
 }  // namespace bj

@@ -72,7 +72,6 @@ struct PlanArgs {
     uint64_t item_cap = 0;
     uint64_t* err = nullptr;
 };
-hipError_t launch_zero_u32(uint32_t* p, uint64_t n, hipStream_t st);
 size_t scan_partials_needed(uint64_t n);
 hipError_t launch_scan(const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* partial,
                        hipStream_t st);

@@ -334,13 +334,6 @@ __device__ __forceinline__ void starts_block(const uint32_t* __restrict__ v, int
     if (threadIdx.x == 0) out[n] = tot;
 }
 
-__global__ void k_zero_u32(uint32_t* __restrict__ p, uint64_t n)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = 0u;
-}
-
 // ============================================================== scan (u32 -> u64 exclusive)
 // Reduce-then-scan over n entries; out has n + 1 entries, out[n] = total.
 constexpr int SCAN_BLOCK = 256;
@@ -1329,14 +1322,6 @@ hipError_t launch_cols(const PartSide* sides, int n, hipStream_t st)
     const Sides S = sides_of(sides, n, [](const PartSide& s) { return cols_wgs(s); }, grid);
     if (S.a.bits > 15 || S.b.bits > 15) return hipErrorInvalidValue;
     k_cols<<<grid, 1024, 0, st>>>(S);
-    return hipGetLastError();
-}
-
-hipError_t launch_zero_u32(uint32_t* p, uint64_t n, hipStream_t st)
-{
-    if (n == 0) return hipSuccess;
-    const int grid = (int)std::min<uint64_t>(4096, (n + 255) / 256);
-    k_zero_u32<<<grid, 256, 0, st>>>(p, n);
     return hipGetLastError();
 }
 
