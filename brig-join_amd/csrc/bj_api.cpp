@@ -115,7 +115,7 @@ void bj::release(DevBuf& b)
 
 namespace bj {
 
-constexpr uint64_t MAX_TUPLES = 0x7FFFFFFFull;  // row ids are 31-bit in the probe's staging
+constexpr uint64_t MAX_TUPLES = 0x7FFFFFFFull;  // positions and counts of one relation are 32-bit in the kernels
 constexpr int MAX_BITS = 15;                     // joint histogram in LDS: 2^15 x 4 B
 constexpr int MAX_LEVEL_BITS = 11;               // fan-out per scatter pass
 constexpr uint64_t SEG_TARGET_BYTES = 64 * 1024; // Bloom segment built in LDS
@@ -136,8 +136,11 @@ constexpr uint64_t SOLO_TUPLES = 32ull << 20;
 // us and 9 ps per tuple.  Both sides of the line, direct against partitioned: 100K x
 // 1M 66 / 72 us, 300K x 300K 66 / 65, 500K x 500K 108 / 71, 16K x 50M 291 / 535,
 // 30K x 30M 331 / 337, 60K x 30M 641 / 317.  With a filter only the survivors are
-// probed (at 10% match 0.8-1.4 ps per pair; twice as much allowed for): 500K x 500K
-// 73 / 101 us, 60K x 30M 229 / 423, 1M x 1M 119 / 114.
+// probed, and nobody knows how many they are: 0.8-1.4 ps per pair at 10% match, up to
+// the unfiltered join's cost where all match, but then the partitioned join is slower
+// too.  With 10 / 50 / 100% of S matching: 500K x 500K 88 / 116 / 148 against 133 / 142 / 151
+// us, 60K x 30M 230 / 410 / 660 against 312 / 420 / 623, 2.5M x 20K 157 / 162 / 170 against
+// 154 / 155 / 160: on the line the choice costs at most 7%.
 constexpr double DIRECT_PS_PROBE = 2.6, DIRECT_PS_SAVED = 35e6, DIRECT_PS_TUPLE = 9.0;
 constexpr double DIRECT_PS_BF_PROBE = 1.0, DIRECT_PS_BF_SAVED = 50e6, DIRECT_PS_BF_TUPLE = 7.0;
 // Probe items below which sub-buckets are sliced finer than 64K probe tuples, and

@@ -653,7 +653,7 @@ __global__ __launch_bounds__(BLOCK) void k_bloom_build(const uint32_t* __restric
 
 // ============================================================== Bloom filter S -> S' (before partitioning)
 // The reference's order (queryAndCompactKernelPartitioned): S is filtered
-// before it is partitioned.  Used when the filter fits the MALL, since each key
+// before it is partitioned.  Used when the filter fits an XCD's L2, since each key
 // probes a random filter block.  Grid-stride over tiles (filter_run).
 template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_bloom_prefilter(
@@ -694,8 +694,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
 // bucket.  Survivors are counting-sorted by sub-bucket in LDS per tile, reserved
 // with one atomic per (tile, sub-bucket) and written, compacted, into their
 // sub-bucket's region of the S layout (sub-bucket sb gets positions
-// sb_start[sb] + [0, s_fill[sb])), so no second pass over S is needed.  Values
-// are read only for survivors.
+// sb_start[sb] + [0, s_fill[sb])), so no second pass over S is needed.  S comes as
+// whole tuples, so the values of tuples that fail are read too.
 //
 // Tile walk of one XCD: bucket p owns ceil(size / T) consecutive tile numbers
 // starting at tb; a workgroup's tile numbers only grow, so it walks forward.
@@ -1016,8 +1016,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(probe_wav
     // Items are claimed PROBE_GRAB at a time (the counter's answer is waited for
     // once per claim), but one by one when there is no more than one claim for each
     // workgroup: 3M x 4.5M has 512 items, which pairs would give to half of the 512
-    // workgroups (46.6 -> 32.2 us with the next line, by 512 threads per table; 16M x 16M, 2048 items: 99-102 us
-    // in pairs, 105 us one by one).  The first claim is the workgroup's number: from
+    // workgroups (46.6 -> 32.2 us with the next line, by 512 threads per table; 16M x
+    // 16M, 2048 items: 99-102 us in pairs, 105 us one by one).  The first claim is the workgroup's number: from
     // the counter, the last of 512 answers would be several us away.
     const int grab = n_work <= (uint64_t)gridDim.x * PROBE_GRAB ? 1 : PROBE_GRAB;
     uint64_t item = (uint64_t)blockIdx.x * grab;
@@ -1117,29 +1117,29 @@ __global__ __launch_bounds__(BLOCK) void k_direct_bloom(const uint32_t* __restri
         if (blk[s] != EMPTY) atomicOr((unsigned long long*)&filter[blk[s]], bits[s]);
 }
 
-// Joins unpartitioned relations: the build side in C chunks of at most CAP
-// tuples, the probe side in slices, one (chunk, slice) pair per workgroup and
-// step.  Every chunk streams all of the probe side past its table, so the work
-// is C * np probes where the partitioned path moves every tuple two to four
-// times through sixteen or more launches.  Bound by launches and the build's
-// latency for small relations (1500 x 2000: 124 -> 53 us a call, 200K x 300K with
-// the filter 233 -> 115 us), by the probe's issue rate for long ones (6001 x 20M:
-// 4.99 -> 0.57 ms; the partitioned path had 32 work items there).  ns_dev, when not null, is the
-// device-side length of S (S' after the filter).  Workgroups of one slice run
-// on one XCD (slices are dealt in multiples of 8), so its keys come from that
+// Joins unpartitioned relations: the build side in C chunks of at most CAP tuples, the
+// probe side in slices, one (chunk, slice) pair per workgroup and step.  Every chunk
+// streams all of the probe side past its table, so the work is C * np probes where the
+// partitioned path moves every tuple two to four times (sixteen or more launches when
+// this was measured, five to twelve now).  Bound by launches and the build's latency
+// for small relations (1500 x 2000: 124 -> 53 us a call, 200K x 300K with the filter
+// 233 -> 115 us), by the probe's issue rate and row writes for long ones (6001 x 20M:
+// 4.99 -> 0.42 ms a call; the partitioned path had 32 work items there).  ns_dev, when
+// not null, is the device-side length of S (S' after the filter).  Workgroups of one
+// slice run on one XCD (slices are dealt in multiples of 8), so its keys come from that
 // XCD's L2 after the first chunk.
-// WATCH (build sides of several chunks): every probe key of a bucket walks its whole run, so a key that fills a good part of
-// every chunk costs far more than here is saved (300K x 200K with 90% of S equal: 1.8
-// ms), where the partitioned join builds the hot sub-bucket's table from the other side.
-// A workgroup whose table has a longer run than it may have sets *long_run and leaves;
-// the host then joins by partitions (of bits radix bits).  With one chunk (C = 1) the
-// partitioned join would build the same table.  Otherwise a run may be DIRECT_MAX_RUN
-// long, or as long as a key that has it in every chunk leaves its sub-bucket of the
-// partitioned join smaller on this side than on the other, so that a C times longer
-// run would be walked there.  Both sides of the line, direct against partitioned: 200K x
-// 300K, 256 copies in a chunk 109 / 76 us (some 40 us more after the attempt), 512 138 /
-// 76, 1024 281 / 76; 300K x 100K 512 119 / 969, 1024 270 / 75; 100K x 1M 1024 398 / 660, 2M x
-// 50K 4096 1582 / 2192.
+// WATCH (build sides of several chunks): every probe key of a bucket walks its whole
+// run, so a key that fills a good part of every chunk costs far more than here is saved
+// (300K x 200K with 90% of S equal: 1.8 ms), where the partitioned join builds the hot
+// sub-bucket's table from the other side.  A workgroup whose table has a longer run than
+// it may have sets *long_run and leaves; the host then joins by partitions (of bits
+// radix bits).  With one chunk (C = 1) the partitioned join would build the same table.
+// Otherwise a run may be DIRECT_MAX_RUN long, or as long as a key that has it in every
+// chunk leaves its sub-bucket of the partitioned join smaller on this side than on the
+// other, so that a C times longer run would be walked there.  Both sides of the line,
+// direct against partitioned: 200K x 300K, 256 copies in a chunk 109 / 76 us (some 40
+// us more after the attempt), 512 138 / 76, 1024 281 / 76; 300K x 100K 512 119 / 969,
+// 1024 270 / 75; 100K x 1M 1024 398 / 660, 2M x 50K 4096 1582 / 2192.
 constexpr uint32_t DIRECT_MAX_RUN = 320;
 
 template <int BLOCK, int CAP, int PITEMS, bool WATCH>

@@ -42,14 +42,14 @@ __device__ __forceinline__ void hist_range(const uint32_t* __restrict__ key, uin
 // ---------------------------------------------------------------- scatter
 // LDS-staged scatter with write-combining carries.
 //
-// Each tile of T tuples is counting-sorted by bucket in LDS (rank from an LDS
-// atomic, offsets from an LDS scan).  Bucket b's tuples go to consecutive global
-// positions starting at cur[b].  Only whole CS-tuple chunks (CS * 4 bytes) are
-// written; the unaligned tail of every bucket (< CS tuples) is carried in LDS
-// to the next tile, so every chunk of the output is written by one workgroup
-// within one tile.  Partial chunks occur only where two workgroups' ranges of
-// a bucket meet.  The next tile is loaded into registers while the current one
-// is written out.
+// Each tile of T tuples is counting-sorted by bucket in LDS (rank from an LDS atomic,
+// offsets from an LDS scan).  Bucket b's tuples go to consecutive global positions
+// starting at cur[b].  Only whole CS-tuple chunks (CS * 8 bytes of whole tuples, CS * 4
+// of each of two arrays) are written; the unaligned tail of every bucket (< CS tuples)
+// is carried in LDS to the next tile, so every chunk of the output is written by one
+// workgroup within one tile.  Partial chunks occur only where two workgroups' ranges of
+// a bucket meet.  The next tile is loaded into registers while the current one is
+// written out.
 // A tuple as one 8-byte unit: key, then value.
 typedef uint32_t Tuple __attribute__((ext_vector_type(2)));
 
@@ -380,17 +380,18 @@ struct FilterTile {
     uint64_t* count;
 };
 
-// Runs tiles through the filter: every key tests its 64-bit block; survivors are
-// ranked by wave ballots per (item, wave) group and a scan of the group counts,
-// staged in LDS and written, compacted, at places reserved with one global atomic
-// per tile.  The reservation and the stores lag one tile behind (two staging
-// buffers) and the next tile's tuples are loaded while this one is staged, so
-// neither latency is on a tile's path.  Values are loaded with the keys: from some
-// 10% survivors on their lines are touched anyway.  Tile numbers run below end:
-// next(t) is the number that follows the one it returned last (thread 0 requests
-// it a tile ahead), desc(t) its tile.  stage: 2 * BLOCK * ITEMS tuples, gcnt: 64
-// counts, s_base / s_next: one word each.  Returns true if a write would pass its
-// tile's out_cap.
+// Runs tiles through the filter: every key tests its 64-bit block; survivors are ranked
+// by wave ballots per (item, wave) group and a scan of the group counts, staged in LDS
+// and written, compacted, at places reserved with one global atomic per tile.  The
+// reservation and the stores lag one tile behind (two staging buffers) and the next
+// tile's tuples are loaded while this one is staged, so neither latency is on a tile's
+// path.  Values are loaded with the keys: from some 10% survivors on their lines are
+// touched anyway, and below that the requests for filter words bound the run, not the
+// bytes (2.5M x 100M with 0 / 1 / 3 / 10% matches: 453 / 456 / 458 / 459 us; the
+// form before, with the values of survivors only, 474 / 495 / 513 / 545).  Tile numbers run below end: next(t)
+// is the number that follows the one it returned last (thread 0 requests it a tile
+// ahead), desc(t) its tile.  stage: 2 * BLOCK * ITEMS tuples, gcnt: 64 counts, s_base /
+// s_next: one word each.  Returns true if a write would pass its tile's out_cap.
 template <int BLOCK, int ITEMS, class Next, class Desc>
 __device__ __forceinline__ bool filter_run(uint32_t end, Next&& next, Desc&& desc, Tuple* stage, uint32_t* gcnt,
                                            uint64_t* s_base, uint32_t* s_next)
@@ -685,8 +686,9 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     // load is on a round's path.
     // One atomic reserves the rows of two rounds (an odd one and the one before): the
     // chip does about 70 atomics on one address per us, and one per round of 5120 keys
-    // was as many (640M x 640M: 125K in 1.94 ms; rounds of 4096 keys took 2.24 ms, of
-    // 6144 keys 1.76).  One per two rounds: 1.69 ms, and 16M x 16M 100 -> 93 us.
+    // (512 threads of 10 keys) was as many (640M x 640M: 125K in 1.94 ms; rounds of 4096
+    // keys took 2.24 ms, of 6144 keys 1.76).  One per two rounds: 1.69 ms, and 16M x 16M 100
+    // -> 93 us; 1024 threads of 4 keys: 1.53 ms.
     constexpr int NR = STAGE / BLOCK;
     uint32_t wk[NR], wp[NR], wb[NR];  // loaded rows: key, probe / build value
     uint32_t n_loaded = 0;          // rows in the registers, stored this round (uniform)

@@ -74,7 +74,13 @@ enum {
     BJ_NUM_PROBE_PHASES
 };
 
-/* ---- per-kernel timing slots (milliseconds, hipEvent on the join stream) */
+/* ---- per-kernel timing slots (milliseconds, hipEvent on the join stream).
+ * Where both relations are below 32M tuples their partition passes may run in the
+ * same launches: such a launch's time is then shared out between its R and its S slot
+ * by the tuples of each side, and is no measure of one against the other.  A slot
+ * whose work ran inside another launch, or not at all, is 0: BJ_K_PLAN where S's
+ * second pass plans the probe, and all but the filter's and the probe's slots where a
+ * small build side is joined without a partition. */
 enum {
     BJ_K_HIST_R = 0,     /* k_hist over R (joint radix histogram)                 */
     BJ_K_SCAN_R,         /* histogram reduction + offset scans of R               */
@@ -86,7 +92,7 @@ enum {
     BJ_K_SCAN_S,
     BJ_K_SCATTER1_S,
     BJ_K_SCATTER2_S,
-    BJ_K_PLAN,           /* vlsplit work planning                                 */
+    BJ_K_PLAN,           /* vlsplit work planning (its own launch, else 0)        */
     BJ_K_PROBE,          /* LDS build + probe + rows                              */
     BJ_NUM_KERNELS
 };
@@ -231,9 +237,10 @@ int  bj_join(bj_ctx *ctx, const bj_params *p,
  * Inputs must be device pointers (p->inputs_on_device = 1) joined in one pass
  * (p->s_chunks = 1), without probe phase timers.  The workspace is carved from a
  * static device array of BJ_NOALLOC_SCRATCH_BYTES per GPU; a join whose
- * workspace (bj_plan's workspace_bytes minus the row buffers) exceeds it is
- * refused with BJ_ERR_SIZE, which at 256 MiB allows about 8-11M tuples per
- * relation.  Rows go to the caller's device arrays out_key / out_rval / out_sval
+ * workspace exceeds it is refused with BJ_ERR_SIZE, which at 256 MiB allows about
+ * 8-11M tuples per relation.  (That is at most bj_plan's workspace_bytes minus the
+ * row buffers: a join near the limit does without the second set of partition
+ * buffers and with half the per-chunk histograms that bj_join takes.)  Rows go to the caller's device arrays out_key / out_rval / out_sval
  * (out_cap rows each; the count stays exact past it, as in bj_join) and
  * out->key / r_val / s_val point there.  Every call on one GPU shares that GPU's
  * array, so calls that overlap on one GPU race: serialise them. */
