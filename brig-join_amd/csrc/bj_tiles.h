@@ -868,7 +868,10 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         auto write_single = [&](uint64_t w) {  // the values of the first HALF groups are loaded
 #pragma unroll
             for (int h = 0; h < PITEMS; h += HALF) {
-                if (h) load_values(h);
+                if (h) {
+                    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the stores of the groups before
+                    load_values(h);
+                }
 #pragma unroll
                 for (int u = 0; u < HALF; u++) {
                     if (h + u >= PITEMS) continue;
@@ -895,18 +898,27 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
         if (threadIdx.x == 0) L.s_direct = sd;
         __syncthreads();
         uint64_t w = uniform_u64(L.s_direct + pre);
-        if (__ballot(multi != 0u) == 0ull) {  // this wave has none
+        if (w >= out_cap) {
+            // all of the wave's rows are past the capacity: counted, no more (7M x 7M with ten
+            // rows per S tuple and room for one: 1640 -> 276 us)
+        } else if (__ballot(multi != 0u) == 0ull) {  // this wave has none
             load_values(0);
             write_single(w);
         } else {
             // duplicate build keys: the wave's rows go through its share of the
             // round's stage (free: stage[r3] was last read a round ago), so the
-            // values of all its rows are in flight instead of one per match of a lane
+            // values of all its rows are in flight instead of one per match of a lane.
+            // Key groups with more than DEEP matches per matching lane are left for last and
+            // read by the whole wave, one run at a time: with every lane adding its own
+            // matches few lanes are busy in a window (3000 x 3000 with 50 copies of each key 553
+            // us, now 108; 1M x 1.5M 1310 -> 360), with four copies they are the faster ones.
+            constexpr uint32_t DEEP = 8;
             constexpr uint32_t FIFO = STAGE / (BLOCK / WAVE);
             static_assert(FIFO == 2 * WAVE || FIFO == WAVE, "one or two rows per lane");
             const uint32_t lane = lane_id();
             uint32_t* fifo = &L.stage[r3][threadIdx.x / WAVE * FIFO];
-            uint32_t n = 0;  // rows in the wave's FIFO (uniform)
+            uint32_t n = 0;     // rows in the wave's FIFO (uniform)
+            uint32_t deep = 0;  // key groups left for the wave to read (uniform)
             auto drain = [&]() {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 constexpr int NF = FIFO / WAVE;
@@ -935,8 +947,7 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             };
 #pragma unroll
             for (int it = 0; it < PITEMS; it++) {
-                // this key's matches (its rows stay next to each other), places in
-                // the wave by a scan; the FIFO takes them in windows of its free room
+                // this key's matches, places in the wave by a scan
                 const uint32_t prow = (uint32_t)it * BLOCK + threadIdx.x, qend = qm[it] >> 16;
                 uint32_t q = qm[it] & 0xFFFFu;
                 uint32_t left = (hitmask >> it) & 1u;
@@ -945,6 +956,11 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
                 const uint32_t inc = wave_inclusive_scan<uint32_t>(left);
                 uint32_t pos = inc - left;  // of this lane's next row
                 const uint32_t rows = __builtin_amdgcn_readlane(inc, WAVE - 1);
+                if (rows > DEEP * (uint32_t)__popcll(__ballot(left != 0u))) {
+                    deep |= 1u << it;
+                    continue;
+                }
+                // the FIFO takes the rows in windows of its free room
                 for (uint32_t w0 = 0; w0 < rows;) {
                     const uint32_t take = min(FIFO - n, rows - w0);
                     while (left && pos < w0 + take) {
@@ -956,6 +972,36 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
                     n += take;
                     w0 += take;
                     if (n == FIFO) drain();
+                }
+            }
+            // groups of many matches per key: lane by lane, the wave reads its run 64 slots
+            // at a time
+            for (; deep && w < out_cap; deep &= deep - 1u) {
+                const int it = __builtin_ctz(deep);
+                uint32_t mine = kk[0], run = qm[0];
+#pragma unroll
+                for (int u = 1; u < PITEMS; u++) {
+                    mine = it == u ? kk[u] : mine;
+                    run = it == u ? qm[u] : run;
+                }
+                for (uint64_t todo = __ballot((hitmask >> it) & 1u); todo && w < out_cap; todo &= todo - 1ull) {
+                    const int l = __builtin_ctzll(todo);
+                    const uint32_t key = __builtin_amdgcn_readlane(mine, l);
+                    const uint32_t q0 = __builtin_amdgcn_readlane(run, l), q1 = q0 >> 16;
+                    const uint32_t row = (uint32_t)it * BLOCK + (threadIdx.x & ~(WAVE - 1u)) + (uint32_t)l;
+                    for (uint32_t x = q0 & 0xFFFFu; x < q1; x += WAVE) {
+                        const uint32_t slot = x + lane;
+                        const bool hit = slot < q1 && L.hkey[min(slot, q1 - 1u)] == key;
+                        const uint64_t m = __ballot(hit);
+                        const uint32_t cnt = (uint32_t)__popcll(m), take = min(FIFO - n, cnt), at = lanes_below(m);
+                        if (hit && at < take) fifo[n + at] = row | slot << 16;
+                        n += take;
+                        if (n == FIFO) {
+                            drain();
+                            if (hit && at >= take) fifo[at - take] = row | slot << 16;
+                            n = cnt - take;
+                        }
+                    }
                 }
             }
             if (n) drain();
