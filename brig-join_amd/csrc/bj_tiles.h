@@ -911,8 +911,10 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             // Key groups with more than DEEP matches per matching lane are left for last and
             // read by the whole wave, one run at a time: with every lane adding its own
             // matches few lanes are busy in a window (3000 x 3000 with 50 copies of each key 553
-            // us, now 108; 1M x 1.5M 1310 -> 360), with four copies they are the faster ones.
-            constexpr uint32_t DEEP = 8;
+            // us, now 108; 1M x 1.5M 1310 -> 360), with fewer they are the faster ones: 7M x 7M, by the
+            // lanes / by the wave, with 10 copies 470 / 497 us, 12 541 / 532, 16 727 / 610; 37K x 394K
+            // with some 10 in a chunk 219 / 291.
+            constexpr uint32_t DEEP = 12;
             constexpr uint32_t FIFO = STAGE / (BLOCK / WAVE);
             static_assert(FIFO == 2 * WAVE || FIFO == WAVE, "one or two rows per lane");
             const uint32_t lane = lane_id();
