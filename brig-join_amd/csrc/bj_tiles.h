@@ -908,19 +908,17 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
             // duplicate build keys: the wave's rows go through its share of the
             // round's stage (free: stage[r3] was last read a round ago), so the
             // values of all its rows are in flight instead of one per match of a lane.
-            // Key groups with more than DEEP matches per matching lane are left for last and
-            // read by the whole wave, one run at a time: with every lane adding its own
-            // matches few lanes are busy in a window (3000 x 3000 with 50 copies of each key 553
-            // us, now 108; 1M x 1.5M 1310 -> 360), with fewer they are the faster ones: 7M x 7M, by the
-            // lanes / by the wave, with 10 copies 470 / 497 us, 12 541 / 532, 16 727 / 610; 37K x 394K
-            // with some 10 in a chunk 219 / 291.
-            constexpr uint32_t DEEP = 12;
+            // Where a lane has a run of more than DEEP slots the whole wave reads the runs, one
+            // after the other: with every lane adding its own matches few lanes are busy in a
+            // window (3000 x 3000 with 50 copies of each key 553 us, now 99; 1M x 1.5M 1310 ->
+            // 358), with short runs they are the faster ones (by the lanes / by the wave, 37K x
+            // 394K with some 10 copies in a chunk 217 / 278 us, 50K x 227K 118 / 150).
+            constexpr uint32_t DEEP = 24;
             constexpr uint32_t FIFO = STAGE / (BLOCK / WAVE);
             static_assert(FIFO == 2 * WAVE || FIFO == WAVE, "one or two rows per lane");
             const uint32_t lane = lane_id();
             uint32_t* fifo = &L.stage[r3][threadIdx.x / WAVE * FIFO];
-            uint32_t n = 0;     // rows in the wave's FIFO (uniform)
-            uint32_t deep = 0;  // key groups left for the wave to read (uniform)
+            uint32_t n = 0;  // rows in the wave's FIFO (uniform)
             auto drain = [&]() {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 constexpr int NF = FIFO / WAVE;
@@ -947,61 +945,63 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
                 n = 0;
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             };
+            uint32_t longest = 0;
 #pragma unroll
-            for (int it = 0; it < PITEMS; it++) {
-                // this key's matches, places in the wave by a scan
-                const uint32_t prow = (uint32_t)it * BLOCK + threadIdx.x, qend = qm[it] >> 16;
-                uint32_t q = qm[it] & 0xFFFFu;
-                uint32_t left = (hitmask >> it) & 1u;
-                if ((multi >> it) & 1u)
-                    for (uint32_t x = q + 1; x < qend; x++) left += L.hkey[x] == kk[it];
-                const uint32_t inc = wave_inclusive_scan<uint32_t>(left);
-                uint32_t pos = inc - left;  // of this lane's next row
-                const uint32_t rows = __builtin_amdgcn_readlane(inc, WAVE - 1);
-                if (rows > DEEP * (uint32_t)__popcll(__ballot(left != 0u))) {
-                    deep |= 1u << it;
-                    continue;
-                }
-                // the FIFO takes the rows in windows of its free room
-                for (uint32_t w0 = 0; w0 < rows;) {
-                    const uint32_t take = min(FIFO - n, rows - w0);
-                    while (left && pos < w0 + take) {
-                        fifo[n + pos - w0] = prow | q << 16;
-                        pos++;
-                        if (--left)
-                            while (L.hkey[++q] != kk[it]) {}
-                    }
-                    n += take;
-                    w0 += take;
-                    if (n == FIFO) drain();
-                }
-            }
-            // groups of many matches per key: lane by lane, the wave reads its run 64 slots
-            // at a time
-            for (; deep && w < out_cap; deep &= deep - 1u) {
-                const int it = __builtin_ctz(deep);
-                uint32_t mine = kk[0], run = qm[0];
+            for (int it = 0; it < PITEMS; it++)
+                if ((multi >> it) & 1u) longest = max(longest, (qm[it] >> 16) - (qm[it] & 0xFFFFu));
+            if (__ballot(longest > DEEP) == 0ull) {
 #pragma unroll
-                for (int u = 1; u < PITEMS; u++) {
-                    mine = it == u ? kk[u] : mine;
-                    run = it == u ? qm[u] : run;
-                }
-                for (uint64_t todo = __ballot((hitmask >> it) & 1u); todo && w < out_cap; todo &= todo - 1ull) {
-                    const int l = __builtin_ctzll(todo);
-                    const uint32_t key = __builtin_amdgcn_readlane(mine, l);
-                    const uint32_t q0 = __builtin_amdgcn_readlane(run, l), q1 = q0 >> 16;
-                    const uint32_t row = (uint32_t)it * BLOCK + (threadIdx.x & ~(WAVE - 1u)) + (uint32_t)l;
-                    for (uint32_t x = q0 & 0xFFFFu; x < q1; x += WAVE) {
-                        const uint32_t slot = x + lane;
-                        const bool hit = slot < q1 && L.hkey[min(slot, q1 - 1u)] == key;
-                        const uint64_t m = __ballot(hit);
-                        const uint32_t cnt = (uint32_t)__popcll(m), take = min(FIFO - n, cnt), at = lanes_below(m);
-                        if (hit && at < take) fifo[n + at] = row | slot << 16;
+                for (int it = 0; it < PITEMS; it++) {
+                    // this key's matches, places in the wave by a scan
+                    const uint32_t prow = (uint32_t)it * BLOCK + threadIdx.x, qend = qm[it] >> 16;
+                    uint32_t q = qm[it] & 0xFFFFu;
+                    uint32_t left = (hitmask >> it) & 1u;
+                    if ((multi >> it) & 1u)
+                        for (uint32_t x = q + 1; x < qend; x++) left += L.hkey[x] == kk[it];
+                    const uint32_t inc = wave_inclusive_scan<uint32_t>(left);
+                    uint32_t pos = inc - left;  // of this lane's next row
+                    const uint32_t rows = __builtin_amdgcn_readlane(inc, WAVE - 1);
+                    // the FIFO takes the rows in windows of its free room
+                    for (uint32_t w0 = 0; w0 < rows;) {
+                        const uint32_t take = min(FIFO - n, rows - w0);
+                        while (left && pos < w0 + take) {
+                            fifo[n + pos - w0] = prow | q << 16;
+                            pos++;
+                            if (--left)
+                                while (L.hkey[++q] != kk[it]) {}
+                        }
                         n += take;
-                        if (n == FIFO) {
-                            drain();
-                            if (hit && at >= take) fifo[at - take] = row | slot << 16;
-                            n = cnt - take;
+                        w0 += take;
+                        if (n == FIFO) drain();
+                    }
+                }
+            } else {
+                // the wave reads one run after the other, 64 slots at a time
+#pragma unroll 1
+                for (int it = 0; it < PITEMS && w < out_cap; it++) {
+                    uint32_t mine = kk[0], run = qm[0];
+#pragma unroll
+                    for (int u = 1; u < PITEMS; u++) {
+                        mine = it == u ? kk[u] : mine;
+                        run = it == u ? qm[u] : run;
+                    }
+                    for (uint64_t todo = __ballot((hitmask >> it) & 1u); todo && w < out_cap; todo &= todo - 1ull) {
+                        const int l = __builtin_ctzll(todo);
+                        const uint32_t key = __builtin_amdgcn_readlane(mine, l);
+                        const uint32_t q0 = __builtin_amdgcn_readlane(run, l), q1 = q0 >> 16;
+                        const uint32_t row = (uint32_t)it * BLOCK + (threadIdx.x & ~(WAVE - 1u)) + (uint32_t)l;
+                        for (uint32_t x = q0 & 0xFFFFu; x < q1; x += WAVE) {
+                            const uint32_t slot = x + lane;
+                            const bool hit = slot < q1 && L.hkey[min(slot, q1 - 1u)] == key;
+                            const uint64_t m = __ballot(hit);
+                            const uint32_t cnt = (uint32_t)__popcll(m), take = min(FIFO - n, cnt), at = lanes_below(m);
+                            if (hit && at < take) fifo[n + at] = row | slot << 16;
+                            n += take;
+                            if (n == FIFO) {
+                                drain();
+                                if (hit && at >= take) fifo[at - take] = row | slot << 16;
+                                n = cnt - take;
+                            }
                         }
                     }
                 }

@@ -28,7 +28,7 @@ def to_dev(host):
 
 @pytest.mark.parametrize("kw", [dict(), dict(radix_bits=1), dict(radix_bits=1, tile=4096), dict(radix_bits=6)])
 @pytest.mark.parametrize("n_r,n_s,copies,match", [
-    (3000, 3000, 12, 1.0), (3000, 3000, 13, 1.0),   # up to and from which number of copies a run is read by the wave
+    (3000, 3000, 12, 1.0), (3000, 3000, 24, 1.0), (3000, 3000, 25, 1.0),   # about the runs that the wave reads
     (3000, 3000, 50, 1.0),
     (8000, 2500, 63, 0.3), (8000, 2500, 64, 0.3), (8000, 2500, 65, 0.3), (8000, 2500, 129, 0.3),   # steps of a run
     (8000, 2500, 4000, 0.01),
