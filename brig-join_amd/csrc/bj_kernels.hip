@@ -1484,7 +1484,7 @@ int probe_grid(int tile, int num_cu) { return tile == 8192 ? num_cu * 2 : num_cu
 // copies of each key 315 -> 259, 64M x 1.28B 289 -> 263, 3M x 4.5M 33.4 -> 29.7.  Rounds
 // of 3 keys per thread leave less of a short probe side's last round empty (ids with 4:
 // 693 us, 3M x 4.5M 35.2); from PROBE_LONG probe tuples per sub-bucket on 4 are better,
-// with fewer reservations (640M x 640M, 39K per sub-bucket: 1.52 ms, 3 keys 1.74).
+// with fewer reservations (640M x 640M, 39K per sub-bucket: 1.56 ms, 3 keys 1.74).
 constexpr int PROBE_ITEMS = 3, PROBE_ITEMS_LONG = 4;
 constexpr uint64_t PROBE_LONG = 16384;
 

@@ -688,7 +688,7 @@ __device__ __forceinline__ bool probe_item(ProbeLds<BLOCK, CAP>& L, const uint32
     // chip does about 70 atomics on one address per us, and one per round of 5120 keys
     // (512 threads of 10 keys) was as many (640M x 640M: 125K in 1.94 ms; rounds of 4096
     // keys took 2.24 ms, of 6144 keys 1.76).  One per two rounds: 1.69 ms, and 16M x 16M 100
-    // -> 93 us; 1024 threads of 4 keys: 1.53 ms.
+    // -> 93 us; 1024 threads of 4 keys: 1.56 ms.
     constexpr int NR = STAGE / BLOCK;
     uint32_t wk[NR], wp[NR], wb[NR];  // loaded rows: key, probe / build value
     uint32_t n_loaded = 0;          // rows in the registers, stored this round (uniform)
